@@ -951,9 +951,7 @@ void offdiag_spmv(owtk_matrix m, const V* vals, const X* x, E e)
         launch_sell_cd_bs<V, X, false, E>(m->bs, s.max_width, grid, st, s.slice_ptr.get(), s.row_len.get(),
                                           s.columns.get(), vals, static_cast<const V*>(nullptr), x, rows, e, scratch);
     } else {
-        std::int64_t blocks = (rows + dev::kWavesPerBlock - 1) / dev::kWavesPerBlock;
-        blocks = std::max<std::int64_t>(1, std::min<std::int64_t>(blocks, dev::kMaxReduceBlocks));
-        spmv_csr_cd<V, X, false, E><<<static_cast<unsigned int>(blocks), kBlock, 0, st>>>(
+        spmv_csr_cd<V, X, false, E, 8><<<dev::stream_grid(rows * m->bs), kBlock, 0, st>>>(
             s.offsets.get(), s.columns.get(), vals, nullptr, x, rows, m->bs, e, scratch);
     }
     OWTK_LAUNCH_CHECK();

@@ -1,0 +1,50 @@
+"""Kernels at the sizes where their tiles, passes and dispatch rules end:
+row lengths around the entries loaded per pass, blocks that do not divide a
+workgroup, vertex counts that leave partial tiles.  Compared with the CPU
+oracle, bit for bit where the kernel keeps the oracle's order."""
+import numpy as np
+import pytest
+
+import owtk
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def ragged_pattern(rng, n, ghost, lengths):
+    """Offsets and ascending columns with the given row lengths, diagonal left out."""
+    offsets = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    columns = []
+    for i in range(n):
+        choice = np.setdiff1d(np.arange(n + ghost), [i])
+        columns.append(np.sort(rng.choice(choice, lengths[i], replace=False)))
+    return offsets, np.concatenate(columns).astype(np.int32)
+
+
+@pytest.mark.parametrize("block", [5, 7, 36, 65, 300])
+def test_row_component_spmv(ctx, block):
+    """Blocks above four components: rows of 0 to 17 entries (8 per pass), rows that straddle waves and
+    workgroups; split and CSR forms bitwise, FP32 storage bitwise, the residual's fused norm."""
+    rng = np.random.default_rng(block)
+    n, ghost = 37, 3
+    lengths = np.concatenate([[0, 1, 7, 8, 9, 15, 16, 17], rng.integers(0, 18, n - 8)])
+    off, col = ragged_pattern(rng, n, ghost, lengths)
+    val = rng.uniform(-1, 1, off[-1] * block)
+    diag = rng.uniform(1, 2, n * block)
+    x = rng.uniform(-1, 1, (n + ghost) * block)
+    xd, yd = ctx.upload(x), ctx.empty(n * block)
+    om = orc.OMatrix.split(n, ghost, block, off, col, diag, val)
+    m = owtk.Matrix.split(ctx, n, ghost, block, off, col, diag, val)
+    m.spmv(xd, yd)
+    ref = om.spmv(x)
+    assert np.array_equal(yd.download(), ref)
+    b = rng.uniform(-1, 1, n * block)
+    m.residual(ctx.upload(b), xd, yd)
+    assert np.array_equal(yd.download(), b - ref)
+    mc = owtk.Matrix.csr(ctx, n, ghost, block, off, col, val)
+    mc.spmv(xd, yd)
+    assert np.array_equal(yd.download(), orc.OMatrix.csr(n, ghost, block, off, col, val).spmv(x))
+    m.add_storage(owtk.F32)
+    yf = ctx.empty(n * block, np.float32)
+    m.spmv(ctx.upload(x.astype(np.float32)), yf, owtk.F32)
+    assert np.array_equal(yf.download(), om.spmv_f32(val, diag, x))
