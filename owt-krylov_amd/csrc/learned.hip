@@ -47,10 +47,8 @@ namespace {
 
 using dev::kBlock;
 constexpr int W = kGnnWidth;
-constexpr int kTile = 64;            // vertices per LDS tile in the gradient reductions
-constexpr int kReduceGrid = 240;     // blocks of the gradient reductions
-constexpr int kMaxOuterOutputs = kGnnMaxOutputs * W + kGnnMaxOutputs;
-constexpr int kOutPerThread = (kMaxOuterOutputs + kBlock - 1) / kBlock;
+constexpr int kReduceGrid = 512;     // blocks of the gradient reductions: two per CU
+constexpr int kMaxOuterOutputs = kGnnMaxOutputs * 2 * W + kGnnMaxOutputs;
 
 unsigned int rows_grid(std::int64_t n)
 {
@@ -556,69 +554,118 @@ __global__ __launch_bounds__(256) void k_gnn_agg_t(std::int64_t n, const std::in
     store_row(dprev + j * W, acc);
 }
 
-__global__ __launch_bounds__(256) void k_tanh_bwd(std::int64_t count, const float* __restrict__ h,
-                                                  float* __restrict__ d)
+// Weight gradients on the matrix cores: over all vertices i,
+//     sum A_i B0_i^T (R x C0),  sum A_i B1_i^T (R x C1, NB = 2),  sum A_i (R),
+// R, C0, C1 <= 32, with A_i scaled by 1 - h_i^2 first when h is given (the
+// encoder's tanh).  A wave takes two vertices per v_mfma_f32_32x32x2_f32:
+// lane l supplies component l % 32 of vertex l / 32, so one load of a
+// 32-wide array is 64 consecutive floats, straight from memory to the matrix
+// cores; kOuterPairs vertex pairs are in flight at once.  The four waves'
+// sums meet in LDS and one partial per block goes to the finisher.  It reads
+// each activation once per layer (A serves both products and the sum).
+// Bound by the latency of its loads: at 131,072 vertices and R = 32 a layer's
+// 50 MB take 15.0 us with two blocks per CU (17.8 us with one).  LDS tiles
+// with one output per thread took 77 us per product (an LDS read pair per FMA
+// and output), 154 us per layer.
+constexpr int kOuterPairs = 8;
+template<int NB, bool TANH>
+__global__ __launch_bounds__(256) void k_outer_mfma(std::int64_t n, const float* __restrict__ A, int R,
+                                                    const float* __restrict__ h, const float* __restrict__ B0, int C0,
+                                                    const float* __restrict__ B1, int C1,
+                                                    float* __restrict__ partials)
 {
-    const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
-    for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < count; t += step)
-        d[t] *= 1.0f - h[t] * h[t];
-}
-
-// Partial sums over vertex tiles of A_i B_i^T (R x C) and A_i (R):
-// partials[block][R*C + R].  B may be null (C = 0).
-__global__ __launch_bounds__(256) void k_outer_partials(std::int64_t n, const float* __restrict__ A, int R,
-                                                        const float* __restrict__ B, int C,
-                                                        float* __restrict__ partials)
-{
-    __shared__ float sa[kTile * kGnnMaxOutputs];
-    __shared__ float sb[kTile * W];
-    const int outs = R * C + R;
-    float acc[kOutPerThread];
+    constexpr int U = kOuterPairs;
+    __shared__ float red[4][NB * W * W + W];
+    const int lane = static_cast<int>(threadIdx.x & 63), m = lane & 31, half = lane >> 5;
+    const int wave = static_cast<int>(threadIdx.x >> 6);
+    const int ma = m < R ? m : R - 1, m0 = m < C0 ? m : C0 - 1, m1 = NB == 2 && m >= C1 ? C1 - 1 : m;
+    f32x16 acc[NB];
 #pragma unroll
-    for (int j = 0; j < kOutPerThread; ++j) acc[j] = 0.f;
-    for (std::int64_t tile = static_cast<std::int64_t>(blockIdx.x) * kTile; tile < n;
-         tile += static_cast<std::int64_t>(gridDim.x) * kTile) {
-        const int cnt = static_cast<int>(std::min<std::int64_t>(kTile, n - tile));
-        for (int q = threadIdx.x; q < cnt * R; q += blockDim.x) sa[q] = A[tile * R + q];
-        for (int q = threadIdx.x; q < cnt * C; q += blockDim.x) sb[q] = B[tile * C + q];
-        __syncthreads();
+    for (int q = 0; q < NB; ++q)
 #pragma unroll
-        for (int j = 0; j < kOutPerThread; ++j) {
-            const int o = threadIdx.x + kBlock * j;
-            if (o < R * C) {
-                const int r = o / C, c = o - (o / C) * C;
-                float s = 0.f;
-                for (int t = 0; t < cnt; ++t) s = __builtin_fmaf(sa[t * R + r], sb[t * C + c], s);
-                acc[j] += s;
-            } else if (o < outs) {
-                const int r = o - R * C;
-                float s = 0.f;
-                for (int t = 0; t < cnt; ++t) s += sa[t * R + r];
-                acc[j] += s;
-            }
+        for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
+    float sum = 0.f;
+    const std::int64_t pairs = (n + 1) / 2;
+    const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * 4 * U;
+    for (std::int64_t p0 = (static_cast<std::int64_t>(blockIdx.x) * 4 + wave) * U; p0 < pairs; p0 += stride) {
+        float a[U], b[NB][U], hv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const std::int64_t v = 2 * (p0 + u) + half;
+            const std::int64_t vc = v < n ? v : n - 1;
+            a[u] = A[vc * R + ma];
+            if constexpr (TANH) hv[u] = h[vc * R + ma];
+            b[0][u] = B0[vc * C0 + m0];
+            if constexpr (NB == 2) b[1][u] = B1[vc * C1 + m1];
         }
-        __syncthreads();
-    }
 #pragma unroll
-    for (int j = 0; j < kOutPerThread; ++j) {
-        const int o = threadIdx.x + kBlock * j;
-        if (o < outs) partials[static_cast<std::int64_t>(blockIdx.x) * outs + o] = acc[j];
+        for (int u = 0; u < U; ++u) {
+            const bool on = 2 * (p0 + u) + half < n;
+            if constexpr (TANH) a[u] *= 1.0f - hv[u] * hv[u];
+            a[u] = on && m < R ? a[u] : 0.f;
+            sum += a[u];
+#pragma unroll
+            for (int q = 0; q < NB; ++q)
+                acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], on ? b[q][u] : 0.f, acc[q], 0, 0, 0);
+        }
+    }
+    // D: lane l holds column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[wave][q * W * W + (8 * (r >> 2) + 4 * half + (r & 3)) * W + m] = acc[q][r];
+    sum += __shfl_xor(sum, 32, 64);
+    if (half == 0) red[wave][NB * W * W + m] = sum;
+    __syncthreads();
+    const int outs = R * (C0 + (NB == 2 ? C1 : 0)) + R;
+    for (int o = threadIdx.x; o < outs; o += kBlock) {
+        int at;
+        if (o < R * C0) at = (o / C0) * W + o % C0;
+        else if (NB == 2 && o < R * (C0 + C1)) at = W * W + ((o - R * C0) / C1) * W + (o - R * C0) % C1;
+        else at = NB * W * W + (o - (outs - R));
+        partials[static_cast<std::int64_t>(blockIdx.x) * outs + o] = (red[0][at] + red[1][at]) + (red[2][at] + red[3][at]);
     }
 }
 
-// grad[mat + r*C + c] += sum of partials (and grad[vec + r] for the sums).
-__global__ __launch_bounds__(256) void k_outer_finish(const float* __restrict__ partials, int blocks, int R, int C,
-                                                      float* __restrict__ mat, float* __restrict__ vec)
+// The partials' sums in FP64 (blocks in a fixed order: eight strided
+// segments, then the segments in order), added to the gradient: R x C0 values
+// to mat0, R x C1 to mat1, R to vec0 and vec1 (null: not wanted).  A block
+// takes 32 outputs with eight threads each, so a segment's loads are 128-byte
+// runs with eight of them in flight: 5.6 us for 2,080 outputs of 512 blocks
+// (one thread per output took 55 us for 1,056 outputs of 240 blocks).
+__global__ __launch_bounds__(256) void k_outer_finish(const float* __restrict__ partials, int blocks, int R, int C0,
+                                                      int C1, float* __restrict__ mat0, float* __restrict__ mat1,
+                                                      float* __restrict__ vec0, float* __restrict__ vec1)
 {
-    const int outs = R * C + R;
-    const int o = static_cast<int>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (o >= outs) return;
+    __shared__ double seg[8][32];
+    const int outs = R * (C0 + C1) + R;
+    const int t = static_cast<int>(threadIdx.x & 31), g = static_cast<int>(threadIdx.x >> 5);
+    const int o = static_cast<int>(blockIdx.x) * 32 + t;
+    const int oc = o < outs ? o : outs - 1;
     double s = 0.0;
-    for (int k = 0; k < blocks; ++k) s += static_cast<double>(partials[static_cast<std::int64_t>(k) * outs + o]);
-    if (o < R * C) {
-        if (mat) mat[o] += static_cast<float>(s);
-    } else if (vec) {
-        vec[o - R * C] += static_cast<float>(s);
+    for (int k0 = g; k0 < blocks; k0 += 64) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int k = k0 + 8 * u < blocks ? k0 + 8 * u : blocks - 1;
+            v[u] = partials[static_cast<std::int64_t>(k) * outs + oc];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += k0 + 8 * u < blocks ? static_cast<double>(v[u]) : 0.0;
+    }
+    seg[g][t] = s;
+    __syncthreads();
+    if (g != 0 || o >= outs) return;
+#pragma unroll
+    for (int q = 1; q < 8; ++q) s += seg[q][t];
+    const float f = static_cast<float>(s);
+    if (o < R * C0) {
+        mat0[o] += f;
+    } else if (o < R * (C0 + C1)) {
+        mat1[o - R * C0] += f;
+    } else {
+        if (vec0) vec0[o - (outs - R)] += f;
+        if (vec1) vec1[o - (outs - R)] += f;
     }
 }
 
@@ -1095,14 +1142,21 @@ void forward(owtk_gnn model, const GnnGraph& g, float* h, float* agg, float* gam
     OWTK_LAUNCH_CHECK();
 }
 
-void outer_reduce(owtk_gnn model, std::int64_t n, const float* A, int R, const float* B, int C, float* mat, float* vec)
+// The gradients of one layer's matrices and biases (see k_outer_mfma); B1, h,
+// mat1 and the vectors may be null.
+void outer_reduce(owtk_gnn model, std::int64_t n, const float* A, int R, const float* h, const float* B0, int C0,
+                  const float* B1, int C1, float* mat0, float* mat1, float* vec0, float* vec1)
 {
     const hipStream_t st = model->ctx->stream;
-    const int blocks = static_cast<int>(std::max<std::int64_t>(1, std::min<std::int64_t>(kReduceGrid, (n + kTile - 1) / kTile)));
-    k_outer_partials<<<blocks, kBlock, 0, st>>>(n, A, R, B, C, model->partials.get());
+    // 64 vertices per block and pass
+    const int blocks = static_cast<int>(std::max<std::int64_t>(1, std::min<std::int64_t>(kReduceGrid, (n + 63) / 64)));
+    float* partials = model->partials.get();
+    if (B1) k_outer_mfma<2, false><<<blocks, kBlock, 0, st>>>(n, A, R, h, B0, C0, B1, C1, partials);
+    else if (h) k_outer_mfma<1, true><<<blocks, kBlock, 0, st>>>(n, A, R, h, B0, C0, B1, C1, partials);
+    else k_outer_mfma<1, false><<<blocks, kBlock, 0, st>>>(n, A, R, h, B0, C0, B1, C1, partials);
     OWTK_LAUNCH_CHECK();
-    const int outs = R * C + R;
-    k_outer_finish<<<(outs + kBlock - 1) / kBlock, kBlock, 0, st>>>(model->partials.get(), blocks, R, C, mat, vec);
+    const int outs = R * (C0 + C1) + R;
+    k_outer_finish<<<(outs + 31) / 32, kBlock, 0, st>>>(partials, blocks, R, C0, C1, mat0, mat1, vec0, vec1);
     OWTK_LAUNCH_CHECK();
 }
 
@@ -1181,8 +1235,8 @@ void accumulate(owtk_gnn model, owtk_gnn_problem prob, double weight)
     k_gnn_decode_bwd<<<grid, kBlock, 0, st>>>(n, g.b, model->outs, model->dgamma.get(), p16, model->off_w_out,
                                               v.dout, v.dh);
     OWTK_LAUNCH_CHECK();
-    outer_reduce(model, n, v.dout, model->outs, h3, W, grad + model->off_w_out, grad + model->off_b_out);
-    outer_reduce(model, n, v.dout, model->outs, nullptr, 0, nullptr, grad + model->off_g);
+    outer_reduce(model, n, v.dout, model->outs, nullptr, h3, W, nullptr, 0, grad + model->off_w_out, nullptr,
+                 grad + model->off_b_out, grad + model->off_g);
     float* dh = v.dh;
     float* dprev = v.dprev;
     for (int l = kGnnLayers - 1; l >= 0; --l) {
@@ -1193,13 +1247,12 @@ void accumulate(owtk_gnn model, owtk_gnn_problem prob, double weight)
         OWTK_LAUNCH_CHECK();
         k_gnn_agg_t<<<grid, kBlock, 0, st>>>(n, g.offsets.get(), g.cols.get(), g.mirror.get(), g.w.get(), v.v, dprev);
         OWTK_LAUNCH_CHECK();
-        outer_reduce(model, n, v.du, W, hin, W, grad + model->off_ws[l], grad + model->off_b[l]);
-        outer_reduce(model, n, v.du, W, agg, W, grad + model->off_wn[l], nullptr);
+        outer_reduce(model, n, v.du, W, nullptr, hin, W, agg, W, grad + model->off_ws[l], grad + model->off_wn[l],
+                     grad + model->off_b[l], nullptr);
         std::swap(dh, dprev);
     }
-    k_tanh_bwd<<<dev::stream_grid(n * W, 4), kBlock, 0, st>>>(n * W, v.h, dh);
-    OWTK_LAUNCH_CHECK();
-    outer_reduce(model, n, dh, W, g.x.get(), model->f0, grad + model->off_w_in, grad + model->off_b_in);
+    outer_reduce(model, n, dh, W, v.h, g.x.get(), model->f0, nullptr, 0, grad + model->off_w_in, nullptr,
+                 grad + model->off_b_in, nullptr);
 }
 
 void refresh_bf16(owtk_gnn g)

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import owtk
+from oracle import gnn
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,33 @@ def test_row_component_spmv(ctx, block):
     yf = ctx.empty(n * block, np.float32)
     m.spmv(ctx.upload(x.astype(np.float32)), yf, owtk.F32)
     assert np.array_equal(yf.download(), om.spmv_f32(val, diag, x))
+
+
+@pytest.mark.parametrize("nx,ny,block,degree", [(2, 2, 1, 1), (5, 3, 3, 9), (33, 2, 2, 3), (47, 31, 3, 4), (183, 180, 3, 4)])
+def test_training_gradient_sizes(ctx, nx, ny, block, degree):
+    """Vertex counts below one matrix-core step, odd, and beyond one pass of the gradient reduction's grid; 2 to 30
+    outputs.  FP32 sums over at most n vertices of FP32 products: 2e-3 of a block's norm holds with the same margin
+    as at the sizes of the other gradient test."""
+    s = owtk.generate_split(nx, ny, block, 3, ordering=owtk.ORDER_HILBERT)
+    m = owtk.Matrix.split(ctx, s.nodes, 0, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    g = gnn.Graph(s.nodes, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    rng = np.random.default_rng(nx)
+    errs = [rng.uniform(-1, 1, (s.nodes, block)) for _ in range(2)]
+    ress = [g.apply(e) for e in errs]
+    lay = gnn.Layout(block, degree)
+    p = lay.unpack(gnn.init_parameters(block, degree, 1))
+    p["w_out"] = rng.normal(0, 0.3, p["w_out"].shape)
+    for layer in range(gnn.LAYERS):
+        p[f"b{layer}"] = rng.normal(0, 0.2, p[f"b{layer}"].shape)
+    params = lay.pack(p).astype(np.float32)
+    model = owtk.GnnModel(ctx, block, degree)
+    model.set_parameters(params)
+    prob = model.problem(m, ctx.upload(np.concatenate(ress).ravel()), ctx.upload(np.concatenate(errs).ravel()), 2)
+    model.zero_grad()
+    model.accumulate(prob, 1.0)
+    loss, grad = model.read()
+    ref_loss, ref_grad = gnn.loss_and_grad(g, gnn.bf16_round(params), degree, ress, errs)
+    got, ref = lay.unpack(grad.astype(np.float64)), lay.unpack(ref_grad)
+    assert abs(loss - ref_loss) <= 1e-4 * ref_loss
+    for k in ref:
+        assert np.linalg.norm(got[k] - ref[k]) <= 2e-3 * max(np.linalg.norm(ref[k]), 1e-6 * np.linalg.norm(ref_grad)), k
