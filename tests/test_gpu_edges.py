@@ -79,3 +79,46 @@ def test_training_gradient_sizes(ctx, nx, ny, block, degree):
     assert abs(loss - ref_loss) <= 1e-4 * ref_loss
     for k in ref:
         assert np.linalg.norm(got[k] - ref[k]) <= 2e-3 * max(np.linalg.norm(ref[k]), 1e-6 * np.linalg.norm(ref_grad)), k
+
+
+def random_dominant(rng, n, block, low, high):
+    """A diagonally dominant CSR matrix with low..high off-diagonal entries per row at random columns near the
+    diagonal (no symmetric pattern)."""
+    offsets, columns, values = [0], [], []
+    for i in range(n):
+        near = np.setdiff1d(np.arange(max(0, i - 40), min(n, i + 41)), [i])
+        own = rng.choice(near, min(rng.integers(low, high + 1), near.size), replace=False)
+        cols = np.sort(np.concatenate([own, [i]]))
+        val = -rng.uniform(0.1, 1.0, (cols.size, block))
+        val[cols == i] = np.abs(val).sum(0) + 0.5
+        columns.append(cols)
+        values.append(val)
+        offsets.append(offsets[-1] + cols.size)
+    return np.array(offsets, np.int32), np.concatenate(columns).astype(np.int32), np.concatenate(values).ravel()
+
+
+@pytest.mark.parametrize("case", ["1-node", "grid-1", "grid-2", "grid-3", "grid-4-rcm", "sparse", "wide", "wider", "dense"])
+def test_red_black_coarse_sweeps(ctx, case):
+    """Red-black multigrid against the oracle after two V cycles: one-chunk and partial chunks, 1 to 4 components,
+    coarse rows of 4 to 16 entries (each slot count of the one-wave sweep), longer ones and unsymmetric patterns
+    (several red levels, the workgroup sweep).  The sweeps keep the oracle's operations and their order; the fine
+    SpMV and the residual sums bound the difference: 1e-13, as for the other multigrid solves."""
+    rng = np.random.default_rng(len(case))
+    if case == "1-node":
+        n, block, off, col, val = 1, 2, np.array([0, 1], np.int32), np.array([0], np.int32), np.array([2.0, 3.0])
+    elif case.startswith("grid"):
+        block = int(case[5])
+        order = owtk.ORDER_RCM if case.endswith("rcm") else owtk.ORDER_HILBERT
+        s = owtk.generate_split(61, 37, block, 2, ordering=order)
+        n, (off, col, val) = s.nodes, s.csr()
+    else:
+        low, high = {"sparse": (0, 2), "wide": (4, 6), "wider": (6, 9), "dense": (20, 30)}[case]
+        n, block = 500, 2
+        off, col, val = random_dominant(rng, n, block, low, high)
+    b = rng.uniform(-1, 1, n * block)
+    kw = dict(relative_tolerance=1e-300, maximum_iterations=2)
+    xo, _ = orc.OMultigrid(orc.OMatrix.csr(n, 0, block, off, col, val), smoother=1).solve(b, cycle=0, **kw)
+    m = owtk.Matrix.csr(ctx, n, 0, block, off, col, val)
+    x = ctx.empty(n * block)
+    owtk.Multigrid(m, smoother=owtk.MG_RED_BLACK).solve(ctx.upload(b), x, owtk.SolverOptions(**kw))
+    assert np.max(np.abs(x.download() - xo)) <= 1e-13 * np.max(np.abs(xo))
