@@ -25,8 +25,6 @@ namespace {
 using dev::kBlock;
 
 constexpr double kTol = 64.0 * std::numeric_limits<double>::epsilon();
-// LDS per chain workgroup above which the block's solution stays in global memory
-constexpr std::size_t kChainLdsBudget = 24 * 1024;
 
 enum Flag : int { flag_ok = 0, flag_zero_pivot = 1, flag_singular_diag = 2, flag_no_diag = 3 };
 
@@ -281,8 +279,6 @@ struct TriArgs {
     const std::int64_t* bptr;
     const std::int32_t* fcol;
     const std::int32_t* bcol;
-    const std::int32_t* fnout;
-    const std::int32_t* bnout;
     std::int64_t fnnz, bnnz, rows;
     int bs;
 };
@@ -726,157 +722,44 @@ __global__ __launch_bounds__(256) void k_tri_apply(TriArgs a, const V* __restric
     }
 }
 
-__device__ inline double lane_value(double v, int lane)
-{
-    const long long bits = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane(static_cast<int>(bits), lane);
-    const int hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), lane);
-    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-
-__device__ inline float lane_value(float v, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
-// One sweep of a chain-scheduled triangular solve by one wave.  Rows are
-// taken in chunks of 64 in sweep order (ascending rows forward, descending
-// backward), lane l owning the chunk's l-th row.  Each row's entries are
-// stored as [entries whose row lies before the chunk] then [entries inside
-// the chunk, by the step at which that row is finished].  The first group is
-// final already and read from LDS.  The second group is scattered into an
-// LDS tile, tile[step][lane] = coefficient (zero elsewhere); step s then
-// broadcasts lane s's finished value with v_readlane and every lane folds in
-// its tile entry for step s.  A lane's entries all precede its own step, so
-// its value is final from its step on and is stored once at the chunk end.
-// Forward sweeps of sorted rows accumulate in the reference's order; backward
-// sweeps take their in-chunk entries in the order they become available.
-template<TriMode MODE, bool FWD, class X, class V, int EI>
-__device__ inline void chain_sweep(const std::int64_t* __restrict__ ptr, const std::int32_t* __restrict__ nout,
-                                   const std::int32_t* __restrict__ cols, const V* __restrict__ vals,
-                                   const X* __restrict__ dv, X* y, int ys, X* tile, int nb, int lane)
-{
-    for (int cs = 0; cs < nb; cs += 64) {
-        const int p = cs + lane;
-        const bool valid = p < nb;
-        const int i = FWD ? p : nb - 1 - p;
-        X acc = X(0);
-        X dmine = X(1);
-        int st[EI];
-#pragma unroll
-        for (int k = 0; k < EI; ++k) st[k] = -1;
-        if (valid) {
-            const std::int64_t e0 = ptr[p];
-            const std::int64_t e1 = ptr[p + 1];
-            const std::int64_t em = e0 + nout[p];
-            if constexpr (MODE == TriMode::ssor || !FWD) dmine = dv[i];
-            if constexpr (MODE == TriMode::ssor && !FWD) acc = dmine * y[i * ys];
-            else acc = y[i * ys];
-            for (std::int64_t e = e0; e < em; ++e)
-                acc = dev::dfma(-static_cast<X>(vload(vals, e)), y[static_cast<std::int64_t>(cols[e]) * ys], acc);
-#pragma unroll
-            for (int k = 0; k < EI; ++k) {
-                if (em + k < e1) {
-                    const int c = cols[em + k];
-                    st[k] = FWD ? c - cs : nb - 1 - cs - c;
-                    tile[st[k] * 64 + lane] = static_cast<X>(vload(vals, em + k));
-                }
-            }
-        }
-        __syncthreads();
-        const int steps = nb - cs < 64 ? nb - cs : 64;
-#pragma unroll
-        for (int s = 0; s < 64; ++s) {
-            if (s < steps) {
-                const X coef = tile[s * 64 + lane];
-                X fin;
-                if constexpr (MODE == TriMode::ssor) fin = acc / dmine;
-                else if constexpr (!FWD) fin = acc * dmine;
-                else fin = acc;
-                const X v = lane_value(fin, s);
-                acc = coef != X(0) ? dev::dfma(-coef, v, acc) : acc;
-            }
-        }
-        X mine;
-        if constexpr (MODE == TriMode::ssor) mine = acc / dmine;
-        else if constexpr (!FWD) mine = acc * dmine;
-        else mine = acc;
-        if (valid) y[i * ys] = mine;
-#pragma unroll
-        for (int k = 0; k < EI; ++k)
-            if (st[k] >= 0) tile[st[k] * 64 + lane] = X(0);
-        __syncthreads();
-    }
-}
-
-// GLOBAL_Y: the block's solution lives in `out` itself (L2-resident, strided by
-// the block size) instead of LDS, so a workgroup needs only the 64 x 64 tile
-// and more of them fit on a CU.  The block's rows belong to this one wave, so
-// no other wave reads or writes them.
-template<TriMode MODE, class X, class V, int EI, bool GLOBAL_Y>
-__global__ __launch_bounds__(64) void k_tri_chain(TriArgs a, const V* __restrict__ fval, const V* __restrict__ bval,
-                                                  const X* __restrict__ dval, const X* in, X* out, X scale,
-                                                  const int* stop)
-{
-    extern __shared__ unsigned char smem_raw[];
-    if (stop && *stop) return;
-    const int bs = a.bs;
-    const int c = blockIdx.x % bs;
-    const int b = blockIdx.x / bs;
-    const std::int64_t r0 = a.row0[b];
-    const int nb = a.nrows[b];
-    const int lane = threadIdx.x;
-    X* tile = reinterpret_cast<X*>(smem_raw);  // [64 steps][64 lanes]
-    for (int s = 0; s < 64; ++s) tile[s * 64 + lane] = X(0);
-    X* y;
-    int ys;
-    if constexpr (GLOBAL_Y) {
-        y = out + r0 * bs + c;
-        ys = bs;
-        if (in != out)
-            for (int i = lane; i < nb; i += 64) y[i * ys] = in[(r0 + i) * bs + c];
-    } else {
-        y = tile + 64 * 64;  // [nb]
-        ys = 1;
-        for (int i = lane; i < nb; i += 64) y[i] = in[(r0 + i) * bs + c];
-    }
-    __syncthreads();
-    const X* dv = dval + static_cast<std::int64_t>(c) * a.rows + r0;
-    chain_sweep<MODE, true, X, V, EI>(a.fptr + r0, a.fnout + r0, a.fcol, fval + static_cast<std::int64_t>(c) * a.fnnz,
-                                      dv, y, ys, tile, nb, lane);
-    chain_sweep<MODE, false, X, V, EI>(a.bptr + r0, a.bnout + r0, a.bcol,
-                                       bval + static_cast<std::int64_t>(c) * a.bnnz, dv, y, ys, tile, nb, lane);
-    const bool scaled = MODE == TriMode::ssor && scale != X(1);
-    if (GLOBAL_Y && !scaled) return;
-    for (int i = lane; i < nb; i += 64) {
-        X v = y[i * ys];
-        if (scaled) v = v * scale;
-        out[(r0 + i) * bs + c] = v;
-    }
-}
-
-// Chain sweeps over an ELL copy of the factors.  A sweep's rows are cut into
-// the same 64-row chunks; for chunk g and slot k < K the 64 rows' k-th entry
-// (chain order) is contiguous: idx[(g*K + k)*64 + lane] and
-// val[c][(g*K + k)*64 + lane].  idx >= 0: block-local column of an entry on a
-// row of an earlier chunk; idx <= -2: in-chunk entry finished at step
-// -idx - 2; -1: padding.  A chunk's description is then K coalesced 16-bit
-// loads with no pointer chase: the next chunk's indices are fetched at the
-// start of a chunk and its values (only the slots that hold an entry) at its
-// end, so both are in flight during the chunk's 64 steps.  In-chunk
-// coefficients go to a packed strictly-lower-triangular LDS tile (position p
-// only depends on steps s < p), half the dense tile, so more one-wave
-// workgroups fit per CU.
-__host__ __device__ constexpr int tri_base(int s) { return (s * (127 - s)) / 2; }  // first packed entry of step s
-
-// The sweep's workgroup is one wave.  LDS instructions of a wave complete in
-// issue order, and so do its vector memory instructions to one address, so
-// lanes see each other's earlier tile and solution writes without a
-// workgroup barrier; only the compiler must keep the order.  (__syncthreads
-// would also wait for every outstanding load, including the next chunk's
-// prefetch.)
-__device__ inline void wave_order() { __asm__ volatile("" ::: "memory"); }
-
+// ------------------------------------------------------------ chain sweeps --
+// Triangular sweeps over blocks whose rows form long dependency chains
+// (Hilbert-ordered blocks of 4,096 rows have about 3,500 levels): one row
+// after the other, at the latency of one instruction per row.
+//
+// A wave walks four chains, one (block, component) per DPP row of 16 lanes,
+// in chunks of 16 rows in sweep order (ascending rows forward, descending
+// backward), lane l of a group owning the chunk's l-th row.  The 15 in-chunk
+// steps are one instruction each: step s broadcasts lane s's finished value
+// within its group and every later lane subtracts it times its coefficient
+// (v_fmac with row_newbcast: 16 clocks a step; a 64-row chunk per wave with
+// the value broadcast through scalar registers took 23 and an LDS read).  A
+// lone wave issues one instruction in four clocks, so a second wave of the
+// workgroup, on another SIMD, prepares the next chunk: it scatters the
+// in-chunk coefficients and gathers the old rows, and the first wave is left
+// with its K near entries, the steps and the results.
+//
+// The host classifies every entry by where its solution value comes from
+// (build_rows16), so a chunk is branch-free but for its far entries:
+//   in-chunk  the coefficient goes to the LDS tile, tile[step][lane]; zeros
+//             elsewhere keep a finished row's value;
+//   near      a row of the last 27 chunks, from an LDS ring of the chunks'
+//             results (the ring's zero for in-chunk entries and padding);
+//   far       an older row (2% of the entries of a Hilbert-ordered grid, none
+//             where a block's bandwidth is below 432 rows), gathered from the
+//             solution P chunks ahead, when any lane of the wave has one, and
+//             handed over in LDS.
+// Entries fold in slot order, then the in-chunk steps, which for sorted rows
+// is the reference's order in the forward sweep; backward sweeps take their
+// entries in the order the rows finish.
+//
+// Measured (FP64, the earlier 64-row sweep in brackets): ILU(0) apply at 2M
+// vertices, block 3, 4,096-row blocks 225 (284) us; 2,048 vertices,
+// 512-row blocks 16.5 (24.4) us; SSOR of 1,296 components on a
+// 32 x 32 grid 46.6 (73) us.  A lone chunk takes about 0.25 us, 243 clocks of
+// it the steps; with 384 workgroups running, the padded values and codes (about
+// 1 GB an apply) add memory time.  One wave doing all of this took 266 us, and
+// a third wave touching the coming chunks' lines 282 us.
 template<class X>
 __device__ inline X chain_finish(X acc, X, X, std::integral_constant<int, 0>)  // ILU forward: unit diagonal
 {
@@ -902,248 +785,382 @@ __device__ inline X chain_finish(X acc, X d, X rinv, std::integral_constant<int,
 template<TriMode MODE, bool FWD>
 using FinishKind = std::integral_constant<int, MODE == TriMode::ssor ? 2 : (FWD ? 0 : 1)>;
 
-// A 64-bit value from another lane chosen per lane (ds_bpermute); every lane
-// of the wave must execute it.
-template<class X>
-__device__ inline X lane_pick(X v, int src)
-{
-    if constexpr (sizeof(X) == 8) {
-        const long long bits = __double_as_longlong(v);
-        const int lo = __shfl(static_cast<int>(bits), src, 64);
-        const int hi = __shfl(static_cast<int>(bits >> 32), src, 64);
-        return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-    } else {
-        return __shfl(v, src, 64);
+// The 15 in-chunk steps: at step s every lane subtracts its coefficient times
+// the finished value of its group's lane s (see chain_finish), rounded once.
+// A DPP operand may not have been written by the two vector instructions
+// before, hence the wait states; one block, because the compiler adds another
+// to every inline statement it puts between.  (KIND as FinishKind.)
+#define OWTK_STEP0(T, S) "s_nop 1\n\tv_fmac_" T "_dpp %0, -%0, %[c" #S "] row_newbcast:" #S " row_mask:0xf bank_mask:0xf\n\t"
+#define OWTK_STEP1(T, S)                                                                                              \
+    "v_mul_" T " %[t], %0, %[d]\n\ts_nop 1\n\tv_fmac_" T "_dpp %0, -%[t], %[c" #S "] row_newbcast:" #S             \
+    " row_mask:0xf bank_mask:0xf\n\t"
+#define OWTK_STEP2(T, S)                                                                                              \
+    "v_mul_" T " %[t], %0, %[r]\n\tv_fma_" T " %[u], -%[t], %[d], %0\n\tv_fma_" T " %[t], %[u], %[r], %[t]\n\t"   \
+    "s_nop 1\n\tv_fmac_" T "_dpp %0, -%[t], %[c" #S "] row_newbcast:" #S " row_mask:0xf bank_mask:0xf\n\t"
+#define OWTK_STEPS(M, T)                                                                                              \
+    M(T, 0) M(T, 1) M(T, 2) M(T, 3) M(T, 4) M(T, 5) M(T, 6) M(T, 7) M(T, 8) M(T, 9) M(T, 10) M(T, 11) M(T, 12) M(T, 13) \
+        M(T, 14)
+#define OWTK_COEFS                                                                                                    \
+    [c0] "v"(c[0]), [c1] "v"(c[1]), [c2] "v"(c[2]), [c3] "v"(c[3]), [c4] "v"(c[4]), [c5] "v"(c[5]), [c6] "v"(c[6]),    \
+        [c7] "v"(c[7]), [c8] "v"(c[8]), [c9] "v"(c[9]), [c10] "v"(c[10]), [c11] "v"(c[11]), [c12] "v"(c[12]),         \
+        [c13] "v"(c[13]), [c14] "v"(c[14])
+#define OWTK_CHAIN_STEPS(X, T)                                                                                        \
+    template<int KIND>                                                                                                \
+    __device__ inline void chain_steps(X& acc, const X (&c)[15], X d, X rinv)                                         \
+    {                                                                                                                 \
+        X t, u;                                                                                                       \
+        if constexpr (KIND == 0) __asm__(OWTK_STEPS(OWTK_STEP0, T) : "+v"(acc) : OWTK_COEFS);                         \
+        else if constexpr (KIND == 1)                                                                                 \
+            __asm__(OWTK_STEPS(OWTK_STEP1, T) : "+v"(acc), [t] "=&v"(t) : OWTK_COEFS, [d] "v"(d));                    \
+        else                                                                                                          \
+            __asm__(OWTK_STEPS(OWTK_STEP2, T)                                                                         \
+                    : "+v"(acc), [t] "=&v"(t), [u] "=&v"(u)                                                           \
+                    : OWTK_COEFS, [d] "v"(d), [r] "v"(rinv));                                                         \
     }
-}
+OWTK_CHAIN_STEPS(double, "f64")
+OWTK_CHAIN_STEPS(float, "f32")
+#undef OWTK_STEP0
+#undef OWTK_STEP1
+#undef OWTK_STEP2
+#undef OWTK_STEPS
+#undef OWTK_COEFS
+#undef OWTK_CHAIN_STEPS
 
-// One sweep over the ELL copy.  The host classifies every slot (see
-// build_ell), so the chunk set-up is branch-free:
-//   idx >= 0              entry on a chunk before q-1: block-local row of y,
-//                         loaded one chunk ahead (it is final by then);
-//   -2018 <= idx <= -3    in-chunk entry: its value goes to packed tile
-//                         entry -idx - 2;
-//   idx <= -2019          entry on chunk q-1: lane -idx - 2019 of that
-//                         chunk, taken from the lanes' final values by a
-//                         cross-lane shuffle;
-//   idx == -1             padding (value 0, contributes nothing).
-// Every slot's index and value is loaded (padding values are zeros), tile
-// writes of other kinds go to a spare LDS entry, and out-of-chunk
-// contributions are selected, not branched on.  Indices are loaded two
-// chunks ahead, values, own row value, diagonal and older y one chunk ahead.
-// Each row folds its out-of-chunk entries in slot order, then the in-chunk
-// steps.  The steps read their tile coefficients at per-lane addresses
-// computed once per kernel (taddr), so a step is one LDS read, the
-// broadcast and one FMA.
-template<TriMode MODE, bool FWD, class X, class V, int E>
-__device__ __attribute__((always_inline)) inline void ell_sweep(const std::int16_t* __restrict__ idx, const V* __restrict__ val, std::int64_t g0,
-                                 const X* __restrict__ dv, X* y, int ys, X* tri, const int (&taddr)[64], int nb,
-                                 int lane)
-{
-    constexpr int kTrash = 1 + tri_base(64);  // spare tile entry for writes that are not in-chunk
-    const int chunks = (nb + 63) >> 6;
-    constexpr std::int64_t stride = static_cast<std::int64_t>(E) * 64;  // one chunk's slots
-    auto row_of = [&](int pos) { return FWD ? pos : nb - 1 - pos; };
-    auto load_idx = [&](int q, int (&out)[E]) {
-        const std::int64_t base = (g0 + (q < chunks ? q : chunks - 1)) * stride + lane;
-#pragma unroll
-        for (int k = 0; k < E; ++k) out[k] = static_cast<int>(__builtin_nontemporal_load(&idx[base + k * 64]));
-    };
-    auto load_val = [&](int q, X (&out)[E]) {
-        const std::int64_t base = (g0 + (q < chunks ? q : chunks - 1)) * stride + lane;
-#pragma unroll
-        for (int k = 0; k < E; ++k) out[k] = static_cast<X>(vload(val, base + k * 64));
-    };
-    // older entries' y, for the slots of the chunk whose indices are `ix`
-    auto load_old = [&](const int (&ix)[E], X (&out)[E]) {
-#pragma unroll
-        for (int k = 0; k < E; ++k) out[k] = y[static_cast<std::int64_t>(ix[k] > 0 ? ix[k] : 0) * ys];
-    };
-    int ci[E], ni[E];
-    X cv[E], pyo[E];
-    load_idx(0, ci);
-    load_idx(1, ni);
-    load_val(0, cv);
-#pragma unroll
-    for (int k = 0; k < E; ++k) pyo[k] = X(0);  // chunk 0 has no older chunks
-    const int p0 = lane < nb ? lane : nb - 1;
-    X cd = X(1);
-    if constexpr (MODE == TriMode::ssor || !FWD) cd = dv[row_of(p0)];
-    X cacc = lane < nb ? y[row_of(p0) * ys] : X(0);
-    X yprev = X(0);  // chunk q-1's final value of this lane's row
-    for (int q = 0; q < chunks; ++q) {
-        const int p = q * 64 + lane;
-        const bool valid = p < nb;
-        // chunk q+1 (indices of q+2), in flight during this chunk's steps
-        int nni[E];
-        load_idx(q + 2, nni);
-        X ncv[E], npyo[E];
-        load_val(q + 1, ncv);
-        const int pn = p + 64 < nb ? p + 64 : nb - 1;
-        X nacc = y[row_of(pn) * ys], nd = X(1);
-        if constexpr (MODE == TriMode::ssor || !FWD) nd = dv[row_of(pn)];
-        // in-chunk coefficients to the tile
-#pragma unroll
-        for (int k = 0; k < E; ++k) tri[ci[k] <= -3 && ci[k] >= -2018 ? -ci[k] - 2 : kTrash] = cv[k];
-        X acc = cacc;
-        if constexpr (MODE == TriMode::ssor && !FWD) acc = cd * acc;
-#pragma unroll
-        for (int k = 0; k < E; ++k) {
-            const X sh = lane_pick(yprev, (-ci[k] - 2019) & 63);
-            const X yo = ci[k] >= 0 ? pyo[k] : sh;
-            const X upd = dev::dfma(-cv[k], yo, acc);
-            acc = ci[k] >= 0 || ci[k] <= -2019 ? upd : acc;
-        }
-        // Chunk q-1's results are stored only now, after the wait for the
-        // loads above: stores count with the loads in vmcnt, so a store
-        // issued before them would be waited for there.  The loads of chunk
-        // q+1's entries on chunks before q (q-1 among them) follow the store
-        // (one wave's accesses to one address stay in order); the next wait
-        // for them is a whole chunk of steps later.
-        if (q > 0) y[row_of(p - 64) * ys] = yprev;
-        load_old(ni, npyo);
-        X rinv = X(1);
-        if constexpr (MODE == TriMode::ssor) rinv = X(1) / cd;
-        wave_order();
-        // step st: lane st's row is final; every later lane folds it in with
-        // its tile coefficient (lanes at or before st read the zero guard, so
-        // a finished row keeps its value)
-        const int steps = nb - q * 64 < 64 ? nb - q * 64 : 64;
-        if (steps == 64) {
-#pragma unroll
-            for (int st = 0; st < 64; ++st) {
-                const X coef = tri[taddr[st]];
-                const X v = lane_value(chain_finish(acc, cd, rinv, FinishKind<MODE, FWD>{}), st);
-                acc = dev::dfma(-coef, v, acc);
-            }
-        } else {
-            for (int st = 0; st < steps; ++st) {
-                const X coef = tri[lane > st ? tri_base(st) + lane - st : 0];
-                const X v = lane_value(chain_finish(acc, cd, rinv, FinishKind<MODE, FWD>{}), st);
-                acc = dev::dfma(-coef, v, acc);
-            }
-        }
-        const X fin = chain_finish(acc, cd, rinv, FinishKind<MODE, FWD>{});
-        yprev = valid ? fin : X(0);
-        if (q + 1 == chunks && valid) y[row_of(p) * ys] = fin;  // the last chunk's results
-#pragma unroll
-        for (int k = 0; k < E; ++k) tri[ci[k] <= -3 && ci[k] >= -2018 ? -ci[k] - 2 : kTrash] = X(0);
-#pragma unroll
-        for (int k = 0; k < E; ++k) {
-            ci[k] = ni[k];
-            ni[k] = nni[k];
-            cv[k] = ncv[k];
-            pyo[k] = npyo[k];
-        }
-        cacc = nacc;
-        cd = nd;
-        wave_order();
-    }
-}
+// LDS of a workgroup, bytes.  Elements sit 8 bytes apart in either precision,
+// so the host's codes serve both.  Per group: 28 ring entries of 16 results,
+// the zero entry, then the far values [parity][K][16]; behind the groups, for
+// even and odd chunks, the tile [15 steps and a spare row][64 lanes] and the
+// right-hand side, diagonal and reciprocal [3][64 lanes].
+constexpr int kRing16 = 28, kRingZero = kRing16 * 128, kFar16 = 4096;
+constexpr int kGroup16 = 8192 + 128;  // the groups' entries start on different LDS banks
+constexpr int kTile16 = 4 * kGroup16, kTileSpare = kTile16 + 15 * 512, kTileBytes = 16 * 512;
+constexpr int kRow16 = kTile16 + 2 * kTileBytes, kRowBytes = 3 * 512, kLds16 = kRow16 + 2 * kRowBytes;
+constexpr int chunks_ahead(int k) { return k <= 8 ? 4 : 2; }  // P, even
+constexpr int kPadChunks16 = 16;  // idle chunks behind the last block: loads run ahead of the sweep
 
-struct EllArgs {
-    const std::int32_t* chunk0;  // [blocks] first global chunk of each block
-    const std::int16_t* fidx;
-    const std::int16_t* bidx;
-    std::int64_t fslots, bslots;  // values per component: chunks * K * 64
-    int fk, bk;                   // slots per row of each sweep (both the kernel's E)
+struct Rows16Args {
+    const std::int32_t* row0;
+    const std::int32_t* nrows;
+    // per sweep, [chunk * 16 + lane][K]: LDS address of an entry's value (near,
+    // within the group) and of its coefficient's tile entry (less the lane's
+    // 8 bytes), and the block-local far row (-1 none)
+    const std::uint16_t *fnear, *bnear, *ftile, *btile;
+    const std::int16_t *ffar, *bfar;
+    std::int64_t slots;         // values per component and sweep: chunks * K * 16
+    std::int64_t rows;
+    int chains, block_chunks;   // blocks * bs; chunks each block has room for
+    int bs;
 };
 
-// Two waves per SIMD at least (at most 256 VGPRs), so all 1,536 one-wave
-// workgroups of a 2M-vertex, 3-component apply in 4096-vertex blocks are
-// resident at once.
-template<TriMode MODE, class X, class V, int E, bool GLOBAL_Y>
-__global__ __launch_bounds__(64, 2) void k_tri_ell(TriArgs a, EllArgs l, const V* __restrict__ fval,
-                                                const V* __restrict__ bval, const X* __restrict__ dval, const X* in,
-                                                X* out, X scale, const int* stop)
+template<class V> struct alignas(2 * sizeof(V)) Pair { V v[2]; };
+// a row's K 16-bit codes, two to a word (the low half first)
+template<int K> struct Codes { std::uint32_t w[K / 2]; };
+template<int K> __device__ inline unsigned int code_of(const Codes<K>& c, int k)
 {
-    extern __shared__ unsigned char smem_raw[];
-    if (stop && *stop) return;
-    const int bs = a.bs;
-    // the bs component waves of one block on one XCD: they read the same indices
-    const unsigned int wg = kern::xcd_block(blockIdx.x, gridDim.x);
-    const int c = static_cast<int>(wg % bs);
-    const int b = static_cast<int>(wg / bs);
-    const std::int64_t r0 = a.row0[b];
-    const int nb = a.nrows[b];
-    const int lane = threadIdx.x;
-    constexpr int kTri = 2 + tri_base(64);  // guard entry, packed triangle, spare entry
-    X* tri = reinterpret_cast<X*>(smem_raw);
-    for (int s = lane; s < kTri; s += 64) tri[s] = X(0);
-    X* y;
-    int ys;
-    if constexpr (GLOBAL_Y) {
-        y = out + r0 * bs + c;
-        ys = bs;
-    } else {
-        y = tri + kTri;  // [nb]
-        ys = 1;
-    }
-    // the right-hand side into y, 16 loads in flight per lane (in and out
-    // may be one vector, so a plain loop would wait for each load in turn)
-    if (!GLOBAL_Y || in != out) {
-        for (int i0 = 0; i0 < nb; i0 += 16 * 64) {
-            const bool full = i0 + 16 * 64 <= nb;  // whole batches store without per-lane branches
-            X v[16];
+    return k & 1 ? c.w[k / 2] >> 16 : c.w[k / 2] & 0xffffU;
+}
+
+// What the two waves of a workgroup share in a sweep; pointers are the lane's.
+template<class X, class V>
+struct Rows16Sweep {
+    const std::uint16_t* __restrict__ near;
+    const std::uint16_t* __restrict__ tile;
+    const std::int16_t* __restrict__ far;
+    const V* __restrict__ val;
+    const X* __restrict__ dv;  // diagonal of the chain's row 0
+    const X* src;              // right-hand side
+    X* y;                      // solution
+    int first, last;           // byte offsets of the chain's first and last row in src and y
+    int row_bytes;
+    unsigned char* lds;
+    int rows, stored;          // rows of the chain; rows to store (0: a group past the last chain)
+    int chunks;                // of the wave's longest chain, rounded up to P
+    int full;                  // chunks whose 64 rows are all stored
+    int lane;
+    __device__ X& at(unsigned int byte) const { return *reinterpret_cast<X*>(lds + byte); }
+};
+
+// One barrier a chunk.  Only LDS is handed over, so only LDS is waited for:
+// the loads of later chunks stay in flight.
+__device__ inline void chunk_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The preparing wave: during chunk q it writes the tile, right-hand side and
+// diagonal of chunk q + 2 (the solving wave reads chunk q + 1's then) and the
+// far values of chunk q + 1.  Codes, values and rows of a chunk load P chunks ahead, the
+// far rows' numbers 2P.  A far row is stored at least 28 - P - 2 chunks
+// before its gather is issued, and the storing wave has since waited for
+// loads it issued after that store.
+template<TriMode MODE, bool FWD, class X, class V, int K>
+__device__ __attribute__((always_inline)) inline void rows16_prepare(const Rows16Sweep<X, V>& s)
+{
+    constexpr int P = chunks_ahead(K);
+    constexpr bool kDiag = MODE == TriMode::ssor || !FWD;
+    const int l = s.lane & 15;
+    const unsigned int group = static_cast<unsigned int>(s.lane >> 4) * kGroup16;
+    const unsigned int lane8 = static_cast<unsigned int>(s.lane) * 8;
+    const auto* pc = reinterpret_cast<const Codes<K>*>(s.tile) + l;
+    const auto* pf = reinterpret_cast<const Codes<K>*>(s.far) + l;
+    const auto* pv = reinterpret_cast<const Pair<V>*>(s.val) + l;
+    Codes<K> cc[P], fr[P];
+    X cv[P][K], xo[P][K], rr[P], dd[P];
+    unsigned int used[2][K];    // tile entries of the last chunk of each parity
+    unsigned int far_mask = 0;  // bit t: stage t has far entries (wave-uniform)
+    int p = l;                  // position and byte offset of the next chunk's row
+    int off = FWD ? s.first + l * s.row_bytes : s.last - l * s.row_bytes;
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int i = i0 + u * 64 + lane;
-                v[u] = in[(r0 + (i < nb ? i : nb - 1)) * bs + c];
+    for (int k = 0; k < K; ++k) used[0][k] = used[1][k] = kTileSpare + lane8;
+    auto load_far = [&](int t) {
+        fr[t] = *pf;
+        pf += 16;
+    };
+    // the next chunk into stage t, its far rows' numbers already there
+    auto load_chunk = [&](int t) {
+        std::uint32_t none = 0x80008000U;
+#pragma unroll
+        for (int k = 0; k < K / 2; ++k) none &= fr[t].w[k];
+        far_mask &= ~(1U << t);
+        if (__builtin_amdgcn_ballot_w64(none != 0x80008000U) != 0) {
+            far_mask |= 1U << t;
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int code = static_cast<std::int16_t>(code_of<K>(fr[t], k));
+                const unsigned int at = static_cast<unsigned int>(s.first + (code > 0 ? code : 0) * s.row_bytes);
+                xo[t][k] = *reinterpret_cast<const X*>(reinterpret_cast<const char*>(s.y) + at);
             }
-            if (full) {
+        }
+        cc[t] = *pc;
+        pc += 16;
 #pragma unroll
-                for (int u = 0; u < 16; ++u) y[(i0 + u * 64 + lane) * ys] = v[u];
+        for (int j = 0; j < K / 2; ++j) {
+            const Pair<V> u = pv[j * 16];
+            cv[t][2 * j] = static_cast<X>(vload(u.v, 0));
+            cv[t][2 * j + 1] = static_cast<X>(vload(u.v, 1));
+        }
+        pv += (K / 2) * 16;
+        const int at = FWD ? min(off, s.last) : max(off, s.first);
+        off = FWD ? off + 16 * s.row_bytes : off - 16 * s.row_bytes;
+        rr[t] = *reinterpret_cast<const X*>(reinterpret_cast<const char*>(s.src) + static_cast<unsigned int>(at));
+        dd[t] = X(1);
+        if constexpr (kDiag) {
+            const int q = min(p, s.rows - 1);
+            dd[t] = s.dv[FWD ? q : s.rows - 1 - q];
+            p += 16;
+        }
+    };
+    // the far values of stage t's chunk; the solving wave reads them at the
+    // start of that chunk, so they go out one chunk later than the tile
+    auto hand_far = [&](int t) {
+        if (far_mask >> t & 1U) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) s.at(group + kFar16 + ((t & 1) * K + k) * 128 + l * 8) = xo[t][k];
+        }
+    };
+    // the chunk of stage t into the LDS of its parity
+    auto build = [&](int t) {
+        const int par = t & 1;
+#pragma unroll
+        for (int k = 0; k < K; ++k) s.at(used[par][k]) = X(0);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            used[par][k] = code_of<K>(cc[t], k) + (lane8 + par * kTileBytes);
+            s.at(used[par][k]) = cv[t][k];
+        }
+        X r0 = rr[t];
+        if constexpr (MODE == TriMode::ssor && !FWD) r0 = dd[t] * r0;
+        s.at(kRow16 + par * kRowBytes + lane8) = r0;
+        if constexpr (kDiag) s.at(kRow16 + par * kRowBytes + 512 + lane8) = dd[t];
+        if constexpr (MODE == TriMode::ssor) s.at(kRow16 + par * kRowBytes + 1024 + lane8) = X(1) / dd[t];
+    };
+#pragma unroll
+    for (int t = 0; t < P; ++t) load_far(t);
+#pragma unroll
+    for (int t = 0; t < P; ++t) {
+        load_chunk(t);
+        load_far(t);
+    }
+    build(0);
+    __syncthreads();
+    load_chunk(0);
+    load_far(0);
+    build(1);
+    __syncthreads();  // the solving wave has read chunk 0's tile
+    for (int q0 = 0; q0 < s.chunks; q0 += P) {
+#pragma unroll
+        for (int t = 0; t < P; ++t) {
+            // stage t + 1 (chunk q0 + t + 1) is built: hand its far values over
+            // and refill it, build chunk q0 + t + 2
+            hand_far((t + 1) % P);
+            load_chunk((t + 1) % P);
+            load_far((t + 1) % P);
+            build((t + 2) % P);
+            chunk_barrier();
+        }
+    }
+    // an empty tile for the next sweep
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        s.at(used[0][k]) = X(0);
+        s.at(used[1][k]) = X(0);
+    }
+    __syncthreads();
+}
+
+// The solving wave.  It reads the next chunk's coefficients, right-hand side
+// and diagonal during a chunk's steps, so a chunk starts with its near reads.
+template<TriMode MODE, bool FWD, class X, class V, int K>
+__device__ __attribute__((always_inline)) inline void rows16_solve(const Rows16Sweep<X, V>& s)
+{
+    constexpr int P = chunks_ahead(K);
+    constexpr bool kDiag = MODE == TriMode::ssor || !FWD;
+    const int l = s.lane & 15;
+    const unsigned int group = static_cast<unsigned int>(s.lane >> 4) * kGroup16;
+    const unsigned int lane8 = static_cast<unsigned int>(s.lane) * 8;
+    const auto* pc = reinterpret_cast<const Codes<K>*>(s.near) + l;
+    const auto* pv = reinterpret_cast<const Pair<V>*>(s.val) + l;
+    Codes<K> cc[P];
+    X cv[P][K];
+    auto load_chunk = [&](int t) {
+        cc[t] = *pc;
+        pc += 16;
+#pragma unroll
+        for (int j = 0; j < K / 2; ++j) {
+            const Pair<V> u = pv[j * 16];
+            cv[t][2 * j] = static_cast<X>(vload(u.v, 0));
+            cv[t][2 * j + 1] = static_cast<X>(vload(u.v, 1));
+        }
+        pv += (K / 2) * 16;
+    };
+    X coef[2][15], rhs[2], dd[2], ri[2];
+    auto read_tile = [&](int par) {
+        rhs[par] = s.at(kRow16 + par * kRowBytes + lane8);
+        dd[par] = ri[par] = X(1);
+        if constexpr (kDiag) dd[par] = s.at(kRow16 + par * kRowBytes + 512 + lane8);
+        if constexpr (MODE == TriMode::ssor) ri[par] = s.at(kRow16 + par * kRowBytes + 1024 + lane8);
+#pragma unroll
+        for (int st = 0; st < 15; ++st) coef[par][st] = s.at(kTile16 + par * kTileBytes + st * 512 + lane8);
+    };
+#pragma unroll
+    for (int t = 0; t < P; ++t) load_chunk(t);
+    __syncthreads();
+    read_tile(0);
+    __syncthreads();
+    const int step_bytes = FWD ? 16 * s.row_bytes : -16 * s.row_bytes;
+    int off = FWD ? s.first + l * s.row_bytes : s.last - l * s.row_bytes;
+    unsigned int ring = group + l * 8;  // ring entry of chunk q0, this lane
+    int ring_q = 0;
+    unsigned int na[K];  // near addresses of the coming chunk
+#pragma unroll
+    for (int k = 0; k < K; ++k) na[k] = code_of<K>(cc[0], k) + group;
+    // MASKED: some row of the chunks may lie past its chain's end
+    auto chunks = [&](int q0, auto masked) {
+#pragma unroll
+        for (int t = 0; t < P; ++t) {
+            const int par = t & 1;
+            // the ring's newest results first; chunk q + 1's tile (built
+            // during chunk q - 1), chunk q + P's loads and chunk q + 1's near
+            // addresses issue while they are on their way
+            X xn[K], mine[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) xn[k] = s.at(na[k]);
+            X acc = rhs[par];
+            const X d = dd[par], rinv = ri[par];
+            read_tile(1 - par);
+#pragma unroll
+            for (int k = 0; k < K; ++k) mine[k] = cv[t][k];
+#pragma unroll
+            for (int k = 0; k < K; ++k) na[k] = code_of<K>(cc[(t + 1) % P], k) + group;
+            load_chunk(t);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < K; ++k) acc = dev::dfma(-mine[k], xn[k], acc);
+            chain_steps<FinishKind<MODE, FWD>::value>(acc, coef[par], d, rinv);
+            const X fin = chain_finish(acc, d, rinv, FinishKind<MODE, FWD>{});
+            s.at(ring + t * 128) = fin;
+            X* const out = reinterpret_cast<X*>(reinterpret_cast<char*>(s.y) + static_cast<unsigned int>(off));
+            if constexpr (decltype(masked)::value) {
+                if ((q0 + t) * 16 + l < s.stored) *out = fin;
             } else {
-#pragma unroll
-                for (int u = 0; u < 16; ++u) {
-                    const int i = i0 + u * 64 + lane;
-                    if (i < nb) y[i * ys] = v[u];
-                }
+                *out = fin;
             }
+            off += step_bytes;
+            chunk_barrier();
         }
-    }
+        ring_q = ring_q == kRing16 - P ? 0 : ring_q + P;
+        ring = group + l * 8 + static_cast<unsigned int>(ring_q) * 128;
+    };
+    int q0 = 0;
+    for (; q0 + P <= s.full; q0 += P) chunks(q0, std::false_type{});
+    for (; q0 < s.chunks; q0 += P) chunks(q0, std::true_type{});
     __syncthreads();
-    const X* dv = dval + static_cast<std::int64_t>(c) * a.rows + r0;
-    const std::int64_t g0 = l.chunk0[b];
-    // tile entry of step st for this lane (the zero guard at or before st);
-    // kept in registers for both sweeps
-    int taddr[64];
-#pragma unroll
-    for (int st = 0; st < 64; ++st) {
-        taddr[st] = lane > st ? tri_base(st) + lane - st : 0;
-        __asm__ volatile("" : "+v"(taddr[st]));
-    }
-    ell_sweep<MODE, true, X, V, E>(l.fidx, fval + static_cast<std::int64_t>(c) * l.fslots, g0, dv, y, ys, tri, taddr,
-                                   nb, lane);
+}
+
+template<TriMode MODE, class X, class V, int K>
+__global__ __launch_bounds__(128) void k_tri_rows16(Rows16Args a, const V* __restrict__ fval,
+                                                    const V* __restrict__ bval, const X* __restrict__ dval,
+                                                    const X* in, X* out, X scale, const int* stop)
+{
+    constexpr int P = chunks_ahead(K);
+    static_assert(2 * K * 128 <= kGroup16 - kFar16 && kTile16 + 16 * 512 <= 65536 && P % 2 == 0 && kRing16 % P == 0 && 3 * P + 2 <= kPadChunks16);
+    static_assert(kRingZero + 128 <= kFar16);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kLds16];
+    if (stop && *stop) return;
+    const int lane = static_cast<int>(threadIdx.x & 63);
+    const bool solver = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) == 0;
+    for (int t = static_cast<int>(threadIdx.x); t < kLds16 / 8; t += 128) *reinterpret_cast<X*>(lds + 8 * t) = X(0);
     __syncthreads();
-    ell_sweep<MODE, false, X, V, E>(l.bidx, bval + static_cast<std::int64_t>(c) * l.bslots, g0, dv, y, ys, tri,
-                                    taddr, nb, lane);
-    const bool scaled = MODE == TriMode::ssor && scale != X(1);
-    if (GLOBAL_Y && !scaled) return;
-    __syncthreads();
-    for (int i0 = 0; i0 < nb; i0 += 16 * 64) {
-        const bool full = i0 + 16 * 64 <= nb;
-        X v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int i = i0 + u * 64 + lane;
-            v[u] = y[(i < nb ? i : nb - 1) * ys];
-            if (scaled) v[u] = v[u] * scale;
-        }
-        if (full) {
-#pragma unroll
-            for (int u = 0; u < 16; ++u) out[(r0 + i0 + u * 64 + lane) * bs + c] = v[u];
-        } else {
-#pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int i = i0 + u * 64 + lane;
-                if (i < nb) out[(r0 + i) * bs + c] = v[u];
-            }
-        }
+    // the component chains of a block side by side: they read the same codes
+    const int first = static_cast<int>(kern::xcd_block(blockIdx.x, gridDim.x)) * 4;
+    const int mine = first + (lane >> 4);
+    const int chain = mine < a.chains ? mine : a.chains - 1;
+    const int b = chain / a.bs, c = chain - b * a.bs;
+    const int rows = a.nrows[b];
+    const int r0 = a.row0[b], r0_first = a.row0[first / a.bs];
+    int nch = (rows + 15) >> 4;
+    nch = max(max(__builtin_amdgcn_readlane(nch, 0), __builtin_amdgcn_readlane(nch, 16)),
+              max(__builtin_amdgcn_readlane(nch, 32), __builtin_amdgcn_readlane(nch, 48)));
+    const std::int64_t start = static_cast<std::int64_t>(__builtin_amdgcn_readfirstlane(r0_first)) * a.bs;
+    Rows16Sweep<X, V> s;
+    s.row_bytes = a.bs * static_cast<int>(sizeof(X));
+    s.first = (r0 - r0_first) * s.row_bytes + c * static_cast<int>(sizeof(X));
+    s.last = s.first + (rows - 1) * s.row_bytes;
+    s.lds = lds;
+    s.rows = rows;
+    s.stored = mine < a.chains ? rows : 0;
+    s.chunks = (nch + P - 1) / P * P;
+    s.full = s.stored >> 4;
+    s.full = min(min(__builtin_amdgcn_readlane(s.full, 0), __builtin_amdgcn_readlane(s.full, 16)),
+                 min(__builtin_amdgcn_readlane(s.full, 32), __builtin_amdgcn_readlane(s.full, 48)));
+    s.lane = lane;
+    s.dv = dval + static_cast<std::int64_t>(c) * a.rows + r0;
+    s.y = out + start;
+    const std::int64_t g0 = static_cast<std::int64_t>(b) * a.block_chunks * (K * 16);
+    const std::int64_t v0 = static_cast<std::int64_t>(c) * a.slots + g0;
+    s.src = in + start;
+    s.near = a.fnear + g0;
+    s.tile = a.ftile + g0;
+    s.far = a.ffar + g0;
+    s.val = fval + v0;
+    if (solver) rows16_solve<MODE, true, X, V, K>(s);
+    else rows16_prepare<MODE, true, X, V, K>(s);
+    s.src = s.y;
+    s.near = a.bnear + g0;
+    s.tile = a.btile + g0;
+    s.far = a.bfar + g0;
+    s.val = bval + v0;
+    if (solver) rows16_solve<MODE, false, X, V, K>(s);
+    else rows16_prepare<MODE, false, X, V, K>(s);
+    if (MODE == TriMode::ssor && scale != X(1) && solver) {
+        X* o = reinterpret_cast<X*>(reinterpret_cast<char*>(s.y) + s.first);
+        for (int i = lane & 15; i < s.stored; i += 16) o[static_cast<std::int64_t>(i) * a.bs] *= scale;
     }
 }
 
-// ELL values from the chain-order values: dst[c][slot] = src[c][map[slot]] (0 for padding)
+// Sweep values from the chain-order values: dst[c][slot] = src[c][map[slot]] (0 for padding)
 template<class V>
 __global__ __launch_bounds__(256) void k_ell_gather(V* __restrict__ dst, const V* __restrict__ src,
                                                     const std::int64_t* __restrict__ map, std::int64_t slots,
@@ -1219,76 +1236,58 @@ struct TriHost {
 
 std::size_t lds_limit(owtk_precond pc);
 
-// ELL copy of a chain layout (see k_tri_ell): slot k of position p holds the
-// p-th row's k-th chain-order entry, encoded by where its value comes from:
-// its block-local column (entry on a chunk before the previous one),
-// -(t + 2) (in-chunk entry finished at step s, t = tri_base(s) + lane - s its
-// packed tile entry, 1..2016), -(l + 2019) (entry on the previous chunk,
-// finished by lane l) or -1 (padding).  Needs block-local columns below 2^15
-// and at most 16 entries per row.
-void build_ell(TriSchedule& tri, const std::vector<std::int64_t>& fptr, const std::vector<std::int32_t>& fnout,
-               const std::vector<std::int32_t>& fcol, const std::vector<std::int64_t>& bptr,
-               const std::vector<std::int32_t>& bnout, const std::vector<std::int32_t>& bcol)
+// Codes and value maps of the chain sweeps (k_tri_rows16) from the chain
+// layout: entry k of the row at position p (chunk q = p / 16, lane l) goes to
+// value slot ((q * K / 2 + k / 2) * 16 + l) * 2 + k % 2 of its block.
+void build_rows16(TriSchedule& tri, const std::vector<std::int64_t>& fptr, const std::vector<std::int32_t>& fcol,
+                  const std::vector<std::int64_t>& bptr, const std::vector<std::int32_t>& bcol)
 {
-    tri.ell = false;
-    if (!tri.chain || tri.max_block_rows > 32767) return;
-    std::vector<std::int32_t> chunk0(tri.blocks);
-    std::int64_t chunks = 0;
-    for (std::int64_t b = 0; b < tri.blocks; ++b) {
-        chunk0[b] = static_cast<std::int32_t>(chunks);
-        chunks += (tri.h_nrows[b] + 63) / 64;
-    }
+    if (!tri.chain) return;
     const std::int64_t n = tri.rows;
-    auto kmax = [&](const std::vector<std::int64_t>& ptr) {
-        std::int64_t k = 1;
-        for (std::int64_t i = 0; i < n; ++i) k = std::max(k, ptr[i + 1] - ptr[i]);
-        return k;
-    };
-    const std::int64_t kneed = std::max(kmax(fptr), kmax(bptr));
-    if (kneed > 16 || chunks > 0x7fffffff) return;
-    // both sweeps padded to the kernel's slot count (4, 6, 8 or 16)
-    const std::int64_t fk = kneed <= 4 ? 4 : kneed <= 6 ? 6 : kneed <= 8 ? 8 : 16, bk = fk;
+    std::int64_t need = 1;
+    for (std::int64_t i = 0; i < n; ++i) need = std::max({need, fptr[i + 1] - fptr[i], bptr[i + 1] - bptr[i]});
+    const int K = need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : 16;
+    // every block has room for the longest one's chunks: a wave's four chains
+    // run as long as its longest block
+    const std::int64_t per = (tri.max_block_rows + 15) / 16;
+    const std::int64_t chunks = tri.blocks * per + kPadChunks16;
     for (int dir = 0; dir < 2; ++dir) {
         const auto& ptr = dir == 0 ? fptr : bptr;
-        const auto& nout = dir == 0 ? fnout : bnout;
         const auto& col = dir == 0 ? fcol : bcol;
-        const std::int64_t K = dir == 0 ? fk : bk;
-        std::vector<std::int16_t> idx(static_cast<std::size_t>(chunks * K * 64), -1);
-        std::vector<std::int64_t> map(idx.size(), -1);
+        std::vector<std::uint16_t> near(static_cast<std::size_t>(chunks * K * 16), kRingZero), tile(near.size(), kTileSpare);
+        std::vector<std::int16_t> far(near.size(), -1);
+        std::vector<std::int64_t> map(near.size(), -1);
         for (std::int64_t b = 0; b < tri.blocks; ++b) {
-            const std::int64_t r0 = tri.h_row0[b];
-            const std::int64_t nb = tri.h_nrows[b];
+            const std::int64_t r0 = tri.h_row0[b], nb = tri.h_nrows[b];
             for (std::int64_t p = 0; p < nb; ++p) {
-                const std::int64_t q = p / 64, lane = p % 64, cs = q * 64;
-                const std::int64_t g = chunk0[b] + q;
-                const std::int64_t e0 = ptr[r0 + p], e1 = ptr[r0 + p + 1], no = nout[r0 + p];
-                for (std::int64_t e = e0; e < e1; ++e) {
-                    const std::int64_t c = col[e];
-                    const std::int64_t pc = dir == 0 ? c : nb - 1 - c;  // position of the column in the sweep
-                    std::int64_t code = c;
-                    if (e - e0 >= no) {
-                        const std::int64_t step = pc - cs;
-                        if (step < 0 || step >= lane) throw std::logic_error("chain layout: in-chunk entry order");
-                        code = -(tri_base(static_cast<int>(step)) + lane - step + 2);
-                    } else if (pc >= cs) {
-                        throw std::logic_error("chain layout: out-of-chunk entry inside the chunk");
-                    } else if (pc >= cs - 64) {
-                        code = -(pc - (cs - 64) + 2019);
+                const std::int64_t q = p / 16, l = p % 16, g = b * per + q;
+                for (std::int64_t e = ptr[r0 + p]; e < ptr[r0 + p + 1]; ++e) {
+                    const int k = static_cast<int>(e - ptr[r0 + p]);
+                    const std::size_t slot = static_cast<std::size_t>(((g * (K / 2) + k / 2) * 16 + l) * 2 + k % 2);
+                    const std::int64_t pc = dir == 0 ? col[e] : nb - 1 - col[e];  // the column's position in the sweep
+                    const std::int64_t qc = pc / 16;
+                    const std::size_t at = static_cast<std::size_t>((g * 16 + l) * K + k);
+                    if (pc >= p) throw std::logic_error("chain layout: entry on a later row");
+                    if (qc == q) {
+                        tile[at] = static_cast<std::uint16_t>(kTile16 + (pc % 16) * 512);
+                    } else if (q - qc < kRing16) {
+                        near[at] = static_cast<std::uint16_t>((qc % kRing16) * 128 + (pc % 16) * 8);
+                    } else {
+                        near[at] = static_cast<std::uint16_t>(kFar16 + ((q % 2) * K + k) * 128 + l * 8);
+                        far[at] = static_cast<std::int16_t>(col[e]);
                     }
-                    const std::size_t slot = static_cast<std::size_t>((g * K + (e - e0)) * 64 + lane);
-                    idx[slot] = static_cast<std::int16_t>(code);
                     map[slot] = e;
                 }
             }
         }
-        upload(dir == 0 ? tri.fidx_ell : tri.bidx_ell, idx);
-        upload(dir == 0 ? tri.fmap_ell : tri.bmap_ell, map);
-        (dir == 0 ? tri.fslots : tri.bslots) = static_cast<std::int64_t>(idx.size());
+        upload(dir == 0 ? tri.fnear : tri.bnear, near);
+        upload(dir == 0 ? tri.ftile : tri.btile, tile);
+        upload(dir == 0 ? tri.ffar : tri.bfar, far);
+        upload(dir == 0 ? tri.fmap : tri.bmap, map);
     }
-    tri.fk = static_cast<int>(fk);
-    tri.bk = static_cast<int>(bk);
-    upload(tri.chunk0, chunk0);
-    tri.ell = true;
+    tri.k16 = K;
+    tri.block_chunks = static_cast<int>(per);
+    tri.slots16 = chunks * K * 16;
 }
 
 void build_schedule(owtk_precond pc, const TriHost& t)
@@ -1344,8 +1343,7 @@ void build_schedule(owtk_precond pc, const TriHost& t)
         throw unsupported_error("chain sweeps need at most 16 entries per row and a block that fits in LDS");
     tri.chain = pc->schedule == 2 || (pc->schedule == 0 && chain_ok && depth_sum * 16 > n);
     // pass 2: level lists and apply arrays
-    std::vector<std::int32_t> frow(n), brow(n), frow_lvl(n), fnout(n, 0), bnout(n, 0);
-    tri.ei_max = 0;
+    std::vector<std::int32_t> frow(n), brow(n), frow_lvl(n);
     std::vector<std::int64_t> fptr(n + 1, 0), bptr(n + 1, 0);
     std::vector<std::int32_t> fcol, bcol;
     std::vector<std::int64_t> fsrc, bsrc;
@@ -1386,7 +1384,6 @@ void build_schedule(owtk_precond pc, const TriHost& t)
             auto& ptr = dir == 0 ? fptr : bptr;
             auto& ocol = dir == 0 ? fcol : bcol;
             auto& osrc = dir == 0 ? fsrc : bsrc;
-            auto& onout = dir == 0 ? fnout : bnout;
             std::vector<std::pair<int, std::int64_t>> inside;
             for (std::int64_t p = 0; p < nb; ++p) {
                 const std::int64_t i = r0 + rowmap[r0 + p];
@@ -1400,7 +1397,6 @@ void build_schedule(owtk_precond pc, const TriHost& t)
                     // in-chunk entries by the step that finishes their row
                     const std::int64_t cs = (p / 64) * 64;
                     inside.clear();
-                    std::int32_t outside = 0;
                     for (std::int64_t e = off[i]; e < off[i + 1]; ++e) {
                         const std::int64_t c = col[e] - r0;
                         const bool in_chunk = dir == 0 ? c >= cs : c <= nb - 1 - cs;
@@ -1409,7 +1405,6 @@ void build_schedule(owtk_precond pc, const TriHost& t)
                         } else {
                             ocol.push_back(static_cast<std::int32_t>(c));
                             osrc.push_back(src[e]);
-                            ++outside;
                         }
                     }
                     std::sort(inside.begin(), inside.end());
@@ -1417,8 +1412,6 @@ void build_schedule(owtk_precond pc, const TriHost& t)
                         ocol.push_back(static_cast<std::int32_t>(col[e] - r0));
                         osrc.push_back(src[e]);
                     }
-                    onout[r0 + p] = outside;
-                    tri.ei_max = std::max<int>(tri.ei_max, static_cast<int>(inside.size()));
                 }
                 ptr[r0 + p + 1] = static_cast<std::int64_t>(ocol.size());
             }
@@ -1426,7 +1419,7 @@ void build_schedule(owtk_precond pc, const TriHost& t)
     }
     tri.fnnz = static_cast<std::int64_t>(fcol.size());
     tri.bnnz = static_cast<std::int64_t>(bcol.size());
-    build_ell(tri, fptr, fnout, fcol, bptr, bnout, bcol);
+    build_rows16(tri, fptr, fcol, bptr, bcol);
     upload(tri.row0, tri.h_row0);
     upload(tri.nrows, tri.h_nrows);
     upload(tri.flev, tri.h_flev);
@@ -1436,8 +1429,6 @@ void build_schedule(owtk_precond pc, const TriHost& t)
     upload(tri.frow, frow);
     upload(tri.brow, brow);
     upload(tri.frow_lvl, frow_lvl);
-    upload(tri.fnout, fnout);
-    upload(tri.bnout, bnout);
     upload(tri.fptr, fptr);
     upload(tri.bptr, bptr);
     upload(tri.fcol, fcol);
@@ -1450,7 +1441,7 @@ TriArgs tri_args(const TriSchedule& t)
 {
     return TriArgs{t.row0.get(), t.nrows.get(), t.flev.get(), t.blev.get(), t.flev_pos.get(), t.blev_pos.get(),
                    t.frow.get(), t.brow.get(), t.fptr.get(), t.bptr.get(), t.fcol.get(), t.bcol.get(),
-                   t.fnout.get(), t.bnout.get(), t.fnnz, t.bnnz, t.rows, t.bs};
+                   t.fnnz, t.bnnz, t.rows, t.bs};
 }
 
 std::size_t lds_limit(owtk_precond pc)
@@ -1483,25 +1474,26 @@ void refresh_storage(owtk_precond pc)
     auto& t = pc->tri;
     const hipStream_t st = pc->m->ctx->stream;
     const int bs = pc->m->bs;
-    if (t.ell) {
-        // ELL values, FP64 from the chain-order factor, then each storage's copy
-        if (!t.fell64.get()) t.fell64.allocate(std::max<std::int64_t>(t.fslots * bs, 1));
-        if (!t.bell64.get()) t.bell64.allocate(std::max<std::int64_t>(t.bslots * bs, 1));
-        k_ell_gather<double><<<grid_for(t.fslots * bs), kBlock, 0, st>>>(t.fell64.get(), t.fval64.get(),
-                                                                         t.fmap_ell.get(), t.fslots, t.fnnz, bs);
-        k_ell_gather<double><<<grid_for(t.bslots * bs), kBlock, 0, st>>>(t.bell64.get(), t.bval64.get(),
-                                                                         t.bmap_ell.get(), t.bslots, t.bnnz, bs);
+    if (t.chain) {
+        // the sweeps' value slots, FP64 from the chain-order factor, then the storage's copy
+        const std::int64_t nv = t.slots16 * bs;
+        if (!t.f16v64.get()) t.f16v64.allocate(nv);
+        if (!t.b16v64.get()) t.b16v64.allocate(nv);
+        k_ell_gather<double><<<grid_for(nv), kBlock, 0, st>>>(t.f16v64.get(), t.fval64.get(), t.fmap.get(), t.slots16,
+                                                              t.fnnz, bs);
+        k_ell_gather<double><<<grid_for(nv), kBlock, 0, st>>>(t.b16v64.get(), t.bval64.get(), t.bmap.get(), t.slots16,
+                                                              t.bnnz, bs);
         OWTK_LAUNCH_CHECK();
         if (pc->storage == OWTK_F32) {
-            if (!t.fell32.get()) t.fell32.allocate(std::max<std::int64_t>(t.fslots * bs, 1));
-            if (!t.bell32.get()) t.bell32.allocate(std::max<std::int64_t>(t.bslots * bs, 1));
-            kern::convert(st, t.fell32.get(), t.fell64.get(), static_cast<std::size_t>(t.fslots * bs));
-            kern::convert(st, t.bell32.get(), t.bell64.get(), static_cast<std::size_t>(t.bslots * bs));
+            if (!t.f16v32.get()) t.f16v32.allocate(nv);
+            if (!t.b16v32.get()) t.b16v32.allocate(nv);
+            kern::convert(st, t.f16v32.get(), t.f16v64.get(), static_cast<std::size_t>(nv));
+            kern::convert(st, t.b16v32.get(), t.b16v64.get(), static_cast<std::size_t>(nv));
         } else if (pc->storage == OWTK_BF16) {
-            if (!t.fell16.get()) t.fell16.allocate(std::max<std::int64_t>(t.fslots * bs, 1));
-            if (!t.bell16.get()) t.bell16.allocate(std::max<std::int64_t>(t.bslots * bs, 1));
-            kern::k_to_bf16<<<grid_for(t.fslots * bs), kBlock, 0, st>>>(t.fell16.get(), t.fell64.get(), t.fslots * bs);
-            kern::k_to_bf16<<<grid_for(t.bslots * bs), kBlock, 0, st>>>(t.bell16.get(), t.bell64.get(), t.bslots * bs);
+            if (!t.f16v16.get()) t.f16v16.allocate(nv);
+            if (!t.b16v16.get()) t.b16v16.allocate(nv);
+            kern::k_to_bf16<<<grid_for(nv), kBlock, 0, st>>>(t.f16v16.get(), t.f16v64.get(), nv);
+            kern::k_to_bf16<<<grid_for(nv), kBlock, 0, st>>>(t.b16v16.get(), t.b16v64.get(), nv);
             OWTK_LAUNCH_CHECK();
         }
     }
@@ -2126,56 +2118,30 @@ void tri_launch(owtk_precond pc, const V* fv, const V* bv, const X* dv, const X*
     const X scale = static_cast<X>(pc->omega * (2.0 - pc->omega));
     const hipStream_t st = pc->m->ctx->stream;
     ProfileScope prof(pc->m->ctx, sizeof(X) == 8 ? prof_precond_f64 : prof_precond_low, precond_apply_bytes(pc));
-    if (t.chain && t.ell) {
-        const TriArgs args = tri_args(t);
-        const EllArgs ea{t.chunk0.get(), t.fidx_ell.get(), t.bidx_ell.get(), t.fslots, t.bslots, t.fk, t.bk};
-        const V* efv;
-        const V* ebv;
+    if (t.chain) {
+        const int chains = static_cast<int>(groups);
+        const Rows16Args ra{t.row0.get(), t.nrows.get(), t.fnear.get(), t.bnear.get(), t.ftile.get(), t.btile.get(),
+                            t.ffar.get(), t.bfar.get(), t.slots16, t.rows, chains, t.block_chunks, t.bs};
+        const V* fvals;
+        const V* bvals;
         if constexpr (std::is_same_v<V, double>) {
-            efv = t.fell64.get();
-            ebv = t.bell64.get();
+            fvals = t.f16v64.get();
+            bvals = t.b16v64.get();
         } else if constexpr (std::is_same_v<V, float>) {
-            efv = t.fell32.get();
-            ebv = t.bell32.get();
+            fvals = t.f16v32.get();
+            bvals = t.b16v32.get();
         } else {
-            efv = t.fell16.get();
-            ebv = t.bell16.get();
+            fvals = t.f16v16.get();
+            bvals = t.b16v16.get();
         }
-        const std::size_t tri_lds = static_cast<std::size_t>(2 + 64 * 63 / 2) * sizeof(X);
-        const bool global_y = need + tri_lds > kChainLdsBudget;
-        const std::size_t lds = global_y ? tri_lds : need + tri_lds;
-        const int k = std::max(t.fk, t.bk);
-        auto launch = [&](auto e, auto gy) {
-            k_tri_ell<MODE, X, V, decltype(e)::value, decltype(gy)::value>
-                <<<groups, 64, lds, st>>>(args, ea, efv, ebv, dv, in, out, scale, stop);
+        const unsigned int waves = static_cast<unsigned int>((chains + 3) / 4);
+        auto launch = [&](auto k) {
+            k_tri_rows16<MODE, X, V, decltype(k)::value><<<waves, 128, 0, st>>>(ra, fvals, bvals, dv, in, out, scale, stop);
         };
-        auto pick = [&](auto e) {
-            if (global_y) launch(e, std::true_type{});
-            else launch(e, std::false_type{});
-        };
-        if (k == 4) pick(std::integral_constant<int, 4>{});
-        else if (k == 6) pick(std::integral_constant<int, 6>{});
-        else if (k == 8) pick(std::integral_constant<int, 8>{});
-        else pick(std::integral_constant<int, 16>{});
-    } else if (t.chain) {
-        const TriArgs args = tri_args(t);
-        // Large blocks keep their solution in global memory (L2): the LDS
-        // then holds only the tile, and more one-wave workgroups fit per CU.
-        const std::size_t tile_lds = 64 * 64 * sizeof(X);
-        const bool global_y = need + tile_lds > kChainLdsBudget;
-        const std::size_t chain_lds = global_y ? tile_lds : need + tile_lds;
-        auto launch = [&](auto ei, auto gy) {
-            k_tri_chain<MODE, X, V, decltype(ei)::value, decltype(gy)::value>
-                <<<groups, 64, chain_lds, st>>>(args, fv, bv, dv, in, out, scale, stop);
-        };
-        auto pick = [&](auto ei) {
-            if (global_y) launch(ei, std::true_type{});
-            else launch(ei, std::false_type{});
-        };
-        if (t.ei_max <= 2) pick(std::integral_constant<int, 2>{});
-        else if (t.ei_max <= 4) pick(std::integral_constant<int, 4>{});
-        else if (t.ei_max <= 8) pick(std::integral_constant<int, 8>{});
-        else pick(std::integral_constant<int, 16>{});
+        if (t.k16 == 4) launch(std::integral_constant<int, 4>{});
+        else if (t.k16 == 6) launch(std::integral_constant<int, 6>{});
+        else if (t.k16 == 8) launch(std::integral_constant<int, 8>{});
+        else launch(std::integral_constant<int, 16>{});
     } else if (need <= lds_limit(pc)) {
         k_tri_apply<MODE, X, V, true><<<groups, threads, need, st>>>(tri_args(t), fv, bv, dv, in, out, scale, stop);
     } else {

@@ -33,8 +33,6 @@ struct TriSchedule {
     DeviceArray<std::int32_t> frow_lvl;  // forward level order (numeric factorization)
     bool chain = false;  // one-wave chain sweeps instead of level barriers
     int emax = 0;        // most entries of one row in one direction
-    int ei_max = 0;      // chain layout: most in-chunk entries of one row
-    DeviceArray<std::int32_t> fnout, bnout;  // chain layout: entries before the chunk
     // entry pointers per position (global), block-local columns
     DeviceArray<std::int64_t> fptr, bptr;
     DeviceArray<std::int32_t> fcol, bcol;
@@ -48,17 +46,17 @@ struct TriSchedule {
     DeviceArray<std::uint16_t> fval16, bval16;
     // gather sources of the apply values (numeric update)
     DeviceArray<std::int64_t> fsrc, bsrc, dsrc;
-    // ELL copy of the chain layout: per 64-row chunk and slot, the rows'
-    // entries contiguous (k_tri_ell); values [c][slot] in each storage
-    bool ell = false;
-    int fk = 0, bk = 0;                       // slots per row, forward / backward sweep
-    std::int64_t fslots = 0, bslots = 0;      // chunks * slots * 64
-    DeviceArray<std::int32_t> chunk0;         // first chunk of each block
-    DeviceArray<std::int16_t> fidx_ell, bidx_ell;
-    DeviceArray<std::int64_t> fmap_ell, bmap_ell;  // chain-order entry of each slot, -1 padding
-    DeviceArray<double> fell64, bell64;
-    DeviceArray<float> fell32, bell32;
-    DeviceArray<std::uint16_t> fell16, bell16;
+    // chain sweeps (k_tri_rows16): slots per row, chunks of 16 rows each block
+    // has room for, values per component and sweep, entry codes (LDS addresses), far rows and
+    // chain-order entry of each value slot (-1 padding), values per storage
+    int k16 = 0, block_chunks = 0;
+    std::int64_t slots16 = 0;
+    DeviceArray<std::uint16_t> fnear, bnear, ftile, btile;
+    DeviceArray<std::int16_t> ffar, bfar;
+    DeviceArray<std::int64_t> fmap, bmap;
+    DeviceArray<double> f16v64, b16v64;
+    DeviceArray<float> f16v32, b16v32;
+    DeviceArray<std::uint16_t> f16v16, b16v16;
 };
 
 // Program of the chunked numeric factorization (k_ilu_factor_chunks): rows

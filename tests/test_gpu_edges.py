@@ -122,3 +122,57 @@ def test_red_black_coarse_sweeps(ctx, case):
     x = ctx.empty(n * block)
     owtk.Multigrid(m, smoother=owtk.MG_RED_BLACK).solve(ctx.upload(b), x, owtk.SolverOptions(**kw))
     assert np.max(np.abs(x.download() - xo)) <= 1e-13 * np.max(np.abs(xo))
+
+
+def banded(rng, n, block, reach, count):
+    """Diagonally dominant split-form rows with up to `count` neighbours on each side, up to `reach` rows away (the
+    farthest always among them), symmetric pattern."""
+    pairs = set()
+    for i in range(n):
+        own = rng.choice(np.arange(1, reach + 1), min(count, reach), replace=False)
+        for d in set(own[: rng.integers(0, count + 1)]) | {reach}:
+            if i + d < n:
+                pairs.add((i, i + int(d)))
+    rows = [[] for _ in range(n)]
+    for i, j in pairs:
+        rows[i].append(j)
+        rows[j].append(i)
+    columns = np.concatenate([np.sort(r) for r in rows if r] or [np.zeros(0)]).astype(np.int32)
+    offsets = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    off = -rng.uniform(0.1, 1.0, (columns.size, block))
+    diag = np.add.reduceat(np.abs(np.vstack([off, np.zeros((1, block))])), offsets[:-1], axis=0) + 0.5
+    diag[np.diff(offsets) == 0] = 1.0
+    return offsets, columns, diag.ravel(), off.ravel()
+
+
+@pytest.mark.parametrize("n,block,block_nodes,reach,count", [
+    (1, 1, 0, 1, 1), (15, 2, 0, 3, 2), (16, 1, 0, 5, 2), (17, 3, 0, 5, 2), (65, 5, 16, 4, 2), (130, 3, 33, 9, 3),
+    (700, 1, 0, 431, 2), (700, 2, 0, 449, 3), (900, 3, 0, 448, 3), (1300, 3, 640, 500, 4), (2100, 7, 0, 900, 5),
+    (1100, 4, 550, 500, 8), (900, 1, 0, 433, 14), (3000, 1, 700, 650, 2)])
+def test_chain_sweeps(ctx, n, block, block_nodes, reach, count):
+    """Chain sweeps (one 16-row chunk after the other): partial chunks and blocks, 1 to 7 components (groups past the
+    last chain), 2 to 15 entries per row (each slot count), entries at the ends of the near range (27 chunks) and
+    beyond it, in place and not, FP64 and FP32 storage.  Backward in-chunk entries fold in the order they become
+    available: 1e-14 of the largest value, as for the other chain sweeps; FP32 at 2^29 times that."""
+    rng = np.random.default_rng(n + reach)
+    off, col, diag, val = banded(rng, n, block, reach, count)
+    om = orc.OMatrix.split(n, 0, block, off, col, diag, val)
+    m = owtk.Matrix.split(ctx, n, 0, block, off, col, diag, val)
+    m.add_storage(owtk.F32)
+    x = rng.uniform(-1, 1, n * block)
+    xd, yd = ctx.upload(x), ctx.empty(n * block)
+    for kind, okind, omega in ((owtk.PC_ILU, 3, 1.0), (owtk.PC_SSOR, orc.OPreconditioner.SSOR, 1.0),
+                               (owtk.PC_SSOR, orc.OPreconditioner.SSOR, 1.3)):
+        opc = orc.OPreconditioner(om, okind, block_nodes=block_nodes, omega=omega)
+        pc = owtk.Preconditioner(m, kind, block_nodes=block_nodes, omega=omega, schedule=2)
+        ref = opc.apply(x)
+        pc.apply(xd, yd)
+        y = yd.download()
+        assert np.max(np.abs(y - ref)) <= 1e-14 * np.max(np.abs(ref))
+        zd = ctx.upload(x)
+        pc.apply(zd, zd)
+        assert np.array_equal(zd.download(), y)
+        low = owtk.Preconditioner(m, kind, block_nodes=block_nodes, omega=omega, schedule=2, storage=owtk.F32)
+        wd = ctx.empty(n * block, np.float32)
+        low.apply(ctx.upload(x.astype(np.float32)), wd)
+        assert np.max(np.abs(wd.download() - ref)) <= 2.0 ** 29 * 1e-14 * np.max(np.abs(ref))
