@@ -81,9 +81,9 @@ __device__ void fin_rho(BicgState* st, double rho, long long it)
 }
 
 // <shadow, r> at (re)start.  CMP: compensated (double-double) accumulation.
-template<bool CMP>
+template<bool CMP, class Fin>
 __global__ __launch_bounds__(256) void k_rho(const double* __restrict__ shadow, const double* __restrict__ r,
-                                             std::int64_t n, BicgState* st, ReduceScratch scratch)
+                                             std::int64_t n, Fin fin, ReduceScratch scratch)
 {
     double red[1] = {0.0}, lo[1] = {0.0};
     const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void k_rho(const double* __restrict__ shadow, 
         else red[0] = __builtin_fma(shadow[i], r[i], red[0]);
     }
     if constexpr (CMP) dev::store_partials_dd<1>(red, lo, 0, scratch);
-    else dev::store_partials<1>(red, 0, scratch);
+    else dev::reduce_end<1>(red, 0, scratch, fin);
 }
 
 struct FinRho {
@@ -116,10 +116,10 @@ __global__ __launch_bounds__(256) void k_p_update(double* __restrict__ p, const 
 }
 
 // s = r - alpha v, ||s||
-template<bool CMP>
+template<bool CMP, class Fin>
 __global__ __launch_bounds__(256) void k_s_update(double* __restrict__ s, const double* __restrict__ r,
                                                   const double* __restrict__ v, std::int64_t n, BicgState* st,
-                                                  ReduceScratch scratch)
+                                                  Fin fin, ReduceScratch scratch)
 {
     if (st->stop) return;
     const double alpha = st->alpha;
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_s_update(double* __restrict__ s, const 
         red[1] = dev::combine<dev::Combine::max>(red[1], __builtin_fabs(si));
     }
     if constexpr (CMP) dev::store_partials_dd<2>(red, lo, 2, scratch);
-    else dev::store_partials<2>(red, 2, scratch);
+    else dev::reduce_end<2>(red, 2, scratch, fin);
 }
 
 struct FinSnorm {
@@ -154,12 +154,12 @@ struct FinSnorm {
 };
 
 // x += alpha z; x += omega y; r = s - omega t; <shadow, r>, ||r||
-template<bool CMP>
+template<bool CMP, class Fin>
 __global__ __launch_bounds__(256) void k_xr_update(double* __restrict__ x, double* __restrict__ r,
                                                    const double* __restrict__ z, const double* __restrict__ y,
                                                    const double* __restrict__ s, const double* __restrict__ t,
                                                    const double* __restrict__ shadow, std::int64_t n, BicgState* st,
-                                                   ReduceScratch scratch)
+                                                   Fin fin, ReduceScratch scratch)
 {
     if (st->stop) return;
     const double alpha = st->alpha, omega = st->omega;
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_xr_update(double* __restrict__ x, doubl
         red[2] = dev::combine<dev::Combine::max>(red[2], __builtin_fabs(ri));
     }
     if constexpr (CMP) dev::store_partials_dd<3>(red, lo, 4, scratch);
-    else dev::store_partials<3>(red, 4, scratch);
+    else dev::reduce_end<3>(red, 4, scratch, fin);
 }
 
 // Compensated-mode reductions that the FP64 path fuses into SpMV epilogues:
@@ -495,8 +495,9 @@ struct ChVecs {
 };
 
 // restart: rp = r and <r, rp>
+template<class Fin>
 __global__ __launch_bounds__(256) void k_ch_rho(const double* __restrict__ r, double* __restrict__ rp, std::int64_t n,
-                                                ReduceScratch scratch)
+                                                Fin fin, ReduceScratch scratch)
 {
     double red[1] = {0.0};
     const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
@@ -505,7 +506,7 @@ __global__ __launch_bounds__(256) void k_ch_rho(const double* __restrict__ r, do
         rp[i] = ri;
         red[0] = __builtin_fma(ri, ri, red[0]);
     }
-    dev::store_partials<1>(red, 0, scratch);
+    dev::reduce_end<1>(red, 0, scratch, fin);
 }
 
 struct FinChRho {
@@ -542,7 +543,9 @@ struct FinChD2 {
 };
 
 // direction updates (or the restart copies), q, q2, y; <q,y>, <y,y>, <q,q>, max|q|
-__global__ __launch_bounds__(256) void k_ch_first(ChVecs V, std::int64_t n, const ChState* st, ReduceScratch scratch)
+template<class Fin>
+__global__ __launch_bounds__(256) void k_ch_first(ChVecs V, std::int64_t n, const ChState* st, Fin fin,
+                                                  ReduceScratch scratch)
 {
     if (st->stop) return;
     const bool first = st->first != 0;
@@ -577,7 +580,7 @@ __global__ __launch_bounds__(256) void k_ch_first(ChVecs V, std::int64_t n, cons
         red[2] = __builtin_fma(q, q, red[2]);
         red[3] = dev::combine<dev::Combine::max>(red[3], __builtin_fabs(q));
     }
-    dev::store_partials<4>(red, 8, scratch);
+    dev::reduce_end<4>(red, 8, scratch, fin);
 }
 
 struct FinChFirst {
@@ -627,8 +630,9 @@ struct FinChFirst {
 };
 
 // x += alpha p2; x += omega q2; r, r2, w; <r,r>, max|r|, <r,rp>, <s,rp>, <w,rp>, <z,rp>
+template<class Fin>
 __global__ __launch_bounds__(256) void k_ch_second(ChVecs V, double* __restrict__ x, std::int64_t n,
-                                                   const ChState* st, ReduceScratch scratch)
+                                                   const ChState* st, Fin fin, ReduceScratch scratch)
 {
     if (st->stop) return;
     const double alpha = st->alpha, omega = st->omega;
@@ -651,7 +655,7 @@ __global__ __launch_bounds__(256) void k_ch_second(ChVecs V, double* __restrict_
         red[4] = __builtin_fma(w, rp, red[4]);
         red[5] = __builtin_fma(V.z[i], rp, red[5]);
     }
-    dev::store_partials<6>(red, 2, scratch);
+    dev::reduce_end<6>(red, 2, scratch, fin);
 }
 
 struct FinChSecond {
@@ -736,7 +740,7 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
         throw std::invalid_argument("FP64 solve needs an FP64 preconditioner");
     owtk_context ctx = m->ctx;
     const hipStream_t st = ctx->stream;
-    const auto scratch = ctx->scratch();
+    const auto scratch = ctx->scratch();  // compensated reductions: partials and a finisher
     const std::int64_t n = m->owned * m->bs;
     const std::int64_t L = m->local() * m->bs;
     Workspace w;
@@ -759,6 +763,7 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
     std::uint64_t ops = 0, pcs = 0, reds = 0;
 
     const unsigned int g = dev::stream_grid(n, 4);
+    const auto fused = dev::scratch_for(ctx->fused_scratch(), g);
     // ||v|| into *out (compensated mode; the FP64 path fuses its norms)
     auto norm_dd = [&](double* v_in, const double* b_in, double* out) {
         k_residual_dd<<<g, kBlock, 0, st>>>(v_in, b_in, n, scratch);
@@ -794,7 +799,7 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
         if (cmp) {
             norm_dd(const_cast<double*>(b), nullptr, slot);  // read only: no b_in
         } else {
-            kern::norm_to(st, scratch, b, n, slot);
+            kern::norm_to(st, ctx->fused_scratch(), b, n, slot);
         }
         ++reds;
     };
@@ -866,11 +871,11 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
         kern::fill_zero_bytes(st, p, n * sizeof(double));
         kern::fill_zero_bytes(st, v, n * sizeof(double));
         if (cmp) {
-            k_rho<true><<<g, kBlock, 0, st>>>(shadow, r, n, dst, scratch);
+            k_rho<true><<<g, kBlock, 0, st>>>(shadow, r, n, FinRho{dst}, scratch);
             dev::launch_finish_dd<1>(st, FinRho{dst}, g, 0, scratch, nullptr);
         } else {
-            k_rho<false><<<g, kBlock, 0, st>>>(shadow, r, n, dst, scratch);
-            dev::launch_finish<1>(st, FinRho{dst}, g, 0, scratch, nullptr);
+            k_rho<false><<<g, kBlock, 0, st>>>(shadow, r, n, FinRho{dst}, fused);
+            dev::launch_finish<1>(st, FinRho{dst}, g, 0, fused, nullptr);
         }
         OWTK_LAUNCH_CHECK();
     };
@@ -897,7 +902,7 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
             spmv_f64(m, z, e);
             k_dot_dd<1><<<g, kBlock, 0, st>>>(v, shadow, n, stop, scratch);
             dev::launch_finish_dd<1>(st, FinDot1<FinAlpha>{FinAlpha{dst}}, g, 0, scratch, stop);
-            k_s_update<true><<<g, kBlock, 0, st>>>(s, r, v, n, dst, scratch);
+            k_s_update<true><<<g, kBlock, 0, st>>>(s, r, v, n, dst, FinSnorm{dst, s, n}, scratch);
             dev::launch_finish_dd<2>(st, FinSnorm{dst, s, n}, g, 2, scratch, stop);
         } else {
             dev::EpiDot1<FinAlpha> e;
@@ -906,8 +911,8 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
             e.stop = stop;
             e.fin = FinAlpha{dst};
             spmv_f64(m, z, e);
-            k_s_update<false><<<g, kBlock, 0, st>>>(s, r, v, n, dst, scratch);
-            dev::launch_finish<2>(st, FinSnorm{dst, s, n}, g, 2, scratch, stop);
+            k_s_update<false><<<g, kBlock, 0, st>>>(s, r, v, n, dst, FinSnorm{dst, s, n}, fused);
+            dev::launch_finish<2>(st, FinSnorm{dst, s, n}, g, 2, fused, stop);
         }
         OWTK_LAUNCH_CHECK();
         apply_pc_f64(pc, s, yv, n, st, stop);
@@ -918,7 +923,7 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
             spmv_f64(m, yv, e);
             k_dot_dd<2><<<g, kBlock, 0, st>>>(t, s, n, stop, scratch);
             dev::launch_finish_dd<2>(st, FinDot2<FinOmega>{FinOmega{dst}}, g, 0, scratch, stop);
-            k_xr_update<true><<<g, kBlock, 0, st>>>(x, r, z, yv, s, t, shadow, n, dst, scratch);
+            k_xr_update<true><<<g, kBlock, 0, st>>>(x, r, z, yv, s, t, shadow, n, dst, FinXr{dst, r, n}, scratch);
             dev::launch_finish_dd<3>(st, FinXr{dst, r, n}, g, 4, scratch, stop);
         } else {
             dev::EpiDot2<FinOmega> e;
@@ -927,8 +932,8 @@ int bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, con
             e.stop = stop;
             e.fin = FinOmega{dst};
             spmv_f64(m, yv, e);
-            k_xr_update<false><<<g, kBlock, 0, st>>>(x, r, z, yv, s, t, shadow, n, dst, scratch);
-            dev::launch_finish<3>(st, FinXr{dst, r, n}, g, 4, scratch, stop);
+            k_xr_update<false><<<g, kBlock, 0, st>>>(x, r, z, yv, s, t, shadow, n, dst, FinXr{dst, r, n}, fused);
+            dev::launch_finish<3>(st, FinXr{dst, r, n}, g, 4, fused, stop);
         }
         OWTK_LAUNCH_CHECK();
     };
@@ -1051,7 +1056,7 @@ int pipelined_bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, doub
         throw std::invalid_argument("FP64 solve needs an FP64 preconditioner");
     owtk_context ctx = m->ctx;
     const hipStream_t st = ctx->stream;
-    const auto scratch = ctx->scratch();
+    const auto scratch = ctx->scratch();  // compensated reductions: partials and a finisher
     const std::int64_t n = m->owned * m->bs;
     const std::int64_t L = m->local() * m->bs;
     Workspace w;
@@ -1106,7 +1111,7 @@ int pipelined_bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, doub
     std::memset(hst, 0, sizeof(BicgState));
     write_state();
     true_residual(&d_norms[1]);
-    kern::norm_to(st, scratch, b, n, &d_norms[0]);
+    kern::norm_to(st, ctx->fused_scratch(), b, n, &d_norms[0]);
     ++reds;  // |b|^2 and |r|^2 are one fused reduction in the reference
     OWTK_HIP(hipMemcpyAsync(norms, d_norms, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
     ctx->sync();
@@ -1124,6 +1129,7 @@ int pipelined_bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, doub
     if (initial <= thr) return finish(status_converged);
 
     const unsigned int g = dev::stream_grid(n, 4);
+    const auto fused = dev::scratch_for(ctx->fused_scratch(), g);
     // shadow = r, p = r (first), rho = <shadow, r>
     auto restart = [&](long long it) {
         hst->alpha = 1;
@@ -1133,8 +1139,8 @@ int pipelined_bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, doub
         hst->iteration = it;
         write_state();
         OWTK_HIP(hipMemcpyAsync(shadow, r, n * sizeof(double), hipMemcpyDeviceToDevice, st));
-        k_rho<false><<<g, kBlock, 0, st>>>(shadow, r, n, dst, scratch);
-        dev::launch_finish<1>(st, FinRhoP{dst}, g, 0, scratch, nullptr);
+        k_rho<false><<<g, kBlock, 0, st>>>(shadow, r, n, FinRhoP{dst}, fused);
+        dev::launch_finish<1>(st, FinRhoP{dst}, g, 0, fused, nullptr);
         OWTK_LAUNCH_CHECK();
         ++reds;
     };
@@ -1173,8 +1179,8 @@ int pipelined_bicgstab_run(owtk_matrix m, owtk_precond pc, const double* b, doub
             e.stop = stop;
             spmv_f64(m, yv, e);
         }
-        k_xr_update<false><<<g, kBlock, 0, st>>>(x, r, z, yv, s, t, shadow, n, dst, scratch);
-        dev::launch_finish<3>(st, FinNextP{dst, r, n}, g, 4, scratch, stop);
+        k_xr_update<false><<<g, kBlock, 0, st>>>(x, r, z, yv, s, t, shadow, n, dst, FinNextP{dst, r, n}, fused);
+        dev::launch_finish<3>(st, FinNextP{dst, r, n}, g, 4, fused, stop);
         OWTK_LAUNCH_CHECK();
     };
     const long long maxit = static_cast<long long>(o->maximum_iterations);
@@ -1277,7 +1283,7 @@ int communication_hiding_bicgstab_run(owtk_matrix m, owtk_precond pc, const doub
         throw std::invalid_argument("FP64 solve needs an FP64 preconditioner");
     owtk_context ctx = m->ctx;
     const hipStream_t st = ctx->stream;
-    const auto scratch = ctx->scratch();
+    const auto scratch = ctx->scratch();  // compensated reductions: partials and a finisher
     const std::int64_t n = m->owned * m->bs;
     const std::int64_t L = m->local() * m->bs;
     DeviceArray<double> vecs;
@@ -1326,7 +1332,7 @@ int communication_hiding_bicgstab_run(owtk_matrix m, owtk_precond pc, const doub
     std::memset(hst, 0, sizeof(ChState));
     write_state();
     true_residual(&d_norms[1]);
-    kern::norm_to(st, scratch, b, n, &d_norms[0]);
+    kern::norm_to(st, ctx->fused_scratch(), b, n, &d_norms[0]);
     ++reds;  // |b|^2 and |r|^2 are one fused reduction in the reference
     OWTK_HIP(hipMemcpyAsync(norms, d_norms, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
     ctx->sync();
@@ -1350,6 +1356,7 @@ int communication_hiding_bicgstab_run(owtk_matrix m, owtk_precond pc, const doub
     hst->max_iterations = static_cast<long long>(o->maximum_iterations);
     hst->replace_interval = static_cast<long long>(o->residual_replacement_interval);
     const unsigned int g = dev::stream_grid(n, 4);
+    const auto fused = dev::scratch_for(ctx->fused_scratch(), g);
     const int* stop = &dst->stop;
     auto plain_op = [&](const double* in, double* out) {
         dev::EpiStore<double> e;
@@ -1364,8 +1371,8 @@ int communication_hiding_bicgstab_run(owtk_matrix m, owtk_precond pc, const doub
         hst->stop = stop_none;
         hst->iteration = it;
         write_state();
-        k_ch_rho<<<g, kBlock, 0, st>>>(V.r, V.rp, n, scratch);
-        dev::launch_finish<1>(st, FinChRho{dst}, g, 0, scratch, nullptr);
+        k_ch_rho<<<g, kBlock, 0, st>>>(V.r, V.rp, n, FinChRho{dst}, fused);
+        dev::launch_finish<1>(st, FinChRho{dst}, g, 0, fused, nullptr);
         OWTK_LAUNCH_CHECK();
         apply_pc_f64(pc, V.r, V.r2, n, st, stop);
         {
@@ -1398,13 +1405,13 @@ int communication_hiding_bicgstab_run(owtk_matrix m, owtk_precond pc, const doub
     }
 
     auto enqueue_iteration = [&] {
-        k_ch_first<<<g, kBlock, 0, st>>>(V, n, dst, scratch);
-        dev::launch_finish<4>(st, FinChFirst{dst, V.q, n}, g, 8, scratch, stop);
+        k_ch_first<<<g, kBlock, 0, st>>>(V, n, dst, FinChFirst{dst, V.q, n}, fused);
+        dev::launch_finish<4>(st, FinChFirst{dst, V.q, n}, g, 8, fused, stop);
         OWTK_LAUNCH_CHECK();
         apply_pc_f64(pc, V.z, V.z2, n, st, stop);
         plain_op(V.z2, V.v);
-        k_ch_second<<<g, kBlock, 0, st>>>(V, x, n, dst, scratch);
-        dev::launch_finish<6>(st, FinChSecond{dst, V.r, n}, g, 2, scratch, stop);
+        k_ch_second<<<g, kBlock, 0, st>>>(V, x, n, dst, FinChSecond{dst, V.r, n}, fused);
+        dev::launch_finish<6>(st, FinChSecond{dst, V.r, n}, g, 2, fused, stop);
         OWTK_LAUNCH_CHECK();
         apply_pc_f64(pc, V.w, V.w2, n, st, stop);
         plain_op(V.w2, V.t);

@@ -57,6 +57,17 @@ void owtk_context_s::activate() const { OWTK_HIP(hipSetDevice(device)); }
 
 void owtk_context_s::sync() const { OWTK_HIP(hipStreamSynchronize(stream)); }
 
+void owtk_context_s::await_mail() const
+{
+    // about a millisecond of polling, then the blocking wait (which also
+    // reports what kept the result from arriving)
+    for (int i = 0; i < 20000; ++i) {
+        if (__atomic_load_n(mail_flag(), __ATOMIC_ACQUIRE) == mail_number) return;
+        __builtin_ia32_pause();
+    }
+    sync();
+}
+
 void owtk_context_s::reserve_partials(std::int64_t blocks)
 {
     if (blocks <= partial_stride) return;
@@ -132,8 +143,12 @@ int owtk_context_create(int device, owtk_context* out)
         OWTK_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
         ctx->reserve_partials(dev::kMaxReduceBlocks);
         ctx->scalars.allocate(1024);
+        ctx->ticket.allocate(1);
+        kern::fill_zero_bytes(ctx->stream, ctx->ticket.get(), ctx->ticket.bytes());
         kern::fill_zero_bytes(ctx->stream, ctx->scalars.get(), ctx->scalars.bytes());
         ctx->pinned.ensure(1 << 16);
+        ctx->mail.ensure((dev::kMaxReduceValues + 1) * sizeof(double));
+        *ctx->mail_flag() = 0;
         ctx->sync();
         *out = ctx.release();
     });
@@ -334,14 +349,14 @@ int owtk_dot(owtk_context ctx, owtk_dtype dtype, size_t n, const void* a, const 
             return;
         }
         if (!a || !b) throw std::invalid_argument("null vector");
-        double* d_out = ctx->scalars.get();
+        double* d_out = ctx->mail_values();
+        const auto mail = ctx->next_mail();
         if (dtype == OWTK_F64)
-            kern::dot_to(ctx->stream, ctx->scratch(), as<double>(a), as<double>(b), static_cast<std::int64_t>(n), d_out);
+            kern::dot_to(ctx->stream, ctx->fused_scratch(), as<double>(a), as<double>(b), static_cast<std::int64_t>(n), d_out, false, mail);
         else
-            kern::dot_to(ctx->stream, ctx->scratch(), as<float>(a), as<float>(b), static_cast<std::int64_t>(n), d_out);
-        OWTK_HIP(hipMemcpyAsync(ctx->pinned.ptr, d_out, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-        *out = *static_cast<double*>(ctx->pinned.ptr);
+            kern::dot_to(ctx->stream, ctx->fused_scratch(), as<float>(a), as<float>(b), static_cast<std::int64_t>(n), d_out, false, mail);
+        ctx->await_mail();
+        *out = *d_out;
     });
 }
 
@@ -356,14 +371,14 @@ int owtk_norm(owtk_context ctx, owtk_dtype dtype, size_t n, const void* a, doubl
             return;
         }
         if (!a) throw std::invalid_argument("null vector");
-        double* d_out = ctx->scalars.get();
+        double* d_out = ctx->mail_values();
+        const auto mail = ctx->next_mail();
         if (dtype == OWTK_F64)
-            kern::norm_to(ctx->stream, ctx->scratch(), as<double>(a), static_cast<std::int64_t>(n), d_out);
+            kern::norm_to(ctx->stream, ctx->fused_scratch(), as<double>(a), static_cast<std::int64_t>(n), d_out, false, mail);
         else
-            kern::norm_to(ctx->stream, ctx->scratch(), as<float>(a), static_cast<std::int64_t>(n), d_out);
-        OWTK_HIP(hipMemcpyAsync(ctx->pinned.ptr, d_out, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-        *out = *static_cast<double*>(ctx->pinned.ptr);
+            kern::norm_to(ctx->stream, ctx->fused_scratch(), as<float>(a), static_cast<std::int64_t>(n), d_out, false, mail);
+        ctx->await_mail();
+        *out = *d_out;
     });
 }
 
@@ -384,16 +399,16 @@ int owtk_reduction_dot(owtk_context ctx, int32_t reduction, owtk_dtype dtype, si
             return;
         }
         if (!a || !b) throw std::invalid_argument("null vector");
-        double* d_out = ctx->scalars.get();
+        double* d_out = ctx->mail_values();
+        const auto mail = ctx->next_mail();
         if (dtype == OWTK_F64)
-            kern::dot_to(ctx->stream, ctx->scratch(), as<double>(a), as<double>(b), static_cast<std::int64_t>(n), d_out,
-                         reduction != OWTK_REDUCTION_SERIAL);
+            kern::dot_to(ctx->stream, ctx->fused_scratch(), as<double>(a), as<double>(b), static_cast<std::int64_t>(n), d_out,
+                         reduction != OWTK_REDUCTION_SERIAL, mail);
         else
-            kern::dot_to(ctx->stream, ctx->scratch(), as<float>(a), as<float>(b), static_cast<std::int64_t>(n), d_out,
-                         reduction == OWTK_REDUCTION_COMPENSATED);
-        OWTK_HIP(hipMemcpyAsync(ctx->pinned.ptr, d_out, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-        *out = *static_cast<double*>(ctx->pinned.ptr);
+            kern::dot_to(ctx->stream, ctx->fused_scratch(), as<float>(a), as<float>(b), static_cast<std::int64_t>(n), d_out,
+                         reduction == OWTK_REDUCTION_COMPENSATED, mail);
+        ctx->await_mail();
+        *out = *d_out;
     });
 }
 
@@ -410,16 +425,16 @@ int owtk_reduction_norm(owtk_context ctx, int32_t reduction, owtk_dtype dtype, s
             return;
         }
         if (!a) throw std::invalid_argument("null vector");
-        double* d_out = ctx->scalars.get();
+        double* d_out = ctx->mail_values();
+        const auto mail = ctx->next_mail();
         if (dtype == OWTK_F64)
-            kern::norm_to(ctx->stream, ctx->scratch(), as<double>(a), static_cast<std::int64_t>(n), d_out,
-                          reduction != OWTK_REDUCTION_SERIAL);
+            kern::norm_to(ctx->stream, ctx->fused_scratch(), as<double>(a), static_cast<std::int64_t>(n), d_out,
+                          reduction != OWTK_REDUCTION_SERIAL, mail);
         else
-            kern::norm_to(ctx->stream, ctx->scratch(), as<float>(a), static_cast<std::int64_t>(n), d_out,
-                          reduction == OWTK_REDUCTION_COMPENSATED);
-        OWTK_HIP(hipMemcpyAsync(ctx->pinned.ptr, d_out, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-        *out = *static_cast<double*>(ctx->pinned.ptr);
+            kern::norm_to(ctx->stream, ctx->fused_scratch(), as<float>(a), static_cast<std::int64_t>(n), d_out,
+                          reduction == OWTK_REDUCTION_COMPENSATED, mail);
+        ctx->await_mail();
+        *out = *d_out;
     });
 }
 
@@ -446,11 +461,11 @@ int owtk_axpy_dot(owtk_context ctx, size_t n, double alpha, const double* x, dou
             return;
         }
         if (!x || !y || !w) throw std::invalid_argument("null vector");
-        double* d_out = ctx->scalars.get();
-        kern::axpy_dot_to(ctx->stream, ctx->scratch(), static_cast<std::int64_t>(n), alpha, x, y, w, d_out);
-        OWTK_HIP(hipMemcpyAsync(ctx->pinned.ptr, d_out, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-        *out = *static_cast<double*>(ctx->pinned.ptr);
+        double* d_out = ctx->mail_values();
+        const auto mail = ctx->next_mail();
+        kern::axpy_dot_to(ctx->stream, ctx->fused_scratch(), static_cast<std::int64_t>(n), alpha, x, y, w, d_out, mail);
+        ctx->await_mail();
+        *out = *d_out;
     });
 }
 
@@ -469,11 +484,11 @@ int owtk_multidot(owtk_context ctx, size_t n, size_t k, const double* const* vs,
         if (!w) throw std::invalid_argument("null vector");
         for (size_t j = 0; j < k; ++j)
             if (!vs[j]) throw std::invalid_argument("null basis vector");
-        double* d_out = ctx->scalars.get();
-        kern::multidot_to(ctx->stream, ctx->scratch(), static_cast<std::int64_t>(n), static_cast<int>(k), vs, w, d_out);
-        OWTK_HIP(hipMemcpyAsync(ctx->pinned.ptr, d_out, (k + 1) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-        std::copy_n(static_cast<double*>(ctx->pinned.ptr), k + 1, out);
+        double* d_out = ctx->mail_values();
+        const auto mail = ctx->next_mail();
+        kern::multidot_to(ctx->stream, ctx->fused_scratch(), static_cast<std::int64_t>(n), static_cast<int>(k), vs, w, d_out, mail);
+        ctx->await_mail();
+        std::copy_n(d_out, k + 1, out);
     });
 }
 

@@ -694,7 +694,7 @@ struct FgEngine {
                 return false;
             residual(b, cand, r, d_norm);
             ++cnt.ops;
-            if constexpr (sizeof(T) == 8) kern::norm_to(st, scratch, reinterpret_cast<const double*>(b), n, d_norm + 1);
+            if constexpr (sizeof(T) == 8) kern::norm_to(st, ctx->fused_scratch(), reinterpret_cast<const double*>(b), n, d_norm + 1);
             double two[2];
             OWTK_HIP(hipMemcpyAsync(two, d_norm, sizeof(two), hipMemcpyDeviceToHost, st));
             ctx->sync();
@@ -715,8 +715,8 @@ struct FgEngine {
         // ||b - A x|| and ||b|| in two slots, read back together
         residual(b, x, r, d_norm);
         ++cnt.ops;
-        if constexpr (sizeof(T) == 8) kern::norm_to(st, scratch, reinterpret_cast<const double*>(b), n, d_norm + 1);
-        else kern::norm_to(st, scratch, reinterpret_cast<const float*>(b), n, d_norm + 1);
+        if constexpr (sizeof(T) == 8) kern::norm_to(st, ctx->fused_scratch(), reinterpret_cast<const double*>(b), n, d_norm + 1);
+        else kern::norm_to(st, ctx->fused_scratch(), reinterpret_cast<const float*>(b), n, d_norm + 1);
         double pair[2];
         OWTK_HIP(hipMemcpyAsync(pair, d_norm, sizeof(pair), hipMemcpyDeviceToHost, st));
         ctx->sync();
@@ -893,7 +893,7 @@ struct FgEngine {
 
     template<int K, int L>
     void passes_l(int k, T* V, std::int64_t ld, T* w, T* vnext, FgState* s, unsigned int gr, hipStream_t st,
-                  ReduceScratch scratch)
+                ReduceScratch scratch)
     {
         const int count = k + 1;
         const int* halt = &s->halt;
@@ -910,7 +910,7 @@ struct FgEngine {
     }
 
     void launch_passes(int k, T* V, std::int64_t ld, T* w, T* vnext, FgState* s, unsigned int gr, hipStream_t st,
-                       ReduceScratch scratch)
+                ReduceScratch scratch)
     {
         const int need = k + 2;
         if (need <= 4) passes<4>(k, V, ld, w, vnext, s, gr, st, scratch);
@@ -1069,7 +1069,7 @@ int fgmres_refined_run(owtk_matrix m, owtk_precond pc, owtk_precond fallback, co
         return read();
     };
     // ||b|| and the initial ||b - A x||, read back together
-    kern::norm_to(st, scratch, b, n, d_norm);
+    kern::norm_to(st, ctx->fused_scratch(), b, n, d_norm);
     ++cnt.reds;
     launch_outer_residual(d_norm + 1);
     double pair[2];
@@ -1283,7 +1283,7 @@ bool rc_add(owtk_recycle_space sp, owtk_matrix m, const double* cand, double tol
         spmv_f64(m, vec.get(), e);
     }
     double* d_norm = ctx->scalars.get() + 24;
-    kern::norm_to(st, scratch, img.get(), n, d_norm);
+    kern::norm_to(st, ctx->fused_scratch(), img.get(), n, d_norm);
     const double orig = read_scalar(ctx, d_norm);
     count(tel, 1, 1);
     if (!std::isfinite(orig) || orig == 0.0) return reject();
@@ -1291,13 +1291,13 @@ bool rc_add(owtk_recycle_space sp, owtk_matrix m, const double* cand, double tol
     const unsigned int g = dev::stream_grid(n, 4);
     for (int pass = 0; pass < 2 && k > 0; ++pass) {
         const auto cp = pointers(sp->v.C);
-        kern::multidot_to(st, scratch, n, k, cp.v, img.get(), sp->coef.get());
+        kern::multidot_to(st, ctx->fused_scratch(), n, k, cp.v, img.get(), sp->coef.get());
         count(tel, 0, 1);
         k_rc_project<<<g, kBlock, 0, st>>>(vec.get(), img.get(), pointers(sp->v.U), cp, sp->coef.get(), k, n, -1.0,
                                            nullptr);
         OWTK_LAUNCH_CHECK();
     }
-    kern::norm_to(st, scratch, img.get(), n, d_norm);
+    kern::norm_to(st, ctx->fused_scratch(), img.get(), n, d_norm);
     const double nv = read_scalar(ctx, d_norm);
     count(tel, 0, 1);
     if (!std::isfinite(nv) || nv == 0.0 || nv / orig <= tol) return reject();
@@ -1331,7 +1331,7 @@ void rc_project(owtk_recycle_space sp, const double* r, double* x, owtk_solver_r
     if (k == 0) return;
     const hipStream_t st = sp->ctx->stream;
     const auto cp = pointers(sp->v.C);
-    kern::multidot_to(st, sp->ctx->scratch(), sp->n, k, cp.v, r, sp->coef.get());
+    kern::multidot_to(st, sp->ctx->fused_scratch(), sp->n, k, cp.v, r, sp->coef.get());
     count(tel, 0, 1);
     k_rc_project<<<dev::stream_grid(sp->n, 4), kBlock, 0, st>>>(x, nullptr, pointers(sp->v.U), cp, sp->coef.get(), k,
                                                                  sp->n, 1.0, nullptr);
@@ -1505,7 +1505,7 @@ int recycled_fgmres_run(owtk_matrix m, owtk_precond pc, const double* b, double*
         base_pc(in, out, stop);
         base_op(out, cached.get(), stop);
         if (k > 0) {
-            kern::multidot_to(st, scratch, n, k, cp.v, cached.get(), dcoef);
+            kern::multidot_to(st, ctx->fused_scratch(), n, k, cp.v, cached.get(), dcoef);
             k_rc_project<<<g, kBlock, 0, st>>>(out, cached.get(), up, cp, dcoef, k, n, -1.0, stop);
             OWTK_LAUNCH_CHECK();
         }

@@ -135,13 +135,13 @@ int idrs_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, const o
         ctx->sync();
     };
     auto dotv = [&](const double* a, const double* bb) {
-        kern::dot_to(st, scratch, a, bb, n, dsc.get());
+        kern::dot_to(st, ctx->fused_scratch(), a, bb, n, dsc.get());
         read(1);
         ++reds;
         return hsc[0];
     };
     auto nrmv = [&](const double* a) {
-        kern::norm_to(st, scratch, a, n, dsc.get());
+        kern::norm_to(st, ctx->fused_scratch(), a, n, dsc.get());
         read(1);
         ++reds;
         return hsc[0];
@@ -150,7 +150,7 @@ int idrs_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, const o
     auto pdots = [&](int first, int count, const double* a, double* out) {
         const double* vs[kMaxShadow];
         for (int j = 0; j < count; ++j) vs[j] = P(first + j);
-        kern::multidot_to(st, scratch, n, count, vs, a, dsc.get());
+        kern::multidot_to(st, ctx->fused_scratch(), n, count, vs, a, dsc.get());
         read(count);
         for (int j = 0; j < count; ++j) out[j] = hsc[j];
         reds += static_cast<std::uint64_t>(count);
@@ -205,7 +205,7 @@ int idrs_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, const o
     };
 
     // true_residual, norm(rhs), norm(residual): one operator application, two reductions
-    kern::norm_to(st, scratch, b, n, dsc.get() + 1);
+    kern::norm_to(st, ctx->fused_scratch(), b, n, dsc.get() + 1);
     {
         dev::EpiResidual e;
         e.y = r;
@@ -385,7 +385,7 @@ int idrs_run(owtk_matrix m, owtk_precond pc, const double* b, double* x, const o
         apply_op(z, w);
         {
             const double* vs[1] = {r};
-            kern::multidot_to(st, scratch, n, 1, vs, w, dsc.get());  // <w, r>, <w, w>
+            kern::multidot_to(st, ctx->fused_scratch(), n, 1, vs, w, dsc.get());  // <w, r>, <w, w>
             read(2);
             reds += 2;
         }

@@ -128,7 +128,22 @@ struct owtk_context_s {
     owtk::DeviceArray<unsigned char> refine_ws;
     std::int64_t refine_layout = -1, refine_owned = -1;
 
+    owtk::DeviceArray<unsigned int> ticket;  // block counter of the fused reductions
+    // scalar results that an entry point waits for: the finishing kernel
+    // writes them to pinned memory and then their number (Mail)
+    owtk::PinnedBuffer mail;
+    unsigned long long mail_number = 0;
+    owtk::dev::Mail next_mail() { return {mail_flag(), ++mail_number}; }
+    double* mail_values() const { return static_cast<double*>(mail.ptr); }
+    unsigned long long* mail_flag() const
+    {
+        return reinterpret_cast<unsigned long long*>(mail_values() + owtk::dev::kMaxReduceValues);
+    }
+    void await_mail() const;  // until the last next_mail() has arrived
     owtk::dev::ReduceScratch scratch() const { return {partials.get(), partial_stride}; }
+    // with the block counter, for kernels that end in reduce_end: small grids
+    // finish their reduction themselves (kernels of a context run one at a time)
+    owtk::dev::ReduceScratch fused_scratch() const { return {partials.get(), partial_stride, ticket.get()}; }
     // Grow the reduction partials to hold `blocks` blocks per value (waits for
     // the stream first: queued kernels may still use the old buffer).
     void reserve_partials(std::int64_t blocks);

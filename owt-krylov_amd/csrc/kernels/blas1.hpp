@@ -65,10 +65,21 @@ __global__ __launch_bounds__(256) void k_to_bf16(std::uint16_t* dst, const doubl
         dst[i] = float_to_bf16(static_cast<float>(src[i]));
 }
 
+struct FinStore {
+    double* out;
+    int count;
+    Mail mail = {};
+    __device__ void operator()(const double* t) const
+    {
+        if (threadIdx.x < count) out[threadIdx.x] = t[threadIdx.x];
+        mail.post();
+    }
+};
+
 // Dot product with FP64 accumulation; CMP: compensated (double-double).
 template<class X, bool CMP = false>
 __global__ __launch_bounds__(256) void k_dot(const X* __restrict__ a, const X* __restrict__ b, std::int64_t n,
-                                             ReduceScratch scratch, double* out)
+                                             ReduceScratch scratch, FinStore fin)
 {
     double red[1] = {0.0}, lo[1] = {0.0};
     const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
@@ -77,36 +88,43 @@ __global__ __launch_bounds__(256) void k_dot(const X* __restrict__ a, const X* _
         else red[0] = __builtin_fma(static_cast<double>(a[i]), static_cast<double>(b[i]), red[0]);
     }
     if constexpr (CMP) store_partials_dd<1>(red, lo, 0, scratch);
-    else store_partials<1>(red, 0, scratch);
+    else reduce_end<1>(red, 0, scratch, fin);
 }
-
-struct FinStore {
-    double* out;
-    int count;
-    __device__ void operator()(const double* t) const
-    {
-        if (threadIdx.x < count) out[threadIdx.x] = t[threadIdx.x];
-    }
-};
 
 template<class X>
 inline void dot_to(hipStream_t st, ReduceScratch scratch, const X* a, const X* b, std::int64_t n, double* out,
-                   bool compensated = false)
+                   bool compensated = false, Mail mail = {})
 {
     const unsigned int g = stream_grid(n, 4);
+    const FinStore fin{out, 1, mail};
     if (compensated) {
-        k_dot<X, true><<<g, kBlock, 0, st>>>(a, b, n, scratch, out);
-        launch_finish_dd<1>(st, FinStore{out, 1}, g, 0, scratch, nullptr);
+        k_dot<X, true><<<g, kBlock, 0, st>>>(a, b, n, scratch, fin);
+        launch_finish_dd<1>(st, fin, g, 0, scratch, nullptr);
     } else {
-        k_dot<X, false><<<g, kBlock, 0, st>>>(a, b, n, scratch, out);
-        launch_finish<1>(st, FinStore{out, 1}, g, 0, scratch, nullptr);
+        const ReduceScratch sc = scratch_for(scratch, g);
+        k_dot<X, false><<<g, kBlock, 0, st>>>(a, b, n, sc, fin);
+        launch_finish<1>(st, fin, g, 0, sc, nullptr);
     }
     OWTK_LAUNCH_CHECK();
 }
 
+template<class X>
+struct FinNorm {
+    const X* a;
+    std::int64_t n;
+    double* out;
+    Mail mail = {};
+    __device__ void operator()(const double* t) const
+    {
+        const double nrm = block_norm(t[0], t[1], a, n);
+        if (threadIdx.x == 0) *out = nrm;
+        mail.post();
+    }
+};
+
 template<class X, bool CMP = false>
 __global__ __launch_bounds__(256) void k_norm(const X* __restrict__ a, std::int64_t n, ReduceScratch scratch,
-                                              double* out)
+                                              FinNorm<X> fin)
 {
     double red[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
     const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
@@ -117,32 +135,22 @@ __global__ __launch_bounds__(256) void k_norm(const X* __restrict__ a, std::int6
         red[1] = combine<Combine::max>(red[1], __builtin_fabs(v));
     }
     if constexpr (CMP) store_partials_dd<2>(red, lo, 2, scratch);
-    else store_partials<2>(red, 2, scratch);
+    else reduce_end<2>(red, 2, scratch, fin);
 }
 
 template<class X>
-struct FinNorm {
-    const X* a;
-    std::int64_t n;
-    double* out;
-    __device__ void operator()(const double* t) const
-    {
-        const double nrm = block_norm(t[0], t[1], a, n);
-        if (threadIdx.x == 0) *out = nrm;
-    }
-};
-
-template<class X>
 inline void norm_to(hipStream_t st, ReduceScratch scratch, const X* a, std::int64_t n, double* out,
-                    bool compensated = false)
+                    bool compensated = false, Mail mail = {})
 {
     const unsigned int g = stream_grid(n, 4);
+    const FinNorm<X> fin{a, n, out, mail};
     if (compensated) {
-        k_norm<X, true><<<g, kBlock, 0, st>>>(a, n, scratch, out);
-        launch_finish_dd<2>(st, FinNorm<X>{a, n, out}, g, 2, scratch, nullptr);
+        k_norm<X, true><<<g, kBlock, 0, st>>>(a, n, scratch, fin);
+        launch_finish_dd<2>(st, fin, g, 2, scratch, nullptr);
     } else {
-        k_norm<X, false><<<g, kBlock, 0, st>>>(a, n, scratch, out);
-        launch_finish<2>(st, FinNorm<X>{a, n, out}, g, 2, scratch, nullptr);
+        const ReduceScratch sc = scratch_for(scratch, g);
+        k_norm<X, false><<<g, kBlock, 0, st>>>(a, n, sc, fin);
+        launch_finish<2>(st, fin, g, 2, sc, nullptr);
     }
     OWTK_LAUNCH_CHECK();
 }
@@ -209,7 +217,7 @@ inline void axpy(hipStream_t st, std::int64_t n, double alpha, const double* x, 
 
 __global__ __launch_bounds__(256) void k_axpy_dot(std::int64_t n, double alpha, const double* __restrict__ x,
                                                   double* __restrict__ y, const double* __restrict__ w,
-                                                  ReduceScratch scratch, double* out)
+                                                  ReduceScratch scratch, FinStore fin)
 {
     double red[1] = {0.0};
     const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
@@ -218,15 +226,17 @@ __global__ __launch_bounds__(256) void k_axpy_dot(std::int64_t n, double alpha, 
         y[i] = v;
         red[0] = __builtin_fma(w[i], v, red[0]);
     }
-    store_partials<1>(red, 0, scratch);
+    reduce_end<1>(red, 0, scratch, fin);
 }
 
 inline void axpy_dot_to(hipStream_t st, ReduceScratch scratch, std::int64_t n, double alpha, const double* x,
-                        double* y, const double* w, double* out)
+                        double* y, const double* w, double* out, Mail mail = {})
 {
     const unsigned int g = stream_grid(n, 4);
-    k_axpy_dot<<<g, kBlock, 0, st>>>(n, alpha, x, y, w, scratch, out);
-    launch_finish<1>(st, FinStore{out, 1}, g, 0, scratch, nullptr);
+    const ReduceScratch sc = scratch_for(scratch, g);
+    const FinStore fin{out, 1, mail};
+    k_axpy_dot<<<g, kBlock, 0, st>>>(n, alpha, x, y, w, sc, fin);
+    launch_finish<1>(st, fin, g, 0, sc, nullptr);
     OWTK_LAUNCH_CHECK();
 }
 
@@ -234,11 +244,24 @@ struct BasisPointers {
     const double* v[kMaxMultidot];
 };
 
+template<int K>
+struct FinMulti {
+    double* out;
+    int k;
+    Mail mail = {};
+    __device__ void operator()(const double* t) const
+    {
+        if (threadIdx.x < k) out[threadIdx.x] = t[threadIdx.x];
+        if (threadIdx.x == 0) out[k] = t[K - 1];
+        mail.post();
+    }
+};
+
 // out[j] = <w, v_j> (j < k), out[k] = <w, w>; K = reduced-value bucket >= k+1.
 template<int K>
 __global__ __launch_bounds__(256) void k_multidot(std::int64_t n, int k, BasisPointers basis,
                                                   const double* __restrict__ w, ReduceScratch scratch,
-                                                  double* out)
+                                                  FinMulti<K> fin)
 {
     double red[K];
 #pragma unroll
@@ -251,24 +274,13 @@ __global__ __launch_bounds__(256) void k_multidot(std::int64_t n, int k, BasisPo
             if (j < k) red[j] = __builtin_fma(wi, basis.v[j][i], red[j]);
         red[K - 1] = __builtin_fma(wi, wi, red[K - 1]);
     }
-    store_partials<K>(red, 0, scratch);
+    // (the finisher's 2 K values per thread would cost the wide kernels waves)
+    if constexpr (K <= 8) reduce_end<K>(red, 0, scratch, fin);
+    else store_partials<K>(red, 0, scratch);
 }
 
-template<int K>
-struct FinMulti {
-    double* out;
-    int k;
-    __device__ void operator()(const double* t) const
-    {
-        if (threadIdx.x == 0) {
-            for (int j = 0; j < k; ++j) out[j] = t[j];
-            out[k] = t[K - 1];
-        }
-    }
-};
-
 inline void multidot_to(hipStream_t st, ReduceScratch scratch, std::int64_t n, int k, const double* const* vs,
-                        const double* w, double* out)
+                        const double* w, double* out, Mail mail = {})
 {
     BasisPointers bp{};
     for (int j = 0; j < k; ++j) bp.v[j] = vs[j];
@@ -276,21 +288,23 @@ inline void multidot_to(hipStream_t st, ReduceScratch scratch, std::int64_t n, i
     if (blocks > kMultidotMaxBlocks) blocks = kMultidotMaxBlocks;
     if (blocks < 1) blocks = 1;
     const unsigned int g = static_cast<unsigned int>(blocks);
+    scratch = scratch_for(scratch, g);
+    if (k + 1 > 8) scratch.ticket = nullptr;
     if (k + 1 <= 4) {
-        k_multidot<4><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, out);
-        launch_finish<4>(st, FinMulti<4>{out, k}, g, 0, scratch, nullptr);
+        k_multidot<4><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, FinMulti<4>{out, k, mail});
+        launch_finish<4>(st, FinMulti<4>{out, k, mail}, g, 0, scratch, nullptr);
     } else if (k + 1 <= 8) {
-        k_multidot<8><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, out);
-        launch_finish<8>(st, FinMulti<8>{out, k}, g, 0, scratch, nullptr);
+        k_multidot<8><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, FinMulti<8>{out, k, mail});
+        launch_finish<8>(st, FinMulti<8>{out, k, mail}, g, 0, scratch, nullptr);
     } else if (k + 1 <= 16) {
-        k_multidot<16><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, out);
-        launch_finish<16>(st, FinMulti<16>{out, k}, g, 0, scratch, nullptr);
+        k_multidot<16><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, FinMulti<16>{out, k, mail});
+        launch_finish<16>(st, FinMulti<16>{out, k, mail}, g, 0, scratch, nullptr);
     } else if (k + 1 <= 32) {
-        k_multidot<32><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, out);
-        launch_finish<32>(st, FinMulti<32>{out, k}, g, 0, scratch, nullptr);
+        k_multidot<32><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, FinMulti<32>{out, k, mail});
+        launch_finish<32>(st, FinMulti<32>{out, k, mail}, g, 0, scratch, nullptr);
     } else {
-        k_multidot<63><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, out);
-        launch_finish<63>(st, FinMulti<63>{out, k}, g, 0, scratch, nullptr);
+        k_multidot<63><<<g, kBlock, 0, st>>>(n, k, bp, w, scratch, FinMulti<63>{out, k, mail});
+        launch_finish<63>(st, FinMulti<63>{out, k, mail}, g, 0, scratch, nullptr);
     }
     OWTK_LAUNCH_CHECK();
 }

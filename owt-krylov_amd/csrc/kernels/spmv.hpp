@@ -199,6 +199,23 @@ struct EpiFinish {
     __device__ void operator()(const double* t) const { e.finalize(t); }
 };
 
+// An epilogue whose kernel finishes its reduction itself (small grids).  A
+// type of its own, so that the finisher's registers stay out of the kernels
+// that stream large matrices.
+template<class E>
+struct Fused : E {
+    static constexpr bool kFused = true;
+};
+
+template<class E>
+__device__ inline void epi_end(const E& e, double (&red)[E::K > 0 ? E::K : 1], ReduceScratch scratch)
+{
+    if constexpr (E::K > 0) {
+        if constexpr (requires { E::kFused; }) reduce_end<E::K>(red, E::kMaxMask, scratch, EpiFinish<E>{e});
+        else store_partials<E::K>(red, E::kMaxMask, scratch);
+    }
+}
+
 } // namespace owtk::dev
 
 namespace owtk::kern {
@@ -299,7 +316,7 @@ __global__ __launch_bounds__(256) void spmv_sell_cd(const std::int32_t* __restri
         }
         epi_row<BS>(e, row * BS, acc, red);
     }
-    if constexpr (E::K > 0) store_partials<E::K>(red, E::kMaxMask, scratch);
+    epi_end(e, red, scratch);
 }
 
 // Launch spmv_sell_cd with the unroll that covers the matrix's slices.
@@ -382,7 +399,7 @@ __global__ __launch_bounds__(256) void spmv_csr_cd(const std::int32_t* __restric
         }
         e.elem(i, acc, red);
     }
-    if constexpr (E::K > 0) store_partials<E::K>(red, E::kMaxMask, scratch);
+    epi_end(e, red, scratch);
 }
 
 // Dense BSR, SELL-64 layout, one lane per row, BS x BS blocks.
@@ -461,7 +478,7 @@ __global__ __launch_bounds__(256) void spmv_sell_bsr(const std::int32_t* __restr
 #pragma unroll
         for (int r = 0; r < BS; ++r) e.elem(row * BS + r, acc[r], red);
     }
-    if constexpr (E::K > 0) store_partials<E::K>(red, E::kMaxMask, scratch);
+    epi_end(e, red, scratch);
 }
 
 // Dense BSR for any block size, reference CSR layout: one thread per
@@ -494,7 +511,7 @@ __global__ __launch_bounds__(256) void spmv_csr_bsr(const std::int32_t* __restri
         }
         e.elem(i, acc, red);
     }
-    if constexpr (E::K > 0) store_partials<E::K>(red, E::kMaxMask, scratch);
+    epi_end(e, red, scratch);
 }
 
 } // namespace owtk::kern
@@ -504,24 +521,16 @@ namespace owtk {
 // Launch the SpMV of m with value storage `dtype` and epilogue e.  V/X are
 // deduced from dtype by the caller through the typed entry below.
 template<class V, class X, class E>
-void spmv_dispatch(owtk_matrix m, const V* vals, const V* diag, const X* x, E e)
+void spmv_launch(owtk_matrix m, unsigned int grid, const V* vals, const V* diag, const X* x, E e, dev::ReduceScratch scratch)
 {
     using namespace owtk::kern;
     const hipStream_t st = m->ctx->stream;
-    const auto scratch = m->ctx->scratch();
     const auto& s = m->s;
     const std::int64_t rows = m->owned;
     constexpr int sv = static_cast<int>(sizeof(V));
     constexpr int category = sv == 8 ? prof_spmv_f64 : (sv == 4 ? prof_spmv_f32 : prof_spmv_bf16);
     ProfileScope prof(m->ctx, category, spmv_bytes(m, sv, static_cast<int>(sizeof(X))));
-    unsigned int launched = 0;
     if (s.layout == Layout::sell) {
-        const std::int64_t blocks = (rows + kBlock - 1) / kBlock;
-        if (E::K > 0 && blocks > scratch.stride)
-            throw std::logic_error("reduction partials smaller than the SpMV grid");
-        if (blocks > 0x7fffffff) throw std::invalid_argument("too many rows");
-        const unsigned int grid = static_cast<unsigned int>(blocks);
-        launched = grid;
         if (m->dense()) {
             // slots per pass: 2 for FP32/BF16 values (4x4 BF16 blocks of a
             // 1M-vertex grid: 54.6 -> 50.7 us), 1 for FP64, whose 16 values
@@ -543,12 +552,8 @@ void spmv_dispatch(owtk_matrix m, const V* vals, const V* diag, const X* x, E e)
         }
     } else {
         if (m->dense()) {
-            const unsigned int grid = stream_grid(rows * m->bs);
-            launched = grid;
             spmv_csr_bsr<V, X, E><<<grid, kBlock, 0, st>>>(s.offsets.get(), s.columns.get(), vals, x, rows, m->bs, e, scratch);
         } else {
-            const unsigned int grid = stream_grid(rows * m->bs);
-            launched = grid;
             if (m->has_diag_array())
                 spmv_csr_cd<V, X, true, E, 8><<<grid, kBlock, 0, st>>>(s.offsets.get(), s.columns.get(), vals, diag, x, rows, m->bs, e, scratch);
             else
@@ -557,9 +562,32 @@ void spmv_dispatch(owtk_matrix m, const V* vals, const V* diag, const X* x, E e)
     }
     OWTK_LAUNCH_CHECK();
     if constexpr (E::K > 0) {
-        launch_finish<E::K>(st, EpiFinish<E>{e}, launched, E::kMaxMask, scratch, e.stop);
+        launch_finish<E::K>(st, EpiFinish<E>{e}, grid, E::kMaxMask, scratch, e.stop);
         OWTK_LAUNCH_CHECK();
     }
+}
+
+template<class V, class X, class E>
+void spmv_dispatch(owtk_matrix m, const V* vals, const V* diag, const X* x, E e)
+{
+    const std::int64_t rows = m->owned;
+    unsigned int grid;
+    if (m->s.layout == Layout::sell) {
+        const std::int64_t blocks = (rows + dev::kBlock - 1) / dev::kBlock;
+        if (E::K > 0 && blocks > m->ctx->scratch().stride)
+            throw std::logic_error("reduction partials smaller than the SpMV grid");
+        if (blocks > 0x7fffffff) throw std::invalid_argument("too many rows");
+        grid = static_cast<unsigned int>(blocks);
+    } else {
+        grid = dev::stream_grid(rows * m->bs);
+    }
+    if constexpr (E::K > 0) {
+        if (grid <= dev::kFuseBlocks) {
+            spmv_launch<V, X>(m, grid, vals, diag, x, dev::Fused<E>{e}, m->ctx->fused_scratch());
+            return;
+        }
+    }
+    spmv_launch<V, X>(m, grid, vals, diag, x, e, m->ctx->scratch());
 }
 
 // FP64 SpMV with an epilogue (the solver path).

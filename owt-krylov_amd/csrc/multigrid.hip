@@ -813,7 +813,7 @@ int mg_solve(owtk_multigrid_s* mg, const double* b, double* x, const owtk_solver
         OWTK_LAUNCH_CHECK();
     };
 
-    kern::norm_to(st, scratch, b, n, d_norm);
+    kern::norm_to(st, ctx->fused_scratch(), b, n, d_norm);
     ++reds;
     const double rhs_norm = read_norm();
     if (!std::isfinite(rhs_norm)) {

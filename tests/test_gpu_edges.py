@@ -176,3 +176,51 @@ def test_chain_sweeps(ctx, n, block, block_nodes, reach, count):
         wd = ctx.empty(n * block, np.float32)
         low.apply(ctx.upload(x.astype(np.float32)), wd)
         assert np.max(np.abs(wd.download() - ref)) <= 2.0 ** 29 * 1e-14 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("n", [1, 2, 1023, 1024, 1025, 6144, 128 * 1024, 128 * 1024 + 1, 300_001])
+def test_reductions_around_the_fused_grid(ctx, n):
+    """Reductions that end in the kernel itself (up to 128 blocks of 1,024 values) and in a finisher, several in a
+    row on one counter.  Tree sums of n products: a few ulp of the sum of magnitudes, 1e-14 holds with room; the
+    norms of extreme values take the scaled second pass."""
+    rng = np.random.default_rng(n)
+    a, b = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    da, db, dy = ctx.upload(a), ctx.upload(b), ctx.upload(b)
+    basis = [ctx.upload(rng.uniform(-1, 1, n)) for _ in range(9)]
+    host = [v.download() for v in basis]
+    for _ in range(3):
+        assert abs(ctx.dot(da, db) - np.dot(a, b)) <= 1e-14 * np.sum(np.abs(a * b))
+        assert abs(ctx.norm(da) - np.linalg.norm(a)) <= 1e-14 * np.linalg.norm(a)
+        for k in (0, 1, 3, 7, 8, 9):
+            got = ctx.multidot(basis[:k], da)
+            ref = np.array([np.dot(a, v) for v in host[:k]] + [np.dot(a, a)])
+            assert np.all(np.abs(got - ref) <= 1e-14 * n)
+    y = b + 0.25 * a
+    assert abs(ctx.axpy_dot(0.25, da, dy, db) - np.dot(b, y)) <= 1e-14 * np.sum(np.abs(b * y))
+    assert np.allclose(dy.download(), y, rtol=0, atol=1e-15)
+    for scale in (1e300, 1e-300):
+        assert abs(ctx.norm(ctx.upload(a * scale)) - np.linalg.norm(a) * scale) <= 1e-13 * np.linalg.norm(a) * scale
+    assert np.isnan(ctx.norm(ctx.upload(np.where(np.arange(n) == n // 2, np.nan, a))))
+    assert np.isinf(ctx.norm(ctx.upload(np.where(np.arange(n) == n - 1, -np.inf, a))))
+
+
+@pytest.mark.parametrize("nx,ny,block", [(5, 3, 1), (128, 128, 2), (128, 256, 1), (130, 255, 3), (130, 130, 5)])
+def test_solvers_around_the_fused_grid(ctx, nx, ny, block):
+    """BiCGSTAB, its pipelined and communication-hiding forms on grids below, at and above 128 SpMV blocks (256 rows)
+    and vector blocks, against the oracle at rtol 1e-8.  The iteration counts agree to one there (near 1e-12, after
+    twice the iterations, the sums' rounding has decoupled the recurrences and they drift by several).  A row's
+    diagonal exceeds the sum of its other entries by 0.05, so |A^-1| <= 20 in the maximum norm and residuals of
+    1e-8 |b| leave the two solutions at most 4e-7 |b| apart."""
+    s = owtk.generate_split(nx, ny, block, 4, ordering=owtk.ORDER_RCM)
+    om = orc.OMatrix.split(s.nodes, 0, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    m = owtk.Matrix.split(ctx, s.nodes, 0, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    pc, opc = owtk.Preconditioner(m, owtk.PC_JACOBI), orc.OPreconditioner(om, orc.OPreconditioner.JACOBI)
+    b, x = ctx.upload(s.rhs), ctx.empty(s.nodes * block)
+    ref, ro = orc.bicgstab(om, opc, s.rhs, relative_tolerance=1e-8, maximum_iterations=500)
+    for solve in (owtk.bicgstab, owtk.pipelined_bicgstab, owtk.communication_hiding_bicgstab):
+        x.zero()
+        res = solve(m, pc, b, x, owtk.SolverOptions(relative_tolerance=1e-8, maximum_iterations=500))
+        assert res["status_name"] == "converged"
+        if solve is owtk.bicgstab:
+            assert abs(res["iterations"] - ro["iterations"]) <= 1
+        assert np.max(np.abs(x.download() - ref)) <= 4e-7 * np.linalg.norm(s.rhs)
