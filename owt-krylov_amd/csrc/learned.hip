@@ -671,23 +671,73 @@ __global__ __launch_bounds__(256) void k_outer_finish(const float* __restrict__ 
 
 // ------------------------------------------------------------ loss kernels --
 
-// z[p] = sum_k gamma_k * u[p][k]
+// The loss kernels take one thread per unknown q = (vertex, component) and PP
+// pairs at a time.  z, ys and g are kept pair-minor, [q][P], so an edge's
+// gather is one run of PP values per thread and 3 PP values per vertex, and
+// the matrix is read once for all of them.  (Pair-major vectors with a thread
+// per vertex and pair read columns and values again for every component and
+// pair: 104 and 111 us for y and g at 131,072 vertices and 10 pairs, 42 and
+// 35 us this way; z, bound by reading u, stays at 25, dgamma 24 -> 21.)
+
+// z_p = sum_k gamma_k * u[p][k]
+template<int PP>
 __global__ __launch_bounds__(256) void k_loss_z(std::int64_t nb, int pairs, int k1, const float* __restrict__ gamma,
                                                 const float* __restrict__ u, float* __restrict__ z)
 {
-    const std::int64_t total = nb * pairs;
-    const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
-    for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total; t += step) {
-        const std::int64_t p = t / nb, q = t - p * nb;
-        float s = 0.f;
-        for (int k = 0; k < k1; ++k) s = __builtin_fmaf(gamma[k * nb + q], u[(p * k1 + k) * nb + q], s);
-        z[t] = s;
+    const std::int64_t q = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (q >= nb) return;
+    for (int p0 = 0; p0 < pairs; p0 += PP) {
+        float acc[PP];
+#pragma unroll
+        for (int j = 0; j < PP; ++j) acc[j] = 0.f;
+        for (int k = 0; k < k1; ++k) {
+            const float gk = gamma[k * nb + q];
+#pragma unroll
+            for (int j = 0; j < PP; ++j) {
+                const int p = p0 + j < pairs ? p0 + j : pairs - 1;
+                acc[j] = __builtin_fmaf(gk, u[(static_cast<std::int64_t>(p) * k1 + k) * nb + q], acc[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PP; ++j)
+            if (p0 + j < pairs) z[q * pairs + p0 + j] = acc[j];
+    }
+}
+
+// Edges of q's row summed for PP pairs from p0: acc_j += a_e v[col(e)][p0 + j].
+// MIRROR: the entry of the transposed matrix.
+template<int PP, bool MIRROR>
+__device__ inline void loss_row(float (&acc)[PP], std::int32_t begin, std::int32_t end, int b, int c, int pairs, int p0,
+                                const std::int32_t* __restrict__ cols, const std::int32_t* __restrict__ mirror,
+                                const float* __restrict__ vals, const float* __restrict__ v)
+{
+    constexpr int U = 2;  // edges in flight
+    for (std::int32_t e0 = begin; e0 < end; e0 += U) {
+        float a[U], x[U][PP];
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+            const std::int32_t e = e0 + t < end ? e0 + t : end - 1;
+            const std::int64_t at = MIRROR ? mirror[e] : e;
+            a[t] = vals[at * b + c];
+            const float* row = v + (static_cast<std::int64_t>(cols[e]) * b + c) * pairs;
+#pragma unroll
+            for (int j = 0; j < PP; ++j) x[t][j] = row[p0 + j < pairs ? p0 + j : pairs - 1];
+        }
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+#pragma unroll
+            for (int j = 0; j < PP; ++j) {
+                const float f = __builtin_fmaf(a[t], x[t][j], acc[j]);
+                acc[j] = e0 + t < end ? f : acc[j];
+            }
+        }
     }
 }
 
 // y = D^-1/2 A z_p - target_p; ys = D^-1/2 y; partial sums of coef_p y^2.
-// Grid: (row blocks, pairs).
-__global__ __launch_bounds__(256) void k_loss_y(std::int64_t n, int b, const std::int32_t* __restrict__ offsets,
+template<int PP>
+__global__ __launch_bounds__(256) void k_loss_y(std::int64_t n, int b, int pairs,
+                                                const std::int32_t* __restrict__ offsets,
                                                 const std::int32_t* __restrict__ cols,
                                                 const float* __restrict__ vals, const float* __restrict__ diag,
                                                 const float* __restrict__ dis, const float* __restrict__ z,
@@ -695,24 +745,31 @@ __global__ __launch_bounds__(256) void k_loss_y(std::int64_t n, int b, const std
                                                 float* __restrict__ ys, double* __restrict__ partials)
 {
     const std::int64_t nb = n * b;
-    const int p = blockIdx.y;
-    const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const std::int64_t q = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     double local = 0.0;
-    if (i < n) {
-        const float* zp = z + p * nb;
-        for (int c = 0; c < b; ++c) {
-            float acc = diag[i * b + c] * zp[i * b + c];
-            for (std::int32_t e = offsets[i]; e < offsets[i + 1]; ++e)
-                acc = __builtin_fmaf(vals[static_cast<std::int64_t>(e) * b + c], zp[static_cast<std::int64_t>(cols[e]) * b + c], acc);
-            const float d = dis[i * b + c];
-            const float y = d * acc - target[p * nb + i * b + c];
-            ys[p * nb + i * b + c] = d * y;
-            local += static_cast<double>(y) * static_cast<double>(y);
+    if (q < nb) {
+        const std::int64_t i = q / b;
+        const int c = static_cast<int>(q - i * b);
+        const std::int32_t begin = offsets[i], end = offsets[i + 1];
+        const float d = dis[q], dq = diag[q];
+        for (int p0 = 0; p0 < pairs; p0 += PP) {
+            float acc[PP];
+#pragma unroll
+            for (int j = 0; j < PP; ++j) acc[j] = dq * z[q * pairs + (p0 + j < pairs ? p0 + j : pairs - 1)];
+            loss_row<PP, false>(acc, begin, end, b, c, pairs, p0, cols, nullptr, vals, z);
+#pragma unroll
+            for (int j = 0; j < PP; ++j) {
+                const int p = p0 + j;
+                if (p < pairs) {
+                    const float y = d * acc[j] - target[p * nb + q];
+                    ys[q * pairs + p] = d * y;
+                    local += static_cast<double>(coef[p]) * (static_cast<double>(y) * static_cast<double>(y));
+                }
+            }
         }
-        local *= static_cast<double>(coef[p]);
     }
     const double s = dev::block_sum_all(local);
-    if (threadIdx.x == 0) partials[static_cast<std::int64_t>(p) * gridDim.x + blockIdx.x] = s;
+    if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
 __global__ void k_loss_finish(const double* __restrict__ partials, int count, double scale, double* __restrict__ loss)
@@ -724,38 +781,54 @@ __global__ void k_loss_finish(const double* __restrict__ partials, int count, do
 }
 
 // g_p = gcoef_p A^T ys_p   (transposed SpMV through the mirror index)
-__global__ __launch_bounds__(256) void k_loss_g(std::int64_t n, int b, const std::int32_t* __restrict__ offsets,
+template<int PP>
+__global__ __launch_bounds__(256) void k_loss_g(std::int64_t n, int b, int pairs,
+                                                const std::int32_t* __restrict__ offsets,
                                                 const std::int32_t* __restrict__ cols,
                                                 const std::int32_t* __restrict__ mirror,
                                                 const float* __restrict__ vals, const float* __restrict__ diag,
                                                 const float* __restrict__ ys, const float* __restrict__ gcoef,
                                                 float* __restrict__ gout)
 {
-    const std::int64_t nb = n * b;
-    const int p = blockIdx.y;
-    const std::int64_t j = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const float* yp = ys + p * nb;
-    for (int c = 0; c < b; ++c) {
-        float g = diag[j * b + c] * yp[j * b + c];
-        for (std::int32_t e = offsets[j]; e < offsets[j + 1]; ++e)
-            g = __builtin_fmaf(vals[static_cast<std::int64_t>(mirror[e]) * b + c],
-                               yp[static_cast<std::int64_t>(cols[e]) * b + c], g);
-        gout[p * nb + j * b + c] = g * gcoef[p];
+    const std::int64_t q = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (q >= n * b) return;
+    const std::int64_t i = q / b;
+    const int c = static_cast<int>(q - i * b);
+    const std::int32_t begin = offsets[i], end = offsets[i + 1];
+    const float dq = diag[q];
+    for (int p0 = 0; p0 < pairs; p0 += PP) {
+        float acc[PP];
+#pragma unroll
+        for (int j = 0; j < PP; ++j) acc[j] = dq * ys[q * pairs + (p0 + j < pairs ? p0 + j : pairs - 1)];
+        loss_row<PP, true>(acc, begin, end, b, c, pairs, p0, cols, mirror, vals, ys);
+#pragma unroll
+        for (int j = 0; j < PP; ++j)
+            if (p0 + j < pairs) gout[q * pairs + p0 + j] = acc[j] * gcoef[p0 + j];
     }
 }
 
-// dgamma_k = sum_p g_p * u[p][k]
+// dgamma_k = sum_p g_p * u[p][k], KK coefficients at a time
+template<int KK>
 __global__ __launch_bounds__(256) void k_loss_dgamma(std::int64_t nb, int pairs, int k1, const float* __restrict__ g,
                                                      const float* __restrict__ u, float* __restrict__ dgamma)
 {
-    const std::int64_t total = nb * k1;
-    const std::int64_t step = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
-    for (std::int64_t t = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; t < total; t += step) {
-        const std::int64_t k = t / nb, q = t - k * nb;
-        float s = 0.f;
-        for (int p = 0; p < pairs; ++p) s = __builtin_fmaf(g[p * nb + q], u[(p * k1 + k) * nb + q], s);
-        dgamma[t] = s;
+    const std::int64_t q = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (q >= nb) return;
+    for (int k0 = 0; k0 < k1; k0 += KK) {
+        float acc[KK];
+#pragma unroll
+        for (int j = 0; j < KK; ++j) acc[j] = 0.f;
+        for (int p = 0; p < pairs; ++p) {
+            const float gp = g[q * pairs + p];
+#pragma unroll
+            for (int j = 0; j < KK; ++j) {
+                const int k = k0 + j < k1 ? k0 + j : k1 - 1;
+                acc[j] = __builtin_fmaf(gp, u[(static_cast<std::int64_t>(p) * k1 + k) * nb + q], acc[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < KK; ++j)
+            if (k0 + j < k1) dgamma[(k0 + j) * nb + q] = acc[j];
     }
 }
 
@@ -1177,7 +1250,7 @@ TrainViews ensure_workspace(owtk_gnn model, std::int64_t n, int pairs, int k1, i
         model->dgamma.allocate(nn * b * k1);
         model->z.allocate(nn * b * pp);
         model->ys.allocate(nn * b * pp);
-        model->loss_partials.allocate(rows_grid(nn) * pp);
+        model->loss_partials.allocate(rows_grid(nn * b));
         model->coef.allocate(2 * pp);
         model->ws_nodes = nn;
         model->ws_pairs = pp;
@@ -1212,21 +1285,28 @@ void accumulate(owtk_gnn model, owtk_gnn_problem prob, double weight)
 
     forward(model, g, v.h, v.agg, model->gamma.get(), true);
     const unsigned int grid = rows_grid(n);
-    k_loss_z<<<dev::stream_grid(nb * P, 4), kBlock, 0, st>>>(nb, P, k1, model->gamma.get(), prob->u.get(), model->z.get());
-    OWTK_LAUNCH_CHECK();
-    k_loss_y<<<dim3(grid, P), kBlock, 0, st>>>(n, g.b, g.offsets.get(), g.cols.get(), g.vals.get(), g.diag.get(),
+    // pairs in registers: 10 cover the solver's usual set in one pass
+    const unsigned int lgrid = rows_grid(nb);
+    auto loss = [&](auto pp) {
+        constexpr int PP = decltype(pp)::value;
+        k_loss_z<PP><<<lgrid, kBlock, 0, st>>>(nb, P, k1, model->gamma.get(), prob->u.get(), model->z.get());
+        OWTK_LAUNCH_CHECK();
+        k_loss_y<PP><<<lgrid, kBlock, 0, st>>>(n, g.b, P, g.offsets.get(), g.cols.get(), g.vals.get(), g.diag.get(),
                                                prob->dis.get(), model->z.get(), prob->target.get(), model->coef.get(),
                                                model->ys.get(), model->loss_partials.get());
-    OWTK_LAUNCH_CHECK();
-    k_loss_finish<<<1, kBlock, 0, st>>>(model->loss_partials.get(), static_cast<int>(grid) * P, weight / P,
-                                        model->loss.get());
-    OWTK_LAUNCH_CHECK();
-    // z is free again: it holds g_p = gcoef_p A^T ys_p
-    k_loss_g<<<dim3(grid, P), kBlock, 0, st>>>(n, g.b, g.offsets.get(), g.cols.get(), g.mirror.get(), g.vals.get(),
+        OWTK_LAUNCH_CHECK();
+        k_loss_finish<<<1, kBlock, 0, st>>>(model->loss_partials.get(), static_cast<int>(lgrid), weight / P,
+                                            model->loss.get());
+        OWTK_LAUNCH_CHECK();
+        // z is free again: it holds g_p = gcoef_p A^T ys_p
+        k_loss_g<PP><<<lgrid, kBlock, 0, st>>>(n, g.b, P, g.offsets.get(), g.cols.get(), g.mirror.get(), g.vals.get(),
                                                g.diag.get(), model->ys.get(), model->coef.get() + P, model->z.get());
-    OWTK_LAUNCH_CHECK();
-    k_loss_dgamma<<<dev::stream_grid(nb * k1, 4), kBlock, 0, st>>>(nb, P, k1, model->z.get(), prob->u.get(),
-                                                                   model->dgamma.get());
+        OWTK_LAUNCH_CHECK();
+    };
+    if (P <= 2) loss(std::integral_constant<int, 2>{});
+    else if (P <= 5) loss(std::integral_constant<int, 5>{});
+    else loss(std::integral_constant<int, 10>{});
+    k_loss_dgamma<5><<<lgrid, kBlock, 0, st>>>(nb, P, k1, model->z.get(), prob->u.get(), model->dgamma.get());
     OWTK_LAUNCH_CHECK();
 
     float* grad = model->grad.get();

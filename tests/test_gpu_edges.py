@@ -81,6 +81,31 @@ def test_training_gradient_sizes(ctx, nx, ny, block, degree):
         assert np.linalg.norm(got[k] - ref[k]) <= 2e-3 * max(np.linalg.norm(ref[k]), 1e-6 * np.linalg.norm(ref_grad)), k
 
 
+@pytest.mark.parametrize("block,pairs", [(1, 1), (4, 2), (2, 3), (3, 5), (1, 6), (3, 10), (2, 11), (1, 21)])
+def test_training_loss_pairs(ctx, block, pairs):
+    """Pair counts at and beyond every register width of the loss kernels (2, 5, 10), rows of unequal length, and a
+    row count that leaves the last block ragged; bounds as in the test above."""
+    s = owtk.generate_split(23, 17, block, 5, ordering=owtk.ORDER_RCM)
+    m = owtk.Matrix.split(ctx, s.nodes, 0, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    g = gnn.Graph(s.nodes, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    rng = np.random.default_rng(pairs)
+    errs = [rng.uniform(-1, 1, (s.nodes, block)) * 10.0 ** (p % 3) for p in range(pairs)]
+    ress = [g.apply(e) for e in errs]
+    lay = gnn.Layout(block, 2)
+    params = gnn.init_parameters(block, 2, 4).astype(np.float32)
+    model = owtk.GnnModel(ctx, block, 2)
+    model.set_parameters(params)
+    prob = model.problem(m, ctx.upload(np.concatenate(ress).ravel()), ctx.upload(np.concatenate(errs).ravel()), pairs)
+    model.zero_grad()
+    model.accumulate(prob, 0.75)
+    loss, grad = model.read()
+    ref_loss, ref_grad = gnn.loss_and_grad(g, gnn.bf16_round(params), 2, ress, errs)
+    got, ref = lay.unpack(grad.astype(np.float64)), lay.unpack(0.75 * ref_grad)
+    assert abs(loss - 0.75 * ref_loss) <= 1e-4 * ref_loss
+    for k in ref:
+        assert np.linalg.norm(got[k] - ref[k]) <= 2e-3 * max(np.linalg.norm(ref[k]), 1e-6 * np.linalg.norm(ref_grad)), k
+
+
 def random_dominant(rng, n, block, low, high):
     """A diagonally dominant CSR matrix with low..high off-diagonal entries per row at random columns near the
     diagonal (no symmetric pattern)."""
