@@ -340,12 +340,12 @@ __global__ __launch_bounds__(256) void k_ilu_factor(TriArgs a, const std::int32_
 //   3. the chunk's own lower entries run in 64 steps: at step s row s is
 //      final, and every lane whose row has an entry in column s divides by
 //      row s's pivot and updates its targets from row s's entries (read from
-//      LDS), which keeps each row's column order.  With a bound NUB on the
-//      updates per op, a step's reads go out together and its updates take
-//      no branch (an ILU(0) factor of a triangulated grid has NUB = 3);
+//      LDS), which keeps each row's column order;
 //   4. the chunk's rows are stored, fenced for the next chunks' gathers.
 // Each row sees the same operations in the same order as the reference's
 // loop, so the factors are bitwise those of the level-scheduled kernel.
+// This general form takes any number of updates per operation; with at most
+// seven k_ilu_factor_rec runs.
 struct IluChunkArgs {
     const std::int32_t* chunk_first;
     const std::int64_t* hdr;
@@ -354,6 +354,7 @@ struct IluChunkArgs {
     const std::uint32_t* op_b;
     const std::uint16_t* upd_a;
     const std::uint16_t* upd_b;
+    const std::uint32_t* rec;
     int kmax, max_src, max_a, max_nua, max_b, max_nub;
 };
 
@@ -378,63 +379,6 @@ __device__ inline void copy_batched(int count, Load load, Store store)
     }
 }
 
-// A chunk's header, row extents, program words and row values held in
-// registers (the prefetching kernel loads chunk ch + 1's during chunk ch).
-// Its caps bound the chunk's row length and program sizes.
-constexpr int kPfRows = 16, kPfOps = 16, kPfUpdates = 48;
-struct ChunkPrefetch {
-    std::int64_t row_first, src_off, base;
-    int cnt, nsrc, na, nua, nb, nub, len;
-    double vd[kPfRows];
-    std::uint32_t v32[kPfOps];      // op words: earlier-chunk ops, then this chunk's
-    std::uint16_t v16[kPfUpdates];  // update words, likewise
-};
-
-// Header, row extents and program words of chunk ch (no row values).
-__device__ inline void prefetch_program(const IluChunkArgs& P, const std::int64_t* __restrict__ offsets, int ch,
-                                        int lane, ChunkPrefetch& n)
-{
-    const std::int64_t* h = P.hdr + static_cast<std::int64_t>(ch) * 12;
-    n.row_first = h[0];
-    n.cnt = static_cast<int>(h[1]);
-    n.src_off = h[2];
-    n.nsrc = static_cast<int>(h[3]);
-    const std::int64_t opa_off = h[4], upa_off = h[6], opb_off = h[8], upb_off = h[10];
-    n.na = static_cast<int>(h[5]);
-    n.nua = static_cast<int>(h[7]);
-    n.nb = static_cast<int>(h[9]);
-    n.nub = static_cast<int>(h[11]);
-    n.base = 0;
-    n.len = 0;
-    if (lane < n.cnt) {
-        n.base = offsets[n.row_first + lane];
-        n.len = static_cast<int>(offsets[n.row_first + lane + 1] - n.base);
-    }
-    const int n32 = n.na + n.nb, na16 = n.na * n.nua, n16 = na16 + n.nb * n.nub;
-#pragma unroll
-    for (int j = 0; j < kPfOps; ++j)
-        if (j < n32) n.v32[j] = j < n.na ? P.op_a[opa_off + j * 64 + lane] : P.op_b[opb_off + (j - n.na) * 64 + lane];
-#pragma unroll
-    for (int j = 0; j < kPfUpdates; ++j)
-        if (j < n16) n.v16[j] = j < na16 ? P.upd_a[upa_off + j * 64 + lane] : P.upd_b[upb_off + (j - na16) * 64 + lane];
-}
-
-// Row values of a prefetched chunk (after its row extents have arrived).
-__device__ inline void prefetch_rows(const double* __restrict__ Fc, int kmax, ChunkPrefetch& n)
-{
-    const int lastq = n.len > 0 ? n.len - 1 : 0;
-#pragma unroll
-    for (int q = 0; q < kPfRows; ++q)
-        if (q < kmax) n.vd[q] = Fc[n.base + (q < lastq ? q : lastq)];
-}
-
-inline bool ilu_chunks_prefetchable(const IluChunkProgram& P)
-{
-    return P.kmax <= kPfRows && P.max_a + P.max_b <= kPfOps
-           && P.max_a * P.max_nua + P.max_b * P.max_nub <= kPfUpdates;
-}
-
-template<int NUB, bool PF>
 __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const std::int64_t* __restrict__ offsets,
                                                           const std::int64_t* __restrict__ diag_pos,
                                                           const std::int32_t* __restrict__ row0,
@@ -454,43 +398,14 @@ __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const 
     auto* upa = reinterpret_cast<std::uint16_t*>(opb + P.max_b * 64);  // [max_a*max_nua][64]
     std::uint16_t* upb = upa + P.max_a * P.max_nua * 64;  // [max_b*max_nub][64]
     const int ch_end = P.chunk_first[b + 1];
-    ChunkPrefetch cur, nxt;
-    if constexpr (PF) {
-        if (P.chunk_first[b] < ch_end) {
-            prefetch_program(P, offsets, P.chunk_first[b], lane, cur);
-            prefetch_rows(Fc, P.kmax, cur);
-        }
-    }
     for (int ch = P.chunk_first[b]; ch < ch_end; ++ch) {
         const std::int64_t* h = P.hdr + static_cast<std::int64_t>(ch) * 12;
-        const int cnt = PF ? cur.cnt : static_cast<int>(h[1]);
-        const std::int64_t src_off = PF ? cur.src_off : h[2];
-        const int nsrc = PF ? cur.nsrc : static_cast<int>(h[3]);
-        const int na = PF ? cur.na : static_cast<int>(h[5]), nua = PF ? cur.nua : static_cast<int>(h[7]);
-        const int nb = PF ? cur.nb : static_cast<int>(h[9]), nub = PF ? cur.nub : static_cast<int>(h[11]);
+        const int cnt = static_cast<int>(h[1]), nsrc = static_cast<int>(h[3]);
+        const std::int64_t src_off = h[2];
+        const int na = static_cast<int>(h[5]), nua = static_cast<int>(h[7]);
+        const int nb = static_cast<int>(h[9]), nub = static_cast<int>(h[11]);
         std::int64_t base = 0;
         int len = 0;
-        if constexpr (PF) {
-            // 1. the prefetched row values and program into LDS; then chunk
-            //    ch + 1's header, row extents and program start loading
-            base = cur.base;
-            len = cur.len;
-#pragma unroll
-            for (int q = 0; q < kPfRows; ++q)
-                if (q < P.kmax) rv[q * 64 + lane] = q < len ? cur.vd[q] : 0.0;
-            const int na16 = na * nua;
-#pragma unroll
-            for (int j = 0; j < kPfOps; ++j) {
-                if (j < na) opa[j * 64 + lane] = cur.v32[j];
-                else if (j < na + nb) opb[(j - na) * 64 + lane] = cur.v32[j];
-            }
-#pragma unroll
-            for (int j = 0; j < kPfUpdates; ++j) {
-                if (j < na16) upa[j * 64 + lane] = cur.v16[j];
-                else if (j < na16 + nb * nub) upb[(j - na16) * 64 + lane] = cur.v16[j];
-            }
-            if (ch + 1 < ch_end) prefetch_program(P, offsets, ch + 1, lane, nxt);
-        } else {
         const std::int64_t row_first = h[0];
         const std::int64_t opa_off = h[4], upa_off = h[6], opb_off = h[8], upb_off = h[10];
         if (lane < cnt) {
@@ -511,7 +426,6 @@ __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const 
                                     [&](int j, std::uint32_t v) { opb[j * 64 + lane] = v; });
         copy_batched<std::uint16_t>(nb * nub, [&](int j) { return P.upd_b[upb_off + j * 64 + lane]; },
                                     [&](int j, std::uint16_t v) { upb[j * 64 + lane] = v; });
-        }
         // 2. earlier chunks: gather (source indices, then values, each batch
         //    in flight together), then the lower entries in column order
         for (int t0 = 0; t0 < nsrc; t0 += 8) {
@@ -527,12 +441,6 @@ __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const 
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (t0 + u < nsrc) ga[(t0 + u) * 64 + lane] = idx[u] >= 0 ? v[u] : 0.0;
-        }
-        // chunk ch + 1's row values (their extents have arrived by now) load
-        // during this chunk's LDS work; no row of chunk ch + 1 is written
-        // before its own store
-        if constexpr (PF) {
-            if (ch + 1 < ch_end) prefetch_rows(Fc, P.kmax, nxt);
         }
         for (int j = 0; j < na; ++j) {
             const std::uint32_t d = opa[j * 64 + lane];
@@ -550,75 +458,24 @@ __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const 
             }
         }
         // 3. the chunk's own lower entries, one pivot row per step
-        if constexpr (NUB > 0) {
-            // At most NUB updates per op: an op's update words load with the
-            // op, and a step issues all its reads (pivot, the lower entry,
-            // row s's sources, its own targets) before its division, then
-            // its stores, with no branch per update (an update past the op's
-            // count reads a valid slot and writes the lane's trash slot).
-            // The targets are distinct slots of the lane's own row, neither
-            // the lower entry nor row s, so the values are those of the
-            // one-at-a-time order.
-            __shared__ double trash[64];
-            int jb = 0;
-            std::uint32_t d = nb > 0 ? opb[lane] : 0xffffffffu;
-            std::uint16_t w[NUB];
-#pragma unroll
-            for (int u = 0; u < NUB; ++u) w[u] = 0;
-            if (nb > 0 && nub > 0) {
-#pragma unroll
-                for (int u = 0; u < NUB; ++u) w[u] = upb[(u < nub ? u : nub - 1) * 64 + lane];
-            }
-            for (int s = 0; s < cnt; ++s) {
-                __builtin_amdgcn_wave_barrier();
-                if (d != 0xffffffffu && static_cast<int>(d & 255u) == s) {
-                    const int es = static_cast<int>((d >> 8) & 255u), ps = static_cast<int>((d >> 16) & 255u);
-                    const int nu = static_cast<int>(d >> 24);
-                    const double pivot = rv[ps * 64 + s];
-                    const double own = rv[es * 64 + lane];
-                    double src[NUB], tgt[NUB];
-                    double* dst[NUB];
-#pragma unroll
-                    for (int u = 0; u < NUB; ++u) {
-                        const bool on = u < nu;
-                        dst[u] = on ? &rv[(w[u] & 255) * 64 + lane] : &trash[lane];
-                        src[u] = rv[(on ? (w[u] >> 8) : 0) * 64 + s];
-                        tgt[u] = *dst[u];
-                    }
-                    if (__builtin_fabs(pivot) <= kTol) atomicExch(flag, static_cast<int>(flag_zero_pivot));
-                    const double lv = own / pivot;
-                    rv[es * 64 + lane] = lv;
-#pragma unroll
-                    for (int u = 0; u < NUB; ++u) *dst[u] = __builtin_fma(-lv, src[u], tgt[u]);
-                    ++jb;
-                    const int jn = jb < nb ? jb : nb - 1;
-                    d = jb < nb ? opb[jn * 64 + lane] : 0xffffffffu;
-                    if (nub > 0) {
-#pragma unroll
-                        for (int u = 0; u < NUB; ++u) w[u] = upb[(jn * nub + (u < nub ? u : nub - 1)) * 64 + lane];
-                    }
+        int jb = 0;
+        std::uint32_t d = nb > 0 ? opb[lane] : 0xffffffffu;
+        for (int s = 0; s < cnt; ++s) {
+            __builtin_amdgcn_wave_barrier();
+            if (d != 0xffffffffu && static_cast<int>(d & 255u) == s) {
+                const int es = static_cast<int>((d >> 8) & 255u), ps = static_cast<int>((d >> 16) & 255u);
+                const int nu = static_cast<int>(d >> 24);
+                const double pivot = rv[ps * 64 + s];
+                if (__builtin_fabs(pivot) <= kTol) atomicExch(flag, static_cast<int>(flag_zero_pivot));
+                const double lv = rv[es * 64 + lane] / pivot;
+                rv[es * 64 + lane] = lv;
+                for (int u = 0; u < nu; ++u) {
+                    const std::uint16_t w = upb[(jb * nub + u) * 64 + lane];
+                    const int ts = w & 255, qs = w >> 8;
+                    rv[ts * 64 + lane] = __builtin_fma(-lv, rv[qs * 64 + s], rv[ts * 64 + lane]);
                 }
-            }
-        } else {
-            int jb = 0;
-            std::uint32_t d = nb > 0 ? opb[lane] : 0xffffffffu;
-            for (int s = 0; s < cnt; ++s) {
-                __builtin_amdgcn_wave_barrier();
-                if (d != 0xffffffffu && static_cast<int>(d & 255u) == s) {
-                    const int es = static_cast<int>((d >> 8) & 255u), ps = static_cast<int>((d >> 16) & 255u);
-                    const int nu = static_cast<int>(d >> 24);
-                    const double pivot = rv[ps * 64 + s];
-                    if (__builtin_fabs(pivot) <= kTol) atomicExch(flag, static_cast<int>(flag_zero_pivot));
-                    const double lv = rv[es * 64 + lane] / pivot;
-                    rv[es * 64 + lane] = lv;
-                    for (int u = 0; u < nu; ++u) {
-                        const std::uint16_t w = upb[(jb * nub + u) * 64 + lane];
-                        const int ts = w & 255, qs = w >> 8;
-                        rv[ts * 64 + lane] = __builtin_fma(-lv, rv[qs * 64 + s], rv[ts * 64 + lane]);
-                    }
-                    ++jb;
-                    d = jb < nb ? opb[jb * 64 + lane] : 0xffffffffu;
-                }
+                ++jb;
+                d = jb < nb ? opb[jb * 64 + lane] : 0xffffffffu;
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -626,7 +483,6 @@ __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const 
         for (int q = 0; q < len; ++q) Fc[base + q] = rv[q * 64 + lane];
         __threadfence_block();
         __builtin_amdgcn_wave_barrier();
-        if constexpr (PF) cur = nxt;
     }
     const std::int64_t r0 = row0[b], n = nrows[b];
     for (std::int64_t i = lane; i < n; i += 64) {
@@ -635,6 +491,147 @@ __global__ __launch_bounds__(64) void k_ilu_factor_chunks(IluChunkArgs P, const 
         if (!(__builtin_isfinite(dg) && __builtin_fabs(dg) > kTol)) atomicExch(flag, static_cast<int>(flag_zero_pivot));
         inv[static_cast<std::int64_t>(c) * rows + row] = 1.0 / dg;
     }
+}
+
+// The same chunks with every operation as one record of LDS byte offsets
+// (IluChunkProgram::rec): its own entry, its pivot, and NU (source, target)
+// pairs.  A record is one load, its halves are the addresses, and a missing
+// pair or lane names a trash entry and a constant one, so an operation has no
+// branch, no count and no address arithmetic beyond unpacking.
+//
+// What bounds it: the chain of a chunk's 64 pivot rows, one after another on
+// one wave.  A step is its reads (~100 clk), a correctly rounded division
+// (~130), the update and the LDS write that the next step reads (65); the
+// rest is issue at 4 clk an instruction.  The step of the general kernel
+// unpacked bytes into addresses and tested a count per update: ~110
+// instructions, 1,940 us for 68 blocks of 4,096 vertices and 3 components
+// (64 chunks one after another); 1,048 us this way, ~600 clk a step.  Holding
+// the next chunk's rows, records and sources in 140 registers was slower
+// (1,327 us against 1,209 without any look-ahead); its header and row
+// extents alone are worth loading early.
+template<int NU> using IluRec = std::uint32_t __attribute__((ext_vector_type(1 + NU)));
+
+constexpr std::size_t ilu_rec_fixed(int kmax, int max_src) { return static_cast<std::size_t>(kmax + 2 + max_src) * 512; }
+
+inline std::size_t ilu_rec_lds(const IluChunkProgram& P)
+{
+    return ilu_rec_fixed(P.kmax, P.max_src) + static_cast<std::size_t>(P.max_a + P.max_b + 1) * 64 * 4 * (1 + P.nu);
+}
+
+// after_reads() runs once the operation's own reads are issued
+template<int NU, class F>
+__device__ inline void ilu_rec_op(unsigned char* lds, const IluRec<NU> r, double& lowest, F after_reads)
+{
+    auto at = [&](int k) -> double& {
+        const std::uint32_t o = k & 1 ? r[k >> 1] >> 16 : r[k >> 1] & 0xffffu;
+        return *reinterpret_cast<double*>(lds + o);
+    };
+    const double pivot = at(1);
+    const double own = at(0);
+    double src[NU], tgt[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        src[u] = at(2 + 2 * u);
+        tgt[u] = at(3 + 2 * u);
+    }
+    after_reads();
+    lowest = __builtin_fmin(lowest, __builtin_fabs(pivot));
+    const double lv = own / pivot;
+    // the targets are distinct slots of the lane's own row, neither its own
+    // lower entry nor the pivot row's: the order of these stores is free
+#pragma unroll
+    for (int u = 0; u < NU; ++u) at(3 + 2 * u) = __builtin_fma(-lv, src[u], tgt[u]);
+    at(0) = lv;
+}
+
+template<int NU>
+__global__ __launch_bounds__(64) void k_ilu_factor_rec(IluChunkArgs P, const std::int64_t* __restrict__ offsets,
+                                                       const std::int64_t* __restrict__ diag_pos, int bs,
+                                                       double* __restrict__ F, std::int64_t nnz, std::int64_t rows,
+                                                       double* __restrict__ inv, int* flag)
+{
+    extern __shared__ __align__(16) unsigned char lds_b[];
+    const int lane = static_cast<int>(threadIdx.x);
+    const int c = static_cast<int>(blockIdx.x) % bs;
+    const int b = static_cast<int>(blockIdx.x) / bs;
+    double* Fc = F + static_cast<std::int64_t>(c) * nnz;
+    double* invc = inv + static_cast<std::int64_t>(c) * rows;
+    double* rv = reinterpret_cast<double*>(lds_b);  // [kmax][64], trash [64], ones [64]
+    double* ga = rv + (P.kmax + 2) * 64;            // [max_src][64]
+    auto* recs = reinterpret_cast<IluRec<NU>*>(ga + P.max_src * 64);
+    rv[P.kmax * 64 + lane] = 0.0;
+    rv[(P.kmax + 1) * 64 + lane] = 1.0;
+    double lowest = 1.0;  // smallest |pivot| divided by
+    bool bad = false;
+    // a chunk's header and row extents, loaded one chunk ahead
+    struct { std::int64_t row, base, end, diag, src_off, rec_off; int cnt, nsrc, na, nb; } h;
+    auto header = [&](int ch) {
+        const std::int64_t* p = P.hdr + static_cast<std::int64_t>(ch) * 12;
+        h.cnt = static_cast<int>(p[1]);
+        h.src_off = p[2];
+        h.nsrc = static_cast<int>(p[3]);
+        h.rec_off = p[4] * 64;
+        h.na = static_cast<int>(p[5]);
+        h.nb = static_cast<int>(p[9]);
+        h.row = p[0] + (lane < h.cnt ? lane : h.cnt - 1);
+        h.base = offsets[h.row];
+        h.end = offsets[h.row + 1];
+        h.diag = diag_pos[h.row];
+    };
+    const int ch_begin = P.chunk_first[b], ch_end = P.chunk_first[b + 1];
+    if (ch_begin < ch_end) header(ch_begin);
+    for (int ch = ch_begin; ch < ch_end; ++ch) {
+        const int cnt = h.cnt, nsrc = h.nsrc, na = h.na, nb = h.nb;
+        const std::int64_t row = h.row, base = h.base, src_off = h.src_off, rec_off = h.rec_off;
+        const int len = lane < cnt ? static_cast<int>(h.end - base) : 0, dslot = static_cast<int>(h.diag - base);
+        const int lastq = len > 0 ? len - 1 : 0;
+        copy_batched<double>(P.kmax, [&](int q) { return Fc[base + (q < lastq ? q : lastq)]; },
+                             [&](int q, double v) { rv[q * 64 + lane] = q < len ? v : 0.0; });
+        const auto* rec = reinterpret_cast<const IluRec<NU>*>(P.rec) + rec_off + lane;
+        copy_batched<IluRec<NU>>(na + nb + 1, [&](int j) { return rec[j * 64]; },
+                                 [&](int j, IluRec<NU> r) { recs[j * 64 + lane] = r; });
+        for (int t0 = 0; t0 < nsrc; t0 += 8) {
+            std::int32_t idx[8];
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) idx[u] = P.src_a[src_off + (t0 + u < nsrc ? t0 + u : nsrc - 1) * 64 + lane];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = Fc[idx[u] >= 0 ? idx[u] : 0];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (t0 + u < nsrc) ga[(t0 + u) * 64 + lane] = v[u];
+        }
+        if (ch + 1 < ch_end) header(ch + 1);
+        __builtin_amdgcn_wave_barrier();
+        for (int j = 0; j < na; ++j) {
+            const IluRec<NU> r = recs[j * 64 + lane];
+            ilu_rec_op<NU>(lds_b, r, lowest, [] {});
+        }
+        // the chunk's own pivot rows; the record after a lane's last names
+        // row 63, which no later row of the chunk can depend on
+        const IluRec<NU>* next = recs + na * 64 + lane;
+        IluRec<NU> r = *next;
+        for (int s = 0; s < cnt - 1; ++s) {
+            __builtin_amdgcn_wave_barrier();
+            if (static_cast<int>((r[0] >> 19) & 63u) == s) {
+                next += 64;
+                IluRec<NU> following;
+                ilu_rec_op<NU>(lds_b, r, lowest, [&] { following = *next; });
+                r = following;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        // store; later chunks of this wave gather these values
+        for (int q = 0; q < len; ++q) Fc[base + q] = rv[q * 64 + lane];
+        if (lane < cnt) {
+            const double dg = rv[dslot * 64 + lane];
+            bad = bad || !(__builtin_isfinite(dg) && __builtin_fabs(dg) > kTol);
+            invc[row] = 1.0 / dg;
+        }
+        __threadfence_block();
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (bad || lowest <= kTol) atomicExch(flag, static_cast<int>(flag_zero_pivot));
 }
 
 enum class TriMode { ilu, ssor };
@@ -1948,15 +1945,63 @@ void build_ilu_chunks(owtk_precond pc, const std::vector<std::int64_t>& upd_ptr,
     P.max_nua = max_nua;
     P.max_b = max_b;
     P.max_nub = max_nub;
-    const std::size_t lds = ilu_chunk_lds(P);
-    if (lds > 64 * 1024) return;
+    // Records: at most 3 updates an operation (16 bytes; an ILU(0) factor of
+    // a triangulated grid) or 7 (32 bytes), values within 16-bit offsets and
+    // the whole within 64 KB of LDS; the general form otherwise.
+    const int updates = std::max(max_nua, max_nub);
+    P.nu = updates <= 3 ? 3 : updates <= 7 ? 7 : 0;
+    if (P.nu && (ilu_rec_fixed(kmax, max_src) > 64 * 1024 || ilu_rec_lds(P) > 64 * 1024)) P.nu = 0;
+    if (P.nu) {
+        std::vector<std::uint32_t> rec;
+        const int nu = P.nu, words = 1 + nu;
+        rec.reserve((op_a.size() + op_b.size() + static_cast<std::size_t>(chunks) * 64) * words);
+        const std::uint32_t trash = kmax * 512, one = (kmax + 1) * 512, gather = (kmax + 2) * 512;
+        for (std::int64_t ch = 0; ch < chunks; ++ch) {
+            std::int64_t* h = &hdr[ch * 12];
+            const std::int64_t opa = h[4], na = h[5], upa = h[6], nua = h[7], opb = h[8], nb = h[9], upb = h[10],
+                               nub = h[11];
+            h[4] = static_cast<std::int64_t>(rec.size()) / (64 * words);
+            const std::size_t at = rec.size();
+            rec.resize(at + static_cast<std::size_t>(na + nb + 1) * 64 * words);
+            for (std::int64_t j = 0; j <= na + nb; ++j)
+                for (std::uint32_t lane = 0; lane < 64; ++lane) {
+                    std::uint32_t* w = &rec[at + (j * 64 + lane) * words];
+                    // no operation: trash / one for earlier chunks, row 63 as
+                    // the pivot for this chunk's
+                    const bool earlier = j < na;
+                    const std::uint32_t d = earlier ? op_a[opa + j * 64 + lane]
+                                            : j < na + nb ? op_b[opb + (j - na) * 64 + lane] : 0xffffffffu;
+                    const std::uint32_t own_trash = trash + 8 * lane;
+                    w[0] = own_trash | (earlier ? one : one + 8 * 63) << 16;
+                    for (int u = 0; u < nu; ++u) w[1 + u] = one | own_trash << 16;
+                    if (d == 0xffffffffu) continue;
+                    const std::uint32_t step = d & 255u;
+                    const std::uint32_t own = (earlier ? d & 255u : (d >> 8) & 255u) * 512 + 8 * lane;
+                    const std::uint32_t pivot = earlier ? gather + ((d >> 8) & 255u) * 512 + 8 * lane
+                                                        : ((d >> 16) & 255u) * 512 + 8 * step;
+                    const int count = static_cast<int>(earlier ? (d >> 16) & 255u : d >> 24);
+                    w[0] = own | pivot << 16;
+                    for (int u = 0; u < count; ++u) {
+                        const std::uint32_t v = earlier ? upd_a[upa + (j * nua + u) * 64 + lane]
+                                                        : upd_b[upb + ((j - na) * nub + u) * 64 + lane];
+                        const std::uint32_t target = (v & 255u) * 512 + 8 * lane;
+                        const std::uint32_t source = earlier ? gather + (v >> 8) * 512 + 8 * lane
+                                                             : (v >> 8) * 512 + 8 * step;
+                        w[1 + u] = source | target << 16;
+                    }
+                }
+        }
+        upload(P.rec, rec);
+    } else {
+        if (ilu_chunk_lds(P) > 64 * 1024) return;
+        upload(P.op_a, op_a);
+        upload(P.op_b, op_b);
+        upload(P.upd_a, upd_a);
+        upload(P.upd_b, upd_b);
+    }
     upload(P.chunk_first, chunk_first);
     upload(P.hdr, hdr);
     upload(P.src_a, src_a);
-    upload(P.op_a, op_a);
-    upload(P.op_b, op_b);
-    upload(P.upd_a, upd_a);
-    upload(P.upd_b, upd_b);
     P.enabled = true;
 }
 
@@ -2076,18 +2121,18 @@ void ilu_numeric(owtk_precond pc)
     if (f.chunks.enabled) {
         const auto& P = f.chunks;
         const IluChunkArgs args{P.chunk_first.get(), P.hdr.get(), P.src_a.get(), P.op_a.get(), P.op_b.get(),
-                                P.upd_a.get(), P.upd_b.get(), P.kmax, P.max_src, P.max_a, P.max_nua, P.max_b,
-                                P.max_nub};
-        // ILU(0) on a triangulated grid has at most 3 updates per op
+                                P.upd_a.get(), P.upd_b.get(), P.rec.get(), P.kmax, P.max_src, P.max_a, P.max_nua,
+                                P.max_b, P.max_nub};
         auto launch = [&](auto kernel) {
-            kernel<<<groups, 64, ilu_chunk_lds(P), st>>>(args, f.offsets.get(), f.diag_pos.get(), t.row0.get(),
-                                                         t.nrows.get(), bs, f.values.get(), f.nnz, t.rows,
-                                                         t.dval64.get(), pc->flag.get());
+            kernel<<<groups, 64, ilu_rec_lds(P), st>>>(args, f.offsets.get(), f.diag_pos.get(), bs, f.values.get(),
+                                                       f.nnz, t.rows, t.dval64.get(), pc->flag.get());
         };
-        const bool pf = ilu_chunks_prefetchable(P);
-        if (P.max_nub <= 3) pf ? launch(k_ilu_factor_chunks<3, true>) : launch(k_ilu_factor_chunks<3, false>);
-        else if (P.max_nub <= 6) pf ? launch(k_ilu_factor_chunks<6, true>) : launch(k_ilu_factor_chunks<6, false>);
-        else pf ? launch(k_ilu_factor_chunks<0, true>) : launch(k_ilu_factor_chunks<0, false>);
+        if (P.nu == 3) launch(k_ilu_factor_rec<3>);
+        else if (P.nu == 7) launch(k_ilu_factor_rec<7>);
+        else
+            k_ilu_factor_chunks<<<groups, 64, ilu_chunk_lds(P), st>>>(args, f.offsets.get(), f.diag_pos.get(),
+                                                                      t.row0.get(), t.nrows.get(), bs, f.values.get(),
+                                                                      f.nnz, t.rows, t.dval64.get(), pc->flag.get());
     } else {
         k_ilu_factor<<<groups, 64, 0, st>>>(tri_args(t), t.frow_lvl.get(), f.offsets.get(), f.diag_pos.get(),
                                             f.upd_ptr.get(), f.upd_target.get(), f.upd_upper.get(), f.columns.get(),

@@ -70,14 +70,20 @@ struct TriSchedule {
 //   updB  [nB*nuB][64] target slot | source slot (in the pivot row) << 8
 // (slots are positions in a row's factor entries; 0xffffffff pads opA/opB)
 // hdr per chunk: row of lane 0, rows, and offset and count of each array.
+// With at most nu = 3 or 7 updates an operation the four arrays are replaced
+// by rec [nA + nB + 1][64], 2 + 2 nu halves an operation (hdr[4]: its first
+// row): LDS byte offsets of own entry, pivot, and (source, target) pairs, in
+// the layout rows [kmax][64] | trash [64] | ones [64] | srcA [nsrc][64].
 struct IluChunkProgram {
     bool enabled = false;
+    int nu = 0;  // updates a record holds; 0: the general form
     int kmax = 0, max_src = 0, max_a = 0, max_nua = 0, max_b = 0, max_nub = 0;
     DeviceArray<std::int32_t> chunk_first;  // per block (blocks + 1)
     DeviceArray<std::int64_t> hdr;          // per chunk: 12 values (see k_ilu_factor_chunks)
     DeviceArray<std::int32_t> src_a;
     DeviceArray<std::uint32_t> op_a, op_b;
     DeviceArray<std::uint16_t> upd_a, upd_b;
+    DeviceArray<std::uint32_t> rec;
 };
 
 struct IluFactor {

@@ -249,3 +249,40 @@ def test_solvers_around_the_fused_grid(ctx, nx, ny, block):
         if solve is owtk.bicgstab:
             assert abs(res["iterations"] - ro["iterations"]) <= 1
         assert np.max(np.abs(x.download() - ref)) <= 4e-7 * np.linalg.norm(s.rhs)
+
+
+@pytest.mark.parametrize("fill", [0, 1, 3])
+@pytest.mark.parametrize("n,block,low,high,nodes", [(1, 1, 0, 0, 0), (63, 3, 1, 4, 0), (64, 1, 2, 6, 0),
+                                                    (65, 2, 2, 6, 0), (200, 1, 0, 12, 0), (391, 2, 1, 5, 130),
+                                                    (320, 1, 30, 40, 64)])
+def test_ilu_factor_forms(ctx, n, block, low, high, nodes, fill):
+    """Every form of the chunked factorization (records of 3 and 7 updates, the general one) and the kernel behind it
+    (long rows), with chunks and blocks that end early: the operations are the oracle's in its order, so the factors
+    are its bits."""
+    offsets, columns, values = random_dominant(np.random.default_rng(n + fill), n, block, low, high)
+    m = owtk.Matrix.csr(ctx, n, 0, block, offsets, columns, values)
+    pc = owtk.Preconditioner(m, owtk.PC_ILU, fill_level=fill, block_nodes=nodes)
+    opc = orc.OPreconditioner(orc.OMatrix.csr(n, 0, block, offsets, columns, values), 3, fill_level=fill,
+                              block_nodes=nodes)
+    for got, ref in zip(pc.ilu_factors(), opc.ilu_factors()):
+        assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("row", [0, 63, 64, 127, 199])
+def test_ilu_small_pivot_anywhere(ctx, row):
+    """A vanishing pivot in a chunk's first or last row, in an earlier chunk, or in the last row of all is reported,
+    and a factorization after it succeeds."""
+    n = 200
+    d, e = np.full(n, 4.0), np.full(2 * (n - 1), -1.0)
+    offsets = np.concatenate([[0], np.cumsum([1 + (1 if i in (0, n - 1) else 2) - 1 for i in range(n)])]).astype(np.int32)
+    columns = np.concatenate([[j for j in (i - 1, i + 1) if 0 <= j < n] for i in range(n)]).astype(np.int32)
+    m = owtk.Matrix.split(ctx, n, 0, 1, offsets, columns, d, e)
+    pc = owtk.Preconditioner(m, owtk.PC_ILU)
+    bad, cut = d.copy(), e.copy()
+    bad[row] = 0.0
+    cut[offsets[row]:offsets[row + 1]][columns[offsets[row]:offsets[row + 1]] < row] = 0.0
+    m.update_values(bad, cut)
+    with pytest.raises(owtk.ZeroPivotError):
+        pc.update_values()
+    m.update_values(d, e)
+    pc.update_values()
