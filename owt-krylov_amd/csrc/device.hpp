@@ -169,9 +169,10 @@ struct ReduceScratch {
 // 63 / 55 at 64,800 (254).
 constexpr unsigned int kFuseBlocks = 128;
 
-// Cross-block reductions run in two launches.  The streaming kernel calls
-// store_partials: each block reduces its values and writes one partial per
-// value.  A one-block finisher (k_finish, launched right after on the same
+// Cross-block reductions of more than kFuseBlocks blocks run in two launches
+// (those of fewer end in the kernel itself, reduce_end).  The streaming kernel
+// calls store_partials: each block reduces its values and writes one partial
+// per value.  A one-block finisher (k_finish, launched right after on the same
 // stream) then sums the partials in a fixed order, so results are
 // deterministic for a fixed grid, and runs the caller's finalizer with all of
 // its threads (totals in LDS, identical on every thread); single-thread state
@@ -189,7 +190,7 @@ __device__ inline void store_partials(double (&v)[K], std::uint64_t max_mask, Re
 }
 
 // Sums the partials of nblocks blocks in a fixed order; totals (LDS) on every
-// thread.
+// thread (the last block of a kernel that ends its own reduction).
 template<int K>
 __device__ inline void finish_totals(double (&totals)[K], unsigned int nblocks, std::uint64_t max_mask,
                                      ReduceScratch scratch)
@@ -275,14 +276,60 @@ __device__ inline void reduce_end(double (&v)[K], std::uint64_t max_mask, Reduce
     fin(static_cast<const double*>(totals));
 }
 
+// One 16-wave block.  What bounds it is latency: the partials come from other
+// XCDs, and nothing else runs.  The waves are dealt out to the values (16 / P
+// waves each, P the power of two from K; in turns for K > 16), so a wave
+// combines one value across its lanes instead of each wave all of them, and
+// 16 loads are in flight per lane.  Three values of 8,192 blocks: 7.8 us, and
+// 10 with four waves that each combined all values; BiCGSTAB + ILU(0) at 2M
+// vertices, four finishers an iteration: 25.7 -> 25.4 ms a solve.
+constexpr int kFinishThreads = 1024;
+
 template<int K, class Fin>
-__global__ __launch_bounds__(256) void k_finish(Fin fin, unsigned int nblocks, std::uint64_t max_mask,
-                                                ReduceScratch scratch, const int* stop, const int* need)
+__global__ __launch_bounds__(kFinishThreads) void k_finish(Fin fin, unsigned int nblocks, std::uint64_t max_mask,
+                                                           ReduceScratch scratch, const int* stop, const int* need)
 {
     if (stop != nullptr && *stop != 0) return;
     if (need != nullptr && *need == 0) return;
-    __shared__ double totals[K > 0 ? K : 1];
-    finish_totals<K>(totals, nblocks, max_mask, scratch);
+    constexpr int kWaves = kFinishThreads / kWave;
+    constexpr int P = K <= 1 ? 1 : K <= 2 ? 2 : K <= 4 ? 4 : K <= 8 ? 8 : 16;
+    constexpr int S = kWaves / P;  // waves per value
+    constexpr int U = 16;
+    __shared__ double parts[K][S];
+    __shared__ double totals[K];
+    const int wave = threadIdx.x / kWave;
+    const unsigned int lane = threadIdx.x & (kWave - 1);
+    const unsigned int first = (wave % S) * kWave + lane;
+    for (int k = wave / S; k < K; k += P) {
+        const double* row = scratch.partials + k * scratch.stride;
+        auto sum = [&]<Combine C>() {
+            double acc = 0.0;
+            for (unsigned int base = first; base < nblocks; base += U * S * kWave) {
+                double p[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const unsigned int b = base + u * S * kWave;
+                    p[u] = b < nblocks ? row[b] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc = combine<C>(acc, p[u]);
+            }
+            return wave_combine<C>(acc);
+        };
+        const double v = ((max_mask >> k) & 1) ? sum.template operator()<Combine::max>()
+                                               : sum.template operator()<Combine::sum>();
+        if (lane == 0) parts[k][wave % S] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < K) {
+        const bool is_max = (max_mask >> threadIdx.x) & 1;
+        double acc = parts[threadIdx.x][0];
+        for (int w = 1; w < S; ++w)
+            acc = is_max ? combine<Combine::max>(acc, parts[threadIdx.x][w])
+                         : combine<Combine::sum>(acc, parts[threadIdx.x][w]);
+        totals[threadIdx.x] = acc;
+    }
+    __syncthreads();
     fin(static_cast<const double*>(totals));
 }
 
@@ -293,7 +340,7 @@ inline void launch_finish(hipStream_t st, const Fin& fin, unsigned int nblocks, 
                           ReduceScratch scratch, const int* stop, const int* need = nullptr)
 {
     if (scratch.ticket != nullptr) return;
-    k_finish<K, Fin><<<1, kBlock, 0, st>>>(fin, nblocks, max_mask, scratch, stop, need);
+    k_finish<K, Fin><<<1, kFinishThreads, 0, st>>>(fin, nblocks, max_mask, scratch, stop, need);
 }
 
 // ------------------------------------------- double-double (compensated) --
@@ -427,17 +474,17 @@ inline void launch_finish_dd(hipStream_t st, const Fin& fin, unsigned int nblock
     k_finish_dd<K, Fin><<<1, kBlock, 0, st>>>(fin, nblocks, max_mask, scratch, stop);
 }
 
-// Sum over the block, result on every thread.
+// Sum over the block (any number of waves), result on every thread.
 __device__ inline double block_sum_all(double v)
 {
-    __shared__ double lds[kWavesPerBlock];
+    __shared__ double lds[kFinishThreads / kWave];
     __shared__ double total;
     v = wave_combine<Combine::sum>(v);
     if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double acc = lds[0];
-        for (int w = 1; w < kWavesPerBlock; ++w) acc += lds[w];
+        for (unsigned int w = 1; w < blockDim.x / kWave; ++w) acc += lds[w];
         total = acc;
     }
     __syncthreads();

@@ -229,6 +229,23 @@ def test_reductions_around_the_fused_grid(ctx, n):
     assert np.isinf(ctx.norm(ctx.upload(np.where(np.arange(n) == n - 1, -np.inf, a))))
 
 
+@pytest.mark.parametrize("k", [0, 1, 2, 3, 4, 8, 9, 15, 16, 30, 31, 32, 62])
+def test_finisher_widths(ctx, k):
+    """The finisher for every number of values and more partials (1,661 blocks) than one pass of a wave takes; a NaN
+    in one vector reaches only that vector's value.  Bounds as in the test above."""
+    n = 1_700_001
+    rng = np.random.default_rng(k)
+    host = [rng.uniform(-1, 1, n) for _ in range(3)]
+    host[1][n // 3] = np.nan
+    vectors = [ctx.upload(v) for v in host]
+    w = rng.uniform(-1, 1, n)
+    got = ctx.multidot([vectors[i % 3] for i in range(k)], ctx.upload(w))
+    exact = [np.dot(v, w) for v in host]
+    for i in range(k):
+        assert np.isnan(got[i]) if i % 3 == 1 else abs(got[i] - exact[i % 3]) <= 1e-14 * n
+    assert abs(got[k] - np.dot(w, w)) <= 1e-14 * n
+
+
 @pytest.mark.parametrize("nx,ny,block", [(5, 3, 1), (128, 128, 2), (128, 256, 1), (130, 255, 3), (130, 130, 5)])
 def test_solvers_around_the_fused_grid(ctx, nx, ny, block):
     """BiCGSTAB, its pipelined and communication-hiding forms on grids below, at and above 128 SpMV blocks (256 rows)
