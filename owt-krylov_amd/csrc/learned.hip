@@ -50,6 +50,13 @@ constexpr int W = kGnnWidth;
 constexpr int kReduceGrid = 512;     // blocks of the gradient reductions: two per CU
 constexpr int kMaxOuterOutputs = kGnnMaxOutputs * 2 * W + kGnnMaxOutputs;
 
+// the matrix-core kernels' grid: four 32-vertex tiles a block, and past 4,096
+// blocks a grid-stride loop
+unsigned int tile_grid(std::int64_t n)
+{
+    return static_cast<unsigned int>(std::max<std::int64_t>(1, std::min<std::int64_t>((n + 127) / 128, 4096)));
+}
+
 unsigned int rows_grid(std::int64_t n)
 {
     const std::int64_t g = (n + kBlock - 1) / kBlock;
@@ -178,36 +185,6 @@ __device__ inline void load_weights(float* dst, const std::uint16_t* __restrict_
     for (int t = threadIdx.x; t < count; t += blockDim.x) dst[t] = dev::bf16_to_float(p16[off + t]);
 }
 
-__global__ __launch_bounds__(256) void k_gnn_encode(std::int64_t n, int f0, const float* __restrict__ x,
-                                                    const std::uint16_t* __restrict__ p16, std::int64_t off_w,
-                                                    std::int64_t off_b, float* __restrict__ h)
-{
-    __shared__ float sw[W * kGnnMaxFeatures];
-    __shared__ float sb[W];
-    load_weights(sw, p16, off_w, W * f0);
-    load_weights(sb, p16, off_b, W);
-    __syncthreads();
-    const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float xi[kGnnMaxFeatures];
-#pragma unroll
-    for (int f = 0; f < kGnnMaxFeatures; ++f) xi[f] = f < f0 ? x[i * f0 + f] : 0.f;
-    float4* out = reinterpret_cast<float4*>(h + i * W);
-    for (int q = 0; q < W / 4; ++q) {
-        float r[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int o = 4 * q + j;
-            float acc = sb[o];
-#pragma unroll
-            for (int f = 0; f < kGnnMaxFeatures; ++f)
-                if (f < f0) acc = __builtin_fmaf(sw[o * f0 + f], xi[f], acc);
-            r[j] = tanhf(acc);
-        }
-        out[q] = make_float4(r[0], r[1], r[2], r[3]);
-    }
-}
-
 __device__ inline void load_row(float (&v)[W], const float* __restrict__ p)
 {
     const float4* q = reinterpret_cast<const float4*>(p);
@@ -228,63 +205,12 @@ __device__ inline void store_row(float* __restrict__ p, const float (&v)[W])
     for (int j = 0; j < W / 4; ++j) q[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
 }
 
-// One message-passing layer.  agg_out (training) keeps the aggregate.
-__global__ __launch_bounds__(256) void k_gnn_layer(std::int64_t n, const std::int32_t* __restrict__ offsets,
-                                                   const std::int32_t* __restrict__ cols, const float* __restrict__ w,
-                                                   const float* __restrict__ hin,
-                                                   const std::uint16_t* __restrict__ p16, std::int64_t off_ws,
-                                                   std::int64_t off_wn, std::int64_t off_b,
-                                                   float* __restrict__ hout, float* __restrict__ agg_out)
-{
-    __shared__ float sws[W * W];
-    __shared__ float swn[W * W];
-    __shared__ float sb[W];
-    load_weights(sws, p16, off_ws, W * W);
-    load_weights(swn, p16, off_wn, W * W);
-    load_weights(sb, p16, off_b, W);
-    __syncthreads();
-    const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float a[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) a[k] = 0.f;
-    for (std::int32_t e = offsets[i]; e < offsets[i + 1]; ++e) {
-        const float we = w[e];
-        const float4* hj = reinterpret_cast<const float4*>(hin + static_cast<std::int64_t>(cols[e]) * W);
-#pragma unroll
-        for (int q = 0; q < W / 4; ++q) {
-            const float4 t = hj[q];
-            a[4 * q] = __builtin_fmaf(we, t.x, a[4 * q]);
-            a[4 * q + 1] = __builtin_fmaf(we, t.y, a[4 * q + 1]);
-            a[4 * q + 2] = __builtin_fmaf(we, t.z, a[4 * q + 2]);
-            a[4 * q + 3] = __builtin_fmaf(we, t.w, a[4 * q + 3]);
-        }
-    }
-    if (agg_out) store_row(agg_out + i * W, a);
-    float h[W];
-    load_row(h, hin + i * W);
-    float4* out = reinterpret_cast<float4*>(hout + i * W);
-    for (int q = 0; q < W / 4; ++q) {
-        float r[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int o = 4 * q + j;
-            float acc = sb[o];
-#pragma unroll
-            for (int k = 0; k < W; ++k) acc = __builtin_fmaf(sws[o * W + k], h[k], acc);
-#pragma unroll
-            for (int k = 0; k < W; ++k) acc = __builtin_fmaf(swn[o * W + k], a[k], acc);
-            r[j] = tanhf(acc);
-        }
-        out[q] = make_float4(r[0], r[1], r[2], r[3]);
-    }
-}
-
 using f32x16 = float __attribute__((ext_vector_type(16)));
 constexpr int kMfmaEdges = 2;  // edges gathered per pass of the aggregation
 
-// One message-passing layer over a SELL-layout graph on the matrix cores
-// (inference).  A wave computes a tile of 32 vertices:
+// One message-passing layer on the matrix cores, over a SELL-layout graph
+// (inference) or a CSR one, keeping the aggregate if agg_out is given
+// (training).  A wave computes a tile of 32 vertices:
 //     out = tanh([h_v | a_v] Wcat^T + b),  Wcat = [Ws | Wn] (32 x 64),
 // as 32 steps of v_mfma_f32_32x32x2_f32.  Lane l supplies row v = l % 32 of
 // the 32 x 2 A slice and column o = l % 32 of the 2 x 32 B slice; the two
@@ -292,17 +218,20 @@ constexpr int kMfmaEdges = 2;  // edges gathered per pass of the aggregation
 //     t < 16: self feature 16 h + t,    t >= 16: aggregate 16 h + t - 16,
 // so each lane gathers and sums only its half of its vertex's features, and
 // its 32 weights stay in registers for the whole launch.  The aggregate is
-// summed in edge order exactly as k_gnn_layer; the products are accumulated
-// in the matrix cores' order.  D: lane l holds column o, rows
+// summed in edge order; the products are accumulated in the matrix cores'
+// order.  Over CSR, 131,072 vertices: 34 us; a thread per vertex
+// with the weights in LDS (an LDS read per FMA) took 39.  D: lane l holds column o, rows
 // 8 (r / 4) + 4 h + r % 4 of register r.
-// The input encoding on the matrix cores (inference): a wave computes a
-// tile of 32 vertices, h = tanh(x W_in^T + b_in) with x feature-major
-// (x[f n + v], as k_gnn_features_sell writes it), the f0 <= 16 features
+// The input encoding on the matrix cores: a wave computes a tile of 32
+// vertices, h = tanh(x W_in^T + b_in) with feature f of vertex v at
+// x[f sf + v sv] (feature-major from k_gnn_features_sell, vertex-major from
+// k_gnn_features), the f0 <= 16 features
 // padded with zeros to 16 and split over the half-waves (step t takes
 // feature t + 8 h), 8 steps of v_mfma_f32_32x32x2_f32; output layout as in
 // k_gnn_layer_mfma, so each store instruction writes two whole rows of h.
 static_assert(kGnnMaxFeatures <= 16, "the matrix-core encoding takes at most 16 features");
 __global__ __launch_bounds__(256) void k_gnn_encode_mfma(std::int64_t n, int f0, const float* __restrict__ x,
+                                                         std::int64_t sf, std::int64_t sv,
                                                          const std::uint16_t* __restrict__ p16, std::int64_t off_w,
                                                          std::int64_t off_b, float* __restrict__ h)
 {
@@ -325,7 +254,7 @@ __global__ __launch_bounds__(256) void k_gnn_encode_mfma(std::int64_t n, int f0,
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int f = 8 * half + t;
-            av[t] = valid && f < f0 ? x[f * n + v] : 0.f;  // feature-major
+            av[t] = valid && f < f0 ? x[f * sf + v * sv] : 0.f;
         }
         f32x16 acc;
 #pragma unroll
@@ -342,13 +271,15 @@ __global__ __launch_bounds__(256) void k_gnn_encode_mfma(std::int64_t n, int f0,
 
 // Three waves per SIMD (at most 168 registers): a tile waits on its gathers,
 // and 2 edges per pass with 3 waves measured faster than 4 edges with 2.
-__global__ __launch_bounds__(256, 3) void k_gnn_layer_mfma(std::int64_t n, const std::int32_t* __restrict__ slice_ptr,
+// rows: slice starts (SELL, with row_len) or row offsets.
+template<bool SELL>
+__global__ __launch_bounds__(256, 3) void k_gnn_layer_mfma(std::int64_t n, const std::int32_t* __restrict__ rows,
                                                         const std::int32_t* __restrict__ row_len,
                                                         const std::int32_t* __restrict__ cols,
                                                         const float* __restrict__ w, const float* __restrict__ hin,
                                                         const std::uint16_t* __restrict__ p16, std::int64_t off_ws,
                                                         std::int64_t off_wn, std::int64_t off_b,
-                                                        float* __restrict__ hout)
+                                                        float* __restrict__ hout, float* __restrict__ agg_out)
 {
     const int l = static_cast<int>(threadIdx.x & 63);
     const int o = l & 31, half = l >> 5;
@@ -380,9 +311,12 @@ __global__ __launch_bounds__(256, 3) void k_gnn_layer_mfma(std::int64_t n, const
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j) av[16 + j] = 0.f;
-        const std::int64_t base = slice_ptr[vc >> 6];
-        const int width = static_cast<int>((slice_ptr[(vc >> 6) + 1] - base) >> 6);
-        const int len = valid ? row_len[vc] : 0;
+        const std::int64_t at = SELL ? vc >> 6 : vc;
+        const std::int64_t base = rows[at];
+        const int width = static_cast<int>((rows[at + 1] - base) >> (SELL ? 6 : 0));
+        int len = 0;
+        if constexpr (SELL) len = valid ? row_len[vc] : 0;
+        else len = valid ? width : 0;
         // kMfmaEdges edges per pass, every load issued before the sums: a
         // slot past the slice's width is clamped to its last run (in
         // bounds) and an edge past the row's length is dropped by a select
@@ -392,7 +326,7 @@ __global__ __launch_bounds__(256, 3) void k_gnn_layer_mfma(std::int64_t n, const
 #pragma unroll
             for (int u = 0; u < kMfmaEdges; ++u) {
                 const int kk = k0 + u < width ? k0 + u : width - 1;
-                const std::int64_t slot = base + 64 * kk + (vc & 63);
+                const std::int64_t slot = SELL ? base + 64 * kk + (vc & 63) : base + kk;
                 ck[u] = cols[slot];
                 wk[u] = w[slot];
             }
@@ -420,6 +354,12 @@ __global__ __launch_bounds__(256, 3) void k_gnn_layer_mfma(std::int64_t n, const
                     a[3] = on ? f3 : a[3];
                 }
             }
+        }
+        if (!SELL && agg_out != nullptr && valid) {
+            float4* out = reinterpret_cast<float4*>(agg_out + v * W + 16 * half);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                out[q] = make_float4(av[16 + 4 * q], av[17 + 4 * q], av[18 + 4 * q], av[19 + 4 * q]);
         }
         f32x16 acc;
 #pragma unroll
@@ -488,70 +428,114 @@ __global__ __launch_bounds__(256) void k_gnn_decode_bwd(std::int64_t n, int b, i
     store_row(dh + i * W, acc);
 }
 
-// du = dh (1 - h^2); s = W_s^T du (written to dprev); v = W_n^T du.
+// du = dh (1 - h^2); s = W_s^T du (written to dprev); v = W_n^T du, on the
+// matrix cores: a wave takes a tile of 32 vertices and the 32 x 64 matrix
+// [Ws | Wn] stays in registers, as in k_gnn_layer_mfma (lane l supplies
+// components 16 h .. 16 h + 15 of vertex l % 32).  Bound by its 84 MB of
+// vectors at 131,072 vertices: 20 us; a thread per vertex with the
+// weights in LDS took 29.
 __global__ __launch_bounds__(256) void k_gnn_layer_bwd(std::int64_t n, const float* __restrict__ h,
                                                        const float* __restrict__ dh,
                                                        const std::uint16_t* __restrict__ p16, std::int64_t off_ws,
                                                        std::int64_t off_wn, float* __restrict__ du_out,
                                                        float* __restrict__ dprev, float* __restrict__ v_out)
 {
-    __shared__ float sws[W * W];
-    __shared__ float swn[W * W];
-    load_weights(sws, p16, off_ws, W * W);
-    load_weights(swn, p16, off_wn, W * W);
-    __syncthreads();
-    const std::int64_t i = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float hv[W], du[W];
-    load_row(hv, h + i * W);
-    load_row(du, dh + i * W);
+    const int l = static_cast<int>(threadIdx.x & 63);
+    const int m = l & 31, half = l >> 5;
+    float ws[16], wn[16];
 #pragma unroll
-    for (int k = 0; k < W; ++k) du[k] *= 1.0f - hv[k] * hv[k];
-    store_row(du_out + i * W, du);
-    float s[W], v[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-        s[k] = 0.f;
-        v[k] = 0.f;
+    for (int t = 0; t < 16; ++t) {
+        ws[t] = dev::bf16_to_float(p16[off_ws + (16 * half + t) * W + m]);
+        wn[t] = dev::bf16_to_float(p16[off_wn + (16 * half + t) * W + m]);
     }
+    const std::int64_t tiles = (n + 31) >> 5;
+    const std::int64_t waves = static_cast<std::int64_t>(gridDim.x) * (blockDim.x >> 6);
+    for (std::int64_t tile = static_cast<std::int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+         tile < tiles; tile += waves) {
+        const std::int64_t i = tile * 32 + m;
+        const std::int64_t at = (i < n ? i : n - 1) * W + 16 * half;
+        const float4* hq = reinterpret_cast<const float4*>(h + at);
+        const float4* dq = reinterpret_cast<const float4*>(dh + at);
+        float4 hv[4], dv[4];
 #pragma unroll
-    for (int o = 0; o < W; ++o) {
-        const float d = du[o];
+        for (int q = 0; q < 4; ++q) {
+            hv[q] = hq[q];
+            dv[q] = dq[q];
+        }
+        float du[16];
 #pragma unroll
-        for (int k = 0; k < W; ++k) {
-            s[k] = __builtin_fmaf(sws[o * W + k], d, s[k]);
-            v[k] = __builtin_fmaf(swn[o * W + k], d, v[k]);
+        for (int q = 0; q < 4; ++q) {
+            du[4 * q] = dv[q].x * (1.0f - hv[q].x * hv[q].x);
+            du[4 * q + 1] = dv[q].y * (1.0f - hv[q].y * hv[q].y);
+            du[4 * q + 2] = dv[q].z * (1.0f - hv[q].z * hv[q].z);
+            du[4 * q + 3] = dv[q].w * (1.0f - hv[q].w * hv[q].w);
+        }
+        if (i < n) {
+            float4* out = reinterpret_cast<float4*>(du_out + at);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out[q] = make_float4(du[4 * q], du[4 * q + 1], du[4 * q + 2], du[4 * q + 3]);
+        }
+        f32x16 s, v;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s[r] = 0.f;
+            v[r] = 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(du[t], ws[t], s, 0, 0, 0);
+            v = __builtin_amdgcn_mfma_f32_32x32x2f32(du[t], wn[t], v, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const std::int64_t vv = tile * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+            if (vv < n) {
+                dprev[vv * W + m] = s[r];
+                v_out[vv * W + m] = v[r];
+            }
         }
     }
-    store_row(dprev + i * W, s);
-    store_row(v_out + i * W, v);
 }
 
 // dprev_j += sum_(e in row j) w_mirror(e) v_col(e): the transposed aggregation
 // (pattern symmetric, weight of entry (col, j) found through the mirror).
+// Eight threads per vertex, four components each, so a neighbour's row is one
+// 128-byte access and four edges are in flight: 17 us at 131,072 vertices
+// (a thread per vertex, one edge at a time: 22.7).
 __global__ __launch_bounds__(256) void k_gnn_agg_t(std::int64_t n, const std::int32_t* __restrict__ offsets,
                                                    const std::int32_t* __restrict__ cols,
                                                    const std::int32_t* __restrict__ mirror,
                                                    const float* __restrict__ w, const float* __restrict__ v,
                                                    float* __restrict__ dprev)
 {
-    const std::int64_t j = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    constexpr int U = 4;
+    const std::int64_t t0 = static_cast<std::int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const std::int64_t j = t0 >> 3;
     if (j >= n) return;
-    float acc[W];
-    load_row(acc, dprev + j * W);
-    for (std::int32_t e = offsets[j]; e < offsets[j + 1]; ++e) {
-        const float we = w[mirror[e]];
-        const float4* vi = reinterpret_cast<const float4*>(v + static_cast<std::int64_t>(cols[e]) * W);
+    const int q = static_cast<int>(t0 & 7);
+    float4* out = reinterpret_cast<float4*>(dprev + j * W) + q;
+    float4 acc = *out;
+    const std::int32_t begin = offsets[j], end = offsets[j + 1];
+    for (std::int32_t e0 = begin; e0 < end; e0 += U) {
+        float we[U];
+        float4 x[U];
 #pragma unroll
-        for (int q = 0; q < W / 4; ++q) {
-            const float4 t = vi[q];
-            acc[4 * q] = __builtin_fmaf(we, t.x, acc[4 * q]);
-            acc[4 * q + 1] = __builtin_fmaf(we, t.y, acc[4 * q + 1]);
-            acc[4 * q + 2] = __builtin_fmaf(we, t.z, acc[4 * q + 2]);
-            acc[4 * q + 3] = __builtin_fmaf(we, t.w, acc[4 * q + 3]);
+        for (int u = 0; u < U; ++u) {
+            const std::int32_t e = e0 + u < end ? e0 + u : end - 1;
+            we[u] = w[mirror[e]];
+            x[u] = reinterpret_cast<const float4*>(v + static_cast<std::int64_t>(cols[e]) * W)[q];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e0 + u < end) {
+                acc.x = __builtin_fmaf(we[u], x[u].x, acc.x);
+                acc.y = __builtin_fmaf(we[u], x[u].y, acc.y);
+                acc.z = __builtin_fmaf(we[u], x[u].z, acc.z);
+                acc.w = __builtin_fmaf(we[u], x[u].w, acc.w);
+            }
         }
     }
-    store_row(dprev + j * W, acc);
+    *out = acc;
 }
 
 // Weight gradients on the matrix cores: over all vertices i,
@@ -1187,26 +1171,22 @@ void forward(owtk_gnn model, const GnnGraph& g, float* h, float* agg, float* gam
     if (g.sell && train) throw std::logic_error("training runs over the CSR graph");
     // the matrix-core kernels keep each wave's weights in registers across a
     // grid-stride loop over the 32-vertex tiles
-    const std::int64_t tiles = (n + 31) / 32;
-    const unsigned int mgrid = static_cast<unsigned int>(std::max<std::int64_t>(1, std::min<std::int64_t>((tiles + 3) / 4, 4096)));
-    if (g.sell)
-        k_gnn_encode_mfma<<<mgrid, kBlock, 0, st>>>(n, model->f0, g.x.get(), p16, model->off_w_in, model->off_b_in, h);
-    else
-        k_gnn_encode<<<grid, kBlock, 0, st>>>(n, model->f0, g.x.get(), p16, model->off_w_in, model->off_b_in, h);
+    const unsigned int mgrid = tile_grid(n);
+    k_gnn_encode_mfma<<<mgrid, kBlock, 0, st>>>(n, model->f0, g.x.get(), g.sell ? n : 1, g.sell ? 1 : model->f0, p16,
+                                                model->off_w_in, model->off_b_in, h);
     OWTK_LAUNCH_CHECK();
     float* cur = h;
     for (int l = 0; l < kGnnLayers; ++l) {
         float* next = train ? h + static_cast<std::int64_t>(l + 1) * n * W : h + ((l + 1) & 1) * n * W;
-        if (g.sell) {
-            k_gnn_layer_mfma<<<mgrid, kBlock, 0, st>>>(n, g.slice_ptr, g.row_len, g.slot_cols, g.slot_w.get(), cur, p16,
-                                                       model->off_ws[l], model->off_wn[l], model->off_b[l], next);
-            OWTK_LAUNCH_CHECK();
-            cur = next;
-            continue;
-        }
-        k_gnn_layer<<<grid, kBlock, 0, st>>>(n, g.offsets.get(), g.cols.get(), g.w.get(), cur, p16, model->off_ws[l],
-                                             model->off_wn[l], model->off_b[l], next,
-                                             train ? agg + static_cast<std::int64_t>(l) * n * W : nullptr);
+        if (g.sell)
+            k_gnn_layer_mfma<true><<<mgrid, kBlock, 0, st>>>(n, g.slice_ptr, g.row_len, g.slot_cols, g.slot_w.get(), cur,
+                                                             p16, model->off_ws[l], model->off_wn[l], model->off_b[l],
+                                                             next, nullptr);
+        else
+            k_gnn_layer_mfma<false><<<mgrid, kBlock, 0, st>>>(n, g.offsets.get(), nullptr, g.cols.get(), g.w.get(), cur,
+                                                              p16, model->off_ws[l], model->off_wn[l], model->off_b[l],
+                                                              next,
+                                                              train ? agg + static_cast<std::int64_t>(l) * n * W : nullptr);
         OWTK_LAUNCH_CHECK();
         cur = next;
     }
@@ -1323,9 +1303,9 @@ void accumulate(owtk_gnn model, owtk_gnn_problem prob, double weight)
         const float* hout = v.h + static_cast<std::int64_t>(l + 1) * n * W;
         const float* hin = v.h + static_cast<std::int64_t>(l) * n * W;
         const float* agg = v.agg + static_cast<std::int64_t>(l) * n * W;
-        k_gnn_layer_bwd<<<grid, kBlock, 0, st>>>(n, hout, dh, p16, model->off_ws[l], model->off_wn[l], v.du, dprev, v.v);
+        k_gnn_layer_bwd<<<tile_grid(n), kBlock, 0, st>>>(n, hout, dh, p16, model->off_ws[l], model->off_wn[l], v.du, dprev, v.v);
         OWTK_LAUNCH_CHECK();
-        k_gnn_agg_t<<<grid, kBlock, 0, st>>>(n, g.offsets.get(), g.cols.get(), g.mirror.get(), g.w.get(), v.v, dprev);
+        k_gnn_agg_t<<<rows_grid(8 * n), kBlock, 0, st>>>(n, g.offsets.get(), g.cols.get(), g.mirror.get(), g.w.get(), v.v, dprev);
         OWTK_LAUNCH_CHECK();
         outer_reduce(model, n, v.du, W, nullptr, hin, W, agg, W, grad + model->off_ws[l], grad + model->off_wn[l],
                      grad + model->off_b[l], nullptr);
