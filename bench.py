@@ -52,8 +52,8 @@ KERNEL_NAMES = {
     "spmv_f64": "split SpMV, FP64 (spmv_sell_cd<3,double,double,true,EpiStore>)",
     "spmv_f32": "split SpMV, FP32 storage (spmv_sell_cd<3,float,float,...>)",
     "spmv_bf16": "split SpMV, BF16 storage (spmv_sell_cd<3,bf16,float,...>)",
-    "precond_f64": "block-Jacobi ILU(0) triangular sweeps, FP64 (k_tri_ell)",
-    "precond_low": "block-Jacobi ILU(0) triangular sweeps, low precision (k_tri_ell)",
+    "precond_f64": "block-Jacobi ILU(0) triangular sweeps, FP64 (k_tri_rows16)",
+    "precond_low": "block-Jacobi ILU(0) triangular sweeps, low precision (k_tri_rows16)",
     "learned": "learned series step, FP32 column-scaled off-diagonal values: SpMV + fused update "
                "(spmv_sell_cd<3,float,float,false,EpiSeries>)",
 }
