@@ -173,10 +173,16 @@ __device__ inline RowRef row_of(const TileRef& T)
     return rr;
 }
 
-// y_c = sum over the row's entries (diagonal included) of a_c x_col,c
-template<int BS, int U = 8>
+// y_c = sum over the row's entries (diagonal included) of a_c x_col,c, with
+// SCALED of a_c (dinv x)_col,c.  The graph path stores neither M p nor M s:
+// an iteration writes and reads back three vectors less, which costs the two
+// products a second gather (64 systems of 32^2 to 512^2 vertices, us per
+// launch: update p 19 -> 12.2, update s 17 -> 10.4, products 37 and 36 -> 42.5
+// and 40.3).  The values are the same bits.
+template<int BS, int U = 8, bool SCALED = false>
 __device__ inline void row_spmv(const Ptrs& P, std::int64_t prow, const double* __restrict__ x, double (&y)[BS])
 {
+    auto at = [&](std::int64_t i) { return SCALED ? P.dinv[i] * x[i] : x[i]; };
     const std::int64_t slice = prow >> 6;
     const int lane = static_cast<int>(prow & 63);
     const std::int64_t base = P.slice_ptr[slice];
@@ -197,7 +203,7 @@ __device__ inline void row_spmv(const Ptrs& P, std::int64_t prow, const double* 
 #pragma unroll
             for (int c = 0; c < BS; ++c) {
                 v[k][c] = vk[64 * c];
-                xv[k][c] = x[static_cast<std::int64_t>(colk[k]) * BS + c];
+                xv[k][c] = at(static_cast<std::int64_t>(colk[k]) * BS + c);
             }
         }
 #pragma unroll
@@ -214,7 +220,7 @@ __device__ inline void row_spmv(const Ptrs& P, std::int64_t prow, const double* 
         const std::int64_t col = P.cols[run + lane];
         const double* vk = P.vals + run * BS + lane;
 #pragma unroll
-        for (int c = 0; c < BS; ++c) y[c] = __builtin_fma(vk[64 * c], x[col * BS + c], y[c]);
+        for (int c = 0; c < BS; ++c) y[c] = __builtin_fma(vk[64 * c], at(col * BS + c), y[c]);
     }
 }
 
@@ -285,11 +291,10 @@ __global__ __launch_bounds__(kMaxTile) void kb_init(Ptrs P, const double* __rest
     store_tile_partials<2>(red, P, tile);
 }
 
-// p = r (first) or r + beta (p - omega v); r^ = r on restart; phat = M p.
+// p = r (first) or r + beta (p - omega v); r^ = r on restart.
 template<int BS>
 __global__ __launch_bounds__(kMaxTile) void kb_update_p(Ptrs P, const double* __restrict__ r, double* __restrict__ rhat,
-                                                        double* __restrict__ p, const double* __restrict__ v,
-                                                        double* __restrict__ phat)
+                                                        double* __restrict__ p, const double* __restrict__ v)
 {
     const int q = static_cast<int>(blockIdx.x);
     if (q >= *P.live_count) return;
@@ -303,43 +308,37 @@ __global__ __launch_bounds__(kMaxTile) void kb_update_p(Ptrs P, const double* __
     // On a first iteration (after the initial kernel or a restart) the p and
     // v values loaded are discarded by the select.
     const std::int64_t i0 = rr.vertex * BS;
-    double rv[BS], pv[BS], vv[BS], dv[BS];
+    double rv[BS], pv[BS], vv[BS];
 #pragma unroll
     for (int c = 0; c < BS; ++c) {
         rv[c] = r[i0 + c];
         pv[c] = p[i0 + c];
         vv[c] = v[i0 + c];
-        dv[c] = P.dinv[i0 + c];
     }
 #pragma unroll
     for (int c = 0; c < BS; ++c) {
         keep(rv[c]);
         keep(pv[c]);
         keep(vv[c]);
-        keep(dv[c]);
     }
     if (phase != 1) return;
-    double pn[BS], ph[BS];
+    double pn[BS];
 #pragma unroll
     for (int c = 0; c < BS; ++c) {
         const double upd = rv[c] + beta * (pv[c] - omega * vv[c]);
         pn[c] = first ? rv[c] : upd;
-        ph[c] = dv[c] * pn[c];
     }
 #pragma unroll
-    for (int c = 0; c < BS; ++c) {
-        p[i0 + c] = pn[c];
-        phat[i0 + c] = ph[c];
-    }
+    for (int c = 0; c < BS; ++c) p[i0 + c] = pn[c];
     if (restart) {
 #pragma unroll
         for (int c = 0; c < BS; ++c) rhat[i0 + c] = rv[c];
     }
 }
 
-// v = A phat; partial <r^, v>
+// v = A M p; partial <r^, v>
 template<int BS>
-__global__ __launch_bounds__(kMaxTile) void kb_spmv_v(Ptrs P, const double* __restrict__ phat,
+__global__ __launch_bounds__(kMaxTile) void kb_spmv_v(Ptrs P, const double* __restrict__ p,
                                                       const double* __restrict__ rhat, double* __restrict__ v)
 {
     const int q = static_cast<int>(blockIdx.x);
@@ -348,7 +347,7 @@ __global__ __launch_bounds__(kMaxTile) void kb_spmv_v(Ptrs P, const double* __re
     const int phase = P.st[rr.sys].phase;
     double y[BS], rh[BS];
     if (rr.vertex >= 0) {
-        row_spmv<BS>(P, rr.prow, phat, y);
+        row_spmv<BS, 8, true>(P, rr.prow, p, y);
 #pragma unroll
         for (int c = 0; c < BS; ++c) rh[c] = rhat[rr.vertex * BS + c];
 #pragma unroll
@@ -369,10 +368,10 @@ __global__ __launch_bounds__(kMaxTile) void kb_spmv_v(Ptrs P, const double* __re
     store_tile_partials<1>(red, P, q);
 }
 
-// s = r - alpha v; shat = M s; partial |s|^2
+// s = r - alpha v; partial |s|^2
 template<int BS>
 __global__ __launch_bounds__(kMaxTile) void kb_update_s(Ptrs P, const double* __restrict__ r, const double* __restrict__ v,
-                                                        double* __restrict__ s, double* __restrict__ shat)
+                                                        double* __restrict__ s)
 {
     const int q = static_cast<int>(blockIdx.x);
     if (q >= *P.live_count) return;
@@ -380,20 +379,18 @@ __global__ __launch_bounds__(kMaxTile) void kb_update_s(Ptrs P, const double* __
     const SysState& st = P.st[rr.sys];
     const int phase = st.phase;
     const double alpha = st.alpha;
-    double rv[BS], vv[BS], dv[BS];
+    double rv[BS], vv[BS];
     if (rr.vertex >= 0) {
 #pragma unroll
         for (int c = 0; c < BS; ++c) {
             const std::int64_t i = rr.vertex * BS + c;
             rv[c] = r[i];
             vv[c] = v[i];
-            dv[c] = P.dinv[i];
         }
 #pragma unroll
         for (int c = 0; c < BS; ++c) {
             keep(rv[c]);
             keep(vv[c]);
-            keep(dv[c]);
         }
     }
     if (phase != 1) return;
@@ -404,18 +401,17 @@ __global__ __launch_bounds__(kMaxTile) void kb_update_s(Ptrs P, const double* __
             const std::int64_t i = rr.vertex * BS + c;
             const double si = rv[c] - alpha * vv[c];
             s[i] = si;
-            shat[i] = dv[c] * si;
             red[0] = __builtin_fma(si, si, red[0]);
         }
     }
     store_tile_partials<1>(red, P, q);
 }
 
-// t = A shat; partials <t, s>, <t, t>.  Early exit: x += alpha phat only.
+// t = A M s; partials <t, s>, <t, t>.  Early exit: x += alpha M p only.
 template<int BS>
-__global__ __launch_bounds__(kMaxTile) void kb_spmv_t(Ptrs P, const double* __restrict__ shat,
-                                                      const double* __restrict__ s, double* __restrict__ t,
-                                                      const double* __restrict__ phat, double* __restrict__ x)
+__global__ __launch_bounds__(kMaxTile) void kb_spmv_t(Ptrs P, const double* __restrict__ s,
+                                                      double* __restrict__ t, const double* __restrict__ p,
+                                                      double* __restrict__ x)
 {
     const int q = static_cast<int>(blockIdx.x);
     if (q >= *P.live_count) return;
@@ -427,7 +423,7 @@ __global__ __launch_bounds__(kMaxTile) void kb_spmv_t(Ptrs P, const double* __re
     // most once per system) discards it.
     double y[BS], sv[BS];
     if (rr.vertex >= 0) {
-        row_spmv<BS>(P, rr.prow, shat, y);
+        row_spmv<BS, 8, true>(P, rr.prow, s, y);
 #pragma unroll
         for (int c = 0; c < BS; ++c) sv[c] = s[rr.vertex * BS + c];
 #pragma unroll
@@ -442,7 +438,7 @@ __global__ __launch_bounds__(kMaxTile) void kb_spmv_t(Ptrs P, const double* __re
 #pragma unroll
             for (int c = 0; c < BS; ++c) {
                 const std::int64_t i = rr.vertex * BS + c;
-                x[i] = __builtin_fma(alpha, phat[i], x[i]);
+                x[i] = __builtin_fma(alpha, P.dinv[i] * p[i], x[i]);
             }
         }
         return;
@@ -459,10 +455,9 @@ __global__ __launch_bounds__(kMaxTile) void kb_spmv_t(Ptrs P, const double* __re
     store_tile_partials<2>(red, P, q);
 }
 
-// x += alpha phat + omega shat; r = s - omega t; partials <r^, r>, |r|^2
+// x += alpha M p + omega M s; r = s - omega t; partials <r^, r>, |r|^2
 template<int BS>
-__global__ __launch_bounds__(kMaxTile) void kb_update_x(Ptrs P, const double* __restrict__ phat,
-                                                        const double* __restrict__ shat, const double* __restrict__ s,
+__global__ __launch_bounds__(kMaxTile) void kb_update_x(Ptrs P, const double* __restrict__ p, const double* __restrict__ s,
                                                         const double* __restrict__ t, const double* __restrict__ rhat,
                                                         double* __restrict__ x, double* __restrict__ r)
 {
@@ -472,13 +467,13 @@ __global__ __launch_bounds__(kMaxTile) void kb_update_x(Ptrs P, const double* __
     const SysState& st = P.st[rr.sys];
     const int phase = st.phase, early = st.early;
     const double alpha = st.alpha, omega = st.omega;
-    double ph[BS], sh[BS], sv[BS], tv[BS], rh[BS], xv[BS];
+    double pv[BS], dv[BS], sv[BS], tv[BS], rh[BS], xv[BS];
     if (rr.vertex >= 0) {
 #pragma unroll
         for (int c = 0; c < BS; ++c) {
             const std::int64_t i = rr.vertex * BS + c;
-            ph[c] = phat[i];
-            sh[c] = shat[i];
+            pv[c] = p[i];
+            dv[c] = P.dinv[i];
             sv[c] = s[i];
             tv[c] = t[i];
             rh[c] = rhat[i];
@@ -486,8 +481,8 @@ __global__ __launch_bounds__(kMaxTile) void kb_update_x(Ptrs P, const double* __
         }
 #pragma unroll
         for (int c = 0; c < BS; ++c) {
-            keep(ph[c]);
-            keep(sh[c]);
+            keep(pv[c]);
+            keep(dv[c]);
             keep(sv[c]);
             keep(tv[c]);
             keep(rh[c]);
@@ -500,7 +495,7 @@ __global__ __launch_bounds__(kMaxTile) void kb_update_x(Ptrs P, const double* __
 #pragma unroll
         for (int c = 0; c < BS; ++c) {
             const std::int64_t i = rr.vertex * BS + c;
-            x[i] = __builtin_fma(omega, sh[c], __builtin_fma(alpha, ph[c], xv[c]));
+            x[i] = __builtin_fma(omega, dv[c] * sv[c], __builtin_fma(alpha, dv[c] * pv[c], xv[c]));
             const double ri = sv[c] - omega * tv[c];
             r[i] = ri;
             red[0] = __builtin_fma(rh[c], ri, red[0]);
@@ -553,12 +548,26 @@ __device__ inline Sums system_sums(const Ptrs& P, const std::int32_t* sys_blk0, 
     const int lane = threadIdx.x;
     const std::int32_t tiles = sys_blk0[sys + 1] - sys_blk0[sys];
     const std::int32_t b0 = INIT ? sys_blk0[sys] : P.live_first[sys], b1 = b0 + tiles;
+    // U tiles of every value in flight: 512 x 512 vertices are 1,024 tiles,
+    // sixteen loads a lane and value one after another otherwise.
+    // The finishers of 64 systems up to that size: 7.2 -> 4.0 us.
+    constexpr int U = 8;
+    double acc[K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-        double acc = 0.0;
-        for (std::int32_t b = b0 + lane; b < b1; b += 64) acc += P.partials[k * P.blocks + b];
-        out.v[k] = dev::wave_sum(acc);
+    for (int k = 0; k < K; ++k) acc[k] = 0.0;
+    for (std::int32_t base = b0 + lane; base < b1; base += 64 * U) {
+        double p[K][U];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int u = 0; u < U; ++u) p[k][u] = P.partials[k * P.blocks + (base + 64 * u < b1 ? base + 64 * u : base)];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc[k] = base + 64 * u < b1 ? acc[k] + p[k][u] : acc[k];
     }
+#pragma unroll
+    for (int k = 0; k < K; ++k) out.v[k] = dev::wave_sum(acc[k]);
     return out;
 }
 
@@ -1108,14 +1117,14 @@ void launch_iteration(owtk_batch bt, Tiling& tl, const double* b, double* x)
     const unsigned int T = static_cast<unsigned int>(tl.tile);
     const unsigned int S = static_cast<unsigned int>(bt->systems);
     const std::int32_t* sb0 = tl.sys_blk0.get();
-    kb_update_p<BS><<<grid, T, 0, st>>>(P, bt->r.get(), bt->rhat.get(), bt->p.get(), bt->v.get(), bt->phat.get());
-    kb_spmv_v<BS><<<grid, T, 0, st>>>(P, bt->phat.get(), bt->rhat.get(), bt->v.get());
+    kb_update_p<BS><<<grid, T, 0, st>>>(P, bt->r.get(), bt->rhat.get(), bt->p.get(), bt->v.get());
+    kb_spmv_v<BS><<<grid, T, 0, st>>>(P, bt->p.get(), bt->rhat.get(), bt->v.get());
     kb_finish<fin_alpha><<<S, 64, 0, st>>>(P, sb0);
-    kb_update_s<BS><<<grid, T, 0, st>>>(P, bt->r.get(), bt->v.get(), bt->s.get(), bt->shat.get());
+    kb_update_s<BS><<<grid, T, 0, st>>>(P, bt->r.get(), bt->v.get(), bt->s.get());
     kb_finish<fin_s><<<S, 64, 0, st>>>(P, sb0);
-    kb_spmv_t<BS><<<grid, T, 0, st>>>(P, bt->shat.get(), bt->s.get(), bt->t.get(), bt->phat.get(), x);
+    kb_spmv_t<BS><<<grid, T, 0, st>>>(P, bt->s.get(), bt->t.get(), bt->p.get(), x);
     kb_finish<fin_omega><<<S, 64, 0, st>>>(P, sb0);
-    kb_update_x<BS><<<grid, T, 0, st>>>(P, bt->phat.get(), bt->shat.get(), bt->s.get(), bt->t.get(), bt->rhat.get(), x,
+    kb_update_x<BS><<<grid, T, 0, st>>>(P, bt->p.get(), bt->s.get(), bt->t.get(), bt->rhat.get(), x,
                                         bt->r.get());
     kb_finish<fin_rho><<<S, 64, 0, st>>>(P, sb0);
     kb_true_residual<BS><<<grid, T, 0, st>>>(P, b, x, bt->r.get());
