@@ -371,12 +371,12 @@ def batched_roofline(systems, vertices, ms_it):
     """Algorithmic HBM bytes of one all-active batched BiCGSTAB + Jacobi
     iteration over the autotuner's time for one. Its two SpMVs each read every
     stored entry (3 FP64 values + a 4-byte column) and the row lengths. Its
-    five streaming kernels move 25 block vectors of 3 FP64 values per vertex:
-    p update 4 read + 2 written, v = A p^ 3 (p^ gathered once, r^, v),
-    s update 3 + 2, t = A s^ 3, x/r update 6 + 2. Finishers and padding slots
-    are overhead, not counted."""
+    five streaming kernels move 22 block vectors of 3 FP64 values per vertex:
+    p update 3 read + 1 written, v = A M p 4 (p and the inverse diagonal
+    gathered once each, r^, v), s update 2 + 1, t = A M s 3, x/r update 6 + 2.
+    Finishers and padding slots are overhead, not counted."""
     entries = sum(int(s[1][-1]) for s in systems)
-    nbytes = 2 * (entries * (BS * 8 + 4) + vertices * 4) + 25 * vertices * BS * 8
+    nbytes = 2 * (entries * (BS * 8 + 4) + vertices * 4) + 22 * vertices * BS * 8
     gbps = nbytes / (ms_it * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": round(gbps, 1), "peak": PEAK_HBM_GBPS, "unit": "GB/s",
             "frac": round(gbps / PEAK_HBM_GBPS, 4), "traffic": None,
