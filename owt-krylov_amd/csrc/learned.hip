@@ -229,6 +229,8 @@ constexpr int kMfmaEdges = 2;  // edges gathered per pass of the aggregation
 // padded with zeros to 16 and split over the half-waves (step t takes
 // feature t + 8 h), 8 steps of v_mfma_f32_32x32x2_f32; output layout as in
 // k_gnn_layer_mfma, so each store instruction writes two whole rows of h.
+// 131,072 vertices, vertex-major features: 12 us (a thread per vertex with the
+// weights in LDS: 26).
 static_assert(kGnnMaxFeatures <= 16, "the matrix-core encoding takes at most 16 features");
 __global__ __launch_bounds__(256) void k_gnn_encode_mfma(std::int64_t n, int f0, const float* __restrict__ x,
                                                          std::int64_t sf, std::int64_t sv,
