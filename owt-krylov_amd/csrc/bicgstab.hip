@@ -115,9 +115,10 @@ __global__ __launch_bounds__(256) void k_p_update(double* __restrict__ p, const 
         p[i] = first ? r[i] : __builtin_fma(beta, __builtin_fma(-omega, v[i], p[i]), r[i]);
 }
 
-// s = r - alpha v, ||s||
+// s = r - alpha v, ||s||  (s is not restrict, nor is r in k_xr_update: the
+// finalizer may read them through pointers of its own)
 template<bool CMP, class Fin>
-__global__ __launch_bounds__(256) void k_s_update(double* __restrict__ s, const double* __restrict__ r,
+__global__ __launch_bounds__(256) void k_s_update(double* s, const double* __restrict__ r,
                                                   const double* __restrict__ v, std::int64_t n, BicgState* st,
                                                   Fin fin, ReduceScratch scratch)
 {
@@ -137,6 +138,7 @@ __global__ __launch_bounds__(256) void k_s_update(double* __restrict__ s, const 
 }
 
 struct FinSnorm {
+    static constexpr bool kReadsStores = true;
     BicgState* st;
     const double* s;
     std::int64_t n;
@@ -155,7 +157,7 @@ struct FinSnorm {
 
 // x += alpha z; x += omega y; r = s - omega t; <shadow, r>, ||r||
 template<bool CMP, class Fin>
-__global__ __launch_bounds__(256) void k_xr_update(double* __restrict__ x, double* __restrict__ r,
+__global__ __launch_bounds__(256) void k_xr_update(double* __restrict__ x, double* r,
                                                    const double* __restrict__ z, const double* __restrict__ y,
                                                    const double* __restrict__ s, const double* __restrict__ t,
                                                    const double* __restrict__ shadow, std::int64_t n, BicgState* st,
@@ -253,6 +255,7 @@ struct FinDot2 {
 };
 
 struct FinXr {
+    static constexpr bool kReadsStores = true;
     BicgState* st;
     const double* r;
     std::int64_t n;
@@ -417,6 +420,7 @@ struct EpiOmegaP : dev::EpiNone {
 
 // after x/r: next rho, recursive |r| (tested every iteration), beta, cadence
 struct FinNextP {
+    static constexpr bool kReadsStores = true;
     BicgState* st;
     const double* r;
     std::int64_t n;
@@ -584,6 +588,7 @@ __global__ __launch_bounds__(256) void k_ch_first(ChVecs V, std::int64_t n, cons
 }
 
 struct FinChFirst {
+    static constexpr bool kReadsStores = true;
     ChState* st;
     const double* q;
     std::int64_t n;
@@ -659,6 +664,7 @@ __global__ __launch_bounds__(256) void k_ch_second(ChVecs V, double* __restrict_
 }
 
 struct FinChSecond {
+    static constexpr bool kReadsStores = true;
     ChState* st;
     const double* r;
     std::int64_t n;

@@ -513,6 +513,7 @@ __global__ __launch_bounds__(256) void k_fg_update(T* __restrict__ x, const T* _
 template<class X>
 struct EpiResidualT : dev::EpiNone {
     static constexpr int K = 2;
+    static constexpr bool kReadsStores = true;
     static constexpr std::uint64_t kMaxMask = 2;
     X* y;
     const X* b;

@@ -58,6 +58,7 @@ struct EpiNone {
     // The matrix is streamed with the non-temporal hint unless an epilogue
     // belongs to a kernel that rereads the same matrix right away.
     static constexpr bool kKeepMatrix = false;
+    static constexpr bool kReadsStores = false;  // finalize reads y (reduce_end)
     const int* stop = nullptr;
     __device__ bool stopped() const { return stop != nullptr && *stop != 0; }
     __device__ void finalize(const double*) const {}
@@ -100,6 +101,7 @@ __device__ inline void epi_row(const E& e, std::int64_t i0, const A (&acc)[BS], 
 // y = b - A x, reduced: sum y^2, max |y|; norm written by finalize.
 struct EpiResidual : EpiNone {
     static constexpr int K = 2;
+    static constexpr bool kReadsStores = true;
     static constexpr std::uint64_t kMaxMask = 2;
     double* y;
     const double* b;
@@ -195,6 +197,7 @@ struct EpiDot2 : EpiNone {
 // Finisher adaptor: runs an epilogue's finalize in the one-block finisher.
 template<class E>
 struct EpiFinish {
+    static constexpr bool kReadsStores = E::kReadsStores;
     E e;
     __device__ void operator()(const double* t) const { e.finalize(t); }
 };

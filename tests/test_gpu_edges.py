@@ -303,3 +303,42 @@ def test_ilu_small_pivot_anywhere(ctx, row):
         pc.update_values()
     m.update_values(d, e)
     pc.update_values()
+
+
+@pytest.mark.parametrize("nx,ny,block", [(9, 7, 2), (128, 128, 3), (128, 256, 1), (60, 40, 5)])
+def test_norms_of_vectors_written_by_their_own_kernel(ctx, nx, ny, block):
+    """Right-hand sides scaled until the sum of squares leaves the range that the norm takes as it is (below 2^-960,
+    or infinite), on grids of at most 128 blocks: the kernels that write s, r, q and b - A x then read them back for
+    the scaled second pass, written by other waves and blocks.  The small scale is a power of two that leaves the
+    products normal (above 1024 times the least normal number down to rtol 1e-5), so the solve is that of the
+    unscaled right-hand side: the same iterations, norms to the rounding of their sums, solutions to 1e-8 (rounding
+    near the subnormal range, grown over the iterations).  At the large one the products are infinite: the first
+    residual's norm, and the status of the oracle."""
+    s = owtk.generate_split(nx, ny, block, 4, ordering=owtk.ORDER_RCM)
+    om = orc.OMatrix.split(s.nodes, 0, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    m = owtk.Matrix.split(ctx, s.nodes, 0, block, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    pc, opc = owtk.Preconditioner(m, owtk.PC_JACOBI), orc.OPreconditioner(om, orc.OPreconditioner.JACOBI)
+    kw = dict(relative_tolerance=1e-5, maximum_iterations=200)
+    norm = np.linalg.norm(s.rhs)
+    small = 2.0 ** np.floor((-964 - np.log2(norm ** 2)) / 2)
+    huge = 2.0 ** 700
+    bs, bl = ctx.upload(s.rhs * small), ctx.upload(s.rhs * huge)
+    b, x = ctx.upload(s.rhs), ctx.empty(s.nodes * block)
+    for solve, oracle in ((owtk.bicgstab, orc.bicgstab), (owtk.pipelined_bicgstab, orc.pipelined_bicgstab),
+                          (owtk.communication_hiding_bicgstab, orc.communication_hiding_bicgstab),
+                          (owtk.fgmres, orc.fgmres)):
+        x.zero()
+        ref = solve(m, pc, b, x, owtk.SolverOptions(**kw))
+        xr = x.download()
+        assert ref["status_name"] == "converged"
+        x.zero()
+        res = solve(m, pc, bs, x, owtk.SolverOptions(**kw))
+        assert res["status_name"] == "converged" and res["iterations"] == ref["iterations"]
+        assert np.max(np.abs(x.download() / small - xr)) <= 1e-8 * np.max(np.abs(xr))
+        for key in ("initial_residual_norm", "true_residual_norm"):
+            assert abs(res[key] / small - ref[key]) <= (1e-13 if key[0] == "i" else 1e-6) * ref[key]
+        x.zero()
+        res = solve(m, pc, bl, x, owtk.SolverOptions(**kw))
+        _, ro = oracle(om, opc, s.rhs * huge, **kw)
+        assert res["status"] == ro["status"]
+        assert abs(res["initial_residual_norm"] / huge - norm) <= 1e-13 * norm
