@@ -618,7 +618,12 @@ int owtk_batch_autotune_groups(owtk_batch batch, const double* b, const owtk_sol
 int owtk_batch_bicgstab(owtk_batch batch, const double* b, double* x, const owtk_solver_options* options,
                         int32_t graph_iterations, owtk_batch_result* results);
 
-/* --------------------------------------------------------- vector kernels -- */
+/* --------------------------------------------------------- vector kernels --
+ * The calls with a result on the host (dot, norm, reduction_*, axpy_dot,
+ * multidot) return when it has arrived there, which may be before the stream
+ * reports itself idle.  By then everything queued on the context's stream
+ * before, their inputs' reads and the vector that axpy_dot writes are complete
+ * and may be used from any stream. */
 /* dot with FP64 accumulation (SerialReduction::dot, reduction.hpp:114-145). */
 int owtk_dot(owtk_context ctx, owtk_dtype dtype, size_t n, const void* a, const void* b,
              double* out);

@@ -255,7 +255,7 @@ inline ReduceScratch scratch_for(ReduceScratch s, unsigned int g)
 }
 
 // Finalizers that read a vector which their own kernel wrote, or report to a
-// host that may, say so: static constexpr bool kReadsStores = true.
+// host that may read it, say so: static constexpr bool kReadsStores = true.
 template<class Fin>
 constexpr bool reads_stores()
 {
@@ -274,9 +274,10 @@ __device__ inline void stores_in_l2()
 // block to arrive does the finisher's work (the same sums in the same order).
 // Thread 0's fence before the counter writes the XCD's L2 back and so publishes
 // what the block had stored there by then: the partials, which thread 0 stored
-// itself, and where the finalizer reads a vector of this kernel (block_norm's
-// second pass) also the vector, because every wave then waits for its own
-// stores before the block's barriers, which wait for LDS only.  (A release
+// itself, and where a vector of this kernel is read next (by block_norm's
+// second pass, or by the host's other streams once it has the result) also the
+// vector, because every wave then waits for its own stores before the block's
+// barriers, which wait for LDS only.  (A release
 // fence in every wave would write the L2 back four times a block: 47 -> 56 us
 // an iteration of BiCGSTAB + Jacobi at 32,768 vertices.)
 template<int K, class Fin>

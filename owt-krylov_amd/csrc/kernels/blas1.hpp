@@ -76,6 +76,12 @@ struct FinStore {
     }
 };
 
+// of a kernel that also writes a vector: when the host has the number, another
+// stream may read the vector (reduce_end)
+struct FinStoreAll : FinStore {
+    static constexpr bool kReadsStores = true;
+};
+
 // Dot product with FP64 accumulation; CMP: compensated (double-double).
 template<class X, bool CMP = false>
 __global__ __launch_bounds__(256) void k_dot(const X* __restrict__ a, const X* __restrict__ b, std::int64_t n,
@@ -217,7 +223,7 @@ inline void axpy(hipStream_t st, std::int64_t n, double alpha, const double* x, 
 
 __global__ __launch_bounds__(256) void k_axpy_dot(std::int64_t n, double alpha, const double* __restrict__ x,
                                                   double* __restrict__ y, const double* __restrict__ w,
-                                                  ReduceScratch scratch, FinStore fin)
+                                                  ReduceScratch scratch, FinStoreAll fin)
 {
     double red[1] = {0.0};
     const std::int64_t stride = static_cast<std::int64_t>(gridDim.x) * blockDim.x;
@@ -234,7 +240,7 @@ inline void axpy_dot_to(hipStream_t st, ReduceScratch scratch, std::int64_t n, d
 {
     const unsigned int g = stream_grid(n, 4);
     const ReduceScratch sc = scratch_for(scratch, g);
-    const FinStore fin{out, 1, mail};
+    const FinStoreAll fin{{out, 1, mail}};
     k_axpy_dot<<<g, kBlock, 0, st>>>(n, alpha, x, y, w, sc, fin);
     launch_finish<1>(st, fin, g, 0, sc, nullptr);
     OWTK_LAUNCH_CHECK();

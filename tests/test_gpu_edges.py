@@ -342,3 +342,14 @@ def test_norms_of_vectors_written_by_their_own_kernel(ctx, nx, ny, block):
         _, ro = oracle(om, opc, s.rhs * huge, **kw)
         assert res["status"] == ro["status"]
         assert abs(res["initial_residual_norm"] / huge - norm) <= 1e-13 * norm
+
+
+@pytest.mark.parametrize("n", [1000, 6144, 128 * 1024, 128 * 1024 + 1])
+def test_axpy_dot_vector_is_complete_on_return(ctx, n):
+    """The vector that axpy_dot writes, read on another context's stream as soon as the call has returned, below, at
+    and above the largest grid that ends its own reduction.  Every element changes each time, by the exact 1."""
+    ones, y = ctx.upload(np.ones(n)), ctx.upload(np.zeros(n))
+    with owtk.Context(0) as other:
+        for k in range(1, 21):
+            assert ctx.axpy_dot(1.0, ones, y, ones) == k * n
+            assert other.dot(y, ones) == k * n
