@@ -180,8 +180,9 @@ typedef struct owtk_precond_params {
     int64_t block_nodes;      /* block-Jacobi partition: consecutive node ranges
                                  of this size; 0 = one block over all owned nodes */
     int32_t fill_level;       /* ILU(k) level (0 = ILU(0)) */
-    int32_t schedule;         /* triangular sweeps: 0 auto, 1 level sets, 2 one-wave chains
-                                 (same results; a performance choice) */
+    int32_t schedule;         /* triangular sweeps: 0 auto, 1 level sets, 2 chains (same results to
+                                 rounding; a performance choice).  Chains take at most 16 entries
+                                 per row and direction and blocks of at most 16384 rows. */
     void* learned_model;      /* owtk_gnn for OWTK_PC_LEARNED */
 } owtk_precond_params;
 

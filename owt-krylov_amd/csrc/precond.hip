@@ -6,6 +6,7 @@
 // GPU.  This is the reference's "symbolic once, numeric many" contract
 // (IluLevelPreconditioner::update_values, preconditioner.hpp:269-311).
 #include "precond.hpp"
+#include "chain_rule.hpp"
 #include "learned.hpp"
 #include "kernels/blas1.hpp"
 #include "kernels/spmv.hpp"
@@ -1104,6 +1105,7 @@ __global__ __launch_bounds__(128) void k_tri_rows16(Rows16Args a, const V* __res
     constexpr int P = chunks_ahead(K);
     static_assert(2 * K * 128 <= kGroup16 - kFar16 && kTile16 + 16 * 512 <= 65536 && P % 2 == 0 && kRing16 % P == 0 && 3 * P + 2 <= kPadChunks16);
     static_assert(kRingZero + 128 <= kFar16);
+    static_assert(K <= kChainEntries && (2 * P + 2) * 16 <= kChainOverrun && kChainRows <= 32767);
     __shared__ __attribute__((aligned(16))) unsigned char lds[kLds16];
     if (stop && *stop) return;
     const int lane = static_cast<int>(threadIdx.x & 63);
@@ -1231,8 +1233,6 @@ struct TriHost {
     std::vector<std::int64_t> f_off, f_col, f_src, b_off, b_col, b_src;
 };
 
-std::size_t lds_limit(owtk_precond pc);
-
 // Codes and value maps of the chain sweeps (k_tri_rows16) from the chain
 // layout: entry k of the row at position p (chunk q = p / 16, lane l) goes to
 // value slot ((q * K / 2 + k / 2) * 16 + l) * 2 + k % 2 of its block.
@@ -1331,14 +1331,18 @@ void build_schedule(owtk_precond pc, const TriHost& t)
         tri.max_blevels = std::max<std::int64_t>(tri.max_blevels, bdepth[b]);
         depth_sum += std::max(fdepth[b], bdepth[b]);
     }
-    // Chain sweeps win when levels are narrow (average width below 16 rows):
-    // a level then costs a barrier for a handful of rows.
+    // Chain sweeps win when levels are narrow: a level then costs a barrier
+    // (about 1.1 us) for a handful of rows, a chain 0.25 us per 16 rows.  The
+    // line at an average width of 16 rows is on the safe side of the crossing:
+    // RCM-ordered 512 x 512 grid, block 3, level sets / chains in us: 917 / 127
+    // at width 8 (4,096-row blocks), 1,233 / 491 at width 30 (16,384); one
+    // 8,192-row block in random order, width 585: 63 / 295.
     tri.emax = emax;
-    const bool chain_ok = emax <= 16
-        && (static_cast<std::size_t>(tri.max_block_rows) + 64 * 64) * sizeof(double) <= lds_limit(pc);
+    const bool chain_ok = emax <= kChainEntries && tri.max_block_rows <= kChainRows;
     if (pc->schedule == 2 && !chain_ok)
-        throw unsupported_error("chain sweeps need at most 16 entries per row and a block that fits in LDS");
-    tri.chain = pc->schedule == 2 || (pc->schedule == 0 && chain_ok && depth_sum * 16 > n);
+        throw unsupported_error("chain sweeps need at most 16 entries per row and blocks of at most 16384 rows");
+    tri.chain = (pc->schedule == 2 || (pc->schedule == 0 && chain_ok && depth_sum * 16 > n))
+        && chain_offsets_fit(tri.blocks, tri.max_block_rows, tri.bs);
     // pass 2: level lists and apply arrays
     std::vector<std::int32_t> frow(n), brow(n), frow_lvl(n);
     std::vector<std::int64_t> fptr(n + 1, 0), bptr(n + 1, 0);

@@ -353,3 +353,22 @@ def test_axpy_dot_vector_is_complete_on_return(ctx, n):
         for k in range(1, 21):
             assert ctx.axpy_dot(1.0, ones, y, ones) == k * n
             assert other.dot(y, ones) == k * n
+
+
+@pytest.mark.parametrize("n", [16384, 16385])
+def test_chain_sweeps_largest_block(ctx, n):
+    """The largest block that the chain sweeps take, and one row more: refused when asked for, level sets otherwise.
+    Bound as for the other chain sweeps."""
+    rng = np.random.default_rng(n)
+    off, col, diag, val = banded(rng, n, 1, 500, 3)
+    m = owtk.Matrix.split(ctx, n, 0, 1, off, col, diag, val)
+    opc = orc.OPreconditioner(orc.OMatrix.split(n, 0, 1, off, col, diag, val), 3)
+    x = rng.uniform(-1, 1, n)
+    xd, yd, ref = ctx.upload(x), ctx.empty(n), opc.apply(x)
+    for schedule in (0, 2):
+        if n > 16384 and schedule == 2:
+            with pytest.raises(owtk.OwtkError, match="16384 rows"):
+                owtk.Preconditioner(m, owtk.PC_ILU, schedule=schedule)
+            continue
+        owtk.Preconditioner(m, owtk.PC_ILU, schedule=schedule).apply(xd, yd)
+        assert np.max(np.abs(yd.download() - ref)) <= 1e-14 * np.max(np.abs(ref))
