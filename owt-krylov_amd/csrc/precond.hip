@@ -878,21 +878,27 @@ struct Rows16Sweep {
     __device__ X& at(unsigned int byte) const { return *reinterpret_cast<X*>(lds + byte); }
 };
 
-// One barrier a chunk.  Only LDS is handed over, so only LDS is waited for:
-// the loads of later chunks stay in flight.
+// One barrier a chunk.  LDS is handed over, and the results in memory that the
+// preparing wave gathers many chunks later.  A workgroup's waves share one L1,
+// which takes their accesses in order, so these fences wait for LDS alone and
+// the loads of later chunks stay in flight (the code is the same as with
+// fences for LDS only).
 __device__ inline void chunk_barrier()
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // The preparing wave: during chunk q it writes the tile, right-hand side and
 // diagonal of chunk q + 2 (the solving wave reads chunk q + 1's then) and the
-// far values of chunk q + 1.  Codes, values and rows of a chunk load P chunks ahead, the
-// far rows' numbers 2P.  A far row is stored at least 28 - P - 2 chunks
-// before its gather is issued, and the storing wave has since waited for
-// loads it issued after that store.
+// far values of chunk q + 1.  Codes, values and rows of a chunk load P chunks
+// ahead, the far rows' numbers 2P.  The rows of chunk q + P + 1 are gathered
+// during chunk q, and a far row of it was stored in chunk q + P + 1 - kRing16
+// or before: kFarBarriers barriers lie between, and the storing wave has
+// waited for loads that it issued after that store (those of the chunk after
+// it, used P + 1 chunks later).
+template<int K> constexpr int kFarBarriers = kRing16 - chunks_ahead(K) - 1;
 template<TriMode MODE, bool FWD, class X, class V, int K>
 __device__ __attribute__((always_inline)) inline void rows16_prepare(const Rows16Sweep<X, V>& s)
 {
@@ -1105,6 +1111,7 @@ __global__ __launch_bounds__(128) void k_tri_rows16(Rows16Args a, const V* __res
     constexpr int P = chunks_ahead(K);
     static_assert(2 * K * 128 <= kGroup16 - kFar16 && kTile16 + 16 * 512 <= 65536 && P % 2 == 0 && kRing16 % P == 0 && 3 * P + 2 <= kPadChunks16);
     static_assert(kRingZero + 128 <= kFar16);
+    static_assert(kFarBarriers<K> >= P + 2, "a far row's store is waited for before its gather");
     static_assert(K <= kChainEntries && (2 * P + 2) * 16 <= kChainOverrun && kChainRows <= 32767);
     __shared__ __attribute__((aligned(16))) unsigned char lds[kLds16];
     if (stop && *stop) return;
