@@ -1294,6 +1294,21 @@ void build_rows16(TriSchedule& tri, const std::vector<std::int64_t>& fptr, const
     tri.slots16 = chunks * K * 16;
 }
 
+// Whether a row names a column more than once in one direction.  The chains'
+// tile has one place for a (row, column of the chunk), so such rows take the
+// level sets, which add the products up.
+bool repeated_columns(const TriHost& t, std::int64_t n)
+{
+    for (std::int64_t i = 0; i < n; ++i)
+        for (const auto* d : {&t.f_off, &t.b_off}) {
+            const auto& col = d == &t.f_off ? t.f_col : t.b_col;
+            for (std::int64_t e = (*d)[i]; e < (*d)[i + 1]; ++e)
+                for (std::int64_t k = (*d)[i]; k < e; ++k)
+                    if (col[k] == col[e]) return true;
+        }
+    return false;
+}
+
 void build_schedule(owtk_precond pc, const TriHost& t)
 {
     auto& tri = pc->tri;
@@ -1349,7 +1364,7 @@ void build_schedule(owtk_precond pc, const TriHost& t)
     if (pc->schedule == 2 && !chain_ok)
         throw unsupported_error("chain sweeps need at most 16 entries per row and blocks of at most 16384 rows");
     tri.chain = (pc->schedule == 2 || (pc->schedule == 0 && chain_ok && depth_sum * 16 > n))
-        && chain_offsets_fit(tri.blocks, tri.max_block_rows, tri.bs);
+        && chain_offsets_fit(tri.blocks, tri.max_block_rows, tri.bs) && !repeated_columns(t, n);
     // pass 2: level lists and apply arrays
     std::vector<std::int32_t> frow(n), brow(n), frow_lvl(n);
     std::vector<std::int64_t> fptr(n + 1, 0), bptr(n + 1, 0);

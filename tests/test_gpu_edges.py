@@ -372,3 +372,29 @@ def test_chain_sweeps_largest_block(ctx, n):
             continue
         owtk.Preconditioner(m, owtk.PC_ILU, schedule=schedule).apply(xd, yd)
         assert np.max(np.abs(yd.download() - ref)) <= 1e-14 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("schedule", [0, 1, 2])
+@pytest.mark.parametrize("block,nodes", [(1, 0), (3, 50)])
+def test_ssor_repeated_columns(ctx, schedule, block, nodes):
+    """SSOR of CSR rows that name a column more than once (their products add up), near the row and farther off, by
+    every schedule.  Bound as for the other sweeps."""
+    rng = np.random.default_rng(7)
+    n = 200
+    offsets, columns, values = [0], [], []
+    for i in range(n):
+        near = np.array([j for j in (i - 70, i - 20, i - 3, i - 1, i + 1, i + 2, i + 33) if 0 <= j < n])
+        twice = rng.choice(near, 2)
+        cols = np.sort(np.concatenate([near, twice, [i]]))
+        val = -rng.uniform(0.1, 1.0, (cols.size, block))
+        val[cols == i] = np.abs(val).sum(0) + 0.5
+        columns.append(cols)
+        values.append(val)
+        offsets.append(offsets[-1] + cols.size)
+    args = (n, 0, block, np.array(offsets, np.int32), np.concatenate(columns).astype(np.int32), np.concatenate(values).ravel())
+    x = rng.uniform(-1, 1, n * block)
+    ref = orc.OPreconditioner(orc.OMatrix.csr(*args), orc.OPreconditioner.SSOR, block_nodes=nodes, omega=1.2).apply(x)
+    yd = ctx.empty(n * block)
+    owtk.Preconditioner(owtk.Matrix.csr(ctx, *args), owtk.PC_SSOR, block_nodes=nodes, omega=1.2,
+                        schedule=schedule).apply(ctx.upload(x), yd)
+    assert np.max(np.abs(yd.download() - ref)) <= 1e-14 * np.max(np.abs(ref))
