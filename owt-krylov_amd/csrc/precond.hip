@@ -1525,6 +1525,7 @@ void refresh_storage(owtk_precond pc)
         if (!t.dval32.get()) t.dval32.allocate(std::max<std::int64_t>(nd, 1));
         kern::convert(st, t.dval32.get(), t.dval64.get(), static_cast<std::size_t>(nd));
     }
+    if (t.chain) return;  // the flat copies are for the level sets alone
     if (pc->storage == OWTK_F32) {
         if (!t.fval32.get()) t.fval32.allocate(std::max<std::int64_t>(t.fnnz * bs, 1));
         if (!t.bval32.get()) t.bval32.allocate(std::max<std::int64_t>(t.bnnz * bs, 1));
