@@ -1288,7 +1288,26 @@ void accumulate(owtk_gnn model, owtk_gnn_problem prob, double weight)
     if (P <= 2) loss(std::integral_constant<int, 2>{});
     else if (P <= 5) loss(std::integral_constant<int, 5>{});
     else loss(std::integral_constant<int, 10>{});
-    k_loss_dgamma<5><<<lgrid, kBlock, 0, st>>>(nb, P, k1, model->z.get(), prob->u.get(), model->dgamma.get());
+    // coefficients in registers: the fewest passes of at most 8, filled evenly.
+    // A pass reads g again and costs its KK loads however few are left: with a
+    // fixed 5, degree 5 (block 3) took 30.7 us at 131,072 vertices and 10
+    // pairs, 23.3 this way; degrees 7 and 10 (block 1) 11.4 -> 8.7 and
+    // 14.9 -> 13.6; degree 4 takes one pass of 5 either way, 21.
+    const int passes = (k1 + 7) / 8;
+    auto dgamma = [&](auto kk) {
+        k_loss_dgamma<decltype(kk)::value><<<lgrid, kBlock, 0, st>>>(nb, P, k1, model->z.get(), prob->u.get(),
+                                                                     model->dgamma.get());
+    };
+    switch ((k1 + passes - 1) / passes) {
+    case 1: dgamma(std::integral_constant<int, 1>{}); break;
+    case 2: dgamma(std::integral_constant<int, 2>{}); break;
+    case 3: dgamma(std::integral_constant<int, 3>{}); break;
+    case 4: dgamma(std::integral_constant<int, 4>{}); break;
+    case 5: dgamma(std::integral_constant<int, 5>{}); break;
+    case 6: dgamma(std::integral_constant<int, 6>{}); break;
+    case 7: dgamma(std::integral_constant<int, 7>{}); break;
+    default: dgamma(std::integral_constant<int, 8>{}); break;
+    }
     OWTK_LAUNCH_CHECK();
 
     float* grad = model->grad.get();

@@ -398,3 +398,10 @@ def test_ssor_repeated_columns(ctx, schedule, block, nodes):
     owtk.Preconditioner(owtk.Matrix.csr(ctx, *args), owtk.PC_SSOR, block_nodes=nodes, omega=1.2,
                         schedule=schedule).apply(ctx.upload(x), yd)
     assert np.max(np.abs(yd.download() - ref)) <= 1e-14 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("block,degree", [(1, 0), (2, 2), (3, 5), (2, 6), (1, 7), (3, 8), (1, 16), (1, 31)])
+def test_training_gradient_degrees(ctx, block, degree):
+    """Coefficient counts in one pass of every width, just beyond one pass, and up to the most outputs; the checks and
+    bounds of the gradient test above."""
+    test_training_gradient_sizes(ctx, 23, 17, block, degree)
