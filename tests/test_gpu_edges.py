@@ -25,7 +25,7 @@ def ragged_pattern(rng, n, ghost, lengths):
 @pytest.mark.parametrize("block", [5, 7, 36, 65, 300])
 def test_row_component_spmv(ctx, block):
     """Blocks above four components: rows of 0 to 17 entries (8 per pass), rows that straddle waves and
-    workgroups; split and CSR forms bitwise, FP32 storage bitwise, the residual's fused norm."""
+    workgroups; split and CSR forms bitwise, FP32 storage bitwise, the residual vector."""
     rng = np.random.default_rng(block)
     n, ghost = 37, 3
     lengths = np.concatenate([[0, 1, 7, 8, 9, 15, 16, 17], rng.integers(0, 18, n - 8)])
@@ -231,8 +231,9 @@ def test_reductions_around_the_fused_grid(ctx, n):
 
 @pytest.mark.parametrize("k", [0, 1, 2, 3, 4, 8, 9, 15, 16, 30, 31, 32, 62])
 def test_finisher_widths(ctx, k):
-    """The finisher for every number of values and more partials (1,661 blocks) than one pass of a wave takes; a NaN
-    in one vector reaches only that vector's value.  Bounds as in the test above."""
+    """The finisher for every number of values, over the multi-dot's largest grid (1,024 blocks: one full pass of a
+    wave above 8 values, part of one below); a NaN in one vector reaches only that vector's value.  Bounds as in the
+    test above."""
     n = 1_700_001
     rng = np.random.default_rng(k)
     host = [rng.uniform(-1, 1, n) for _ in range(3)]
@@ -405,3 +406,56 @@ def test_training_gradient_degrees(ctx, block, degree):
     """Coefficient counts in one pass of every width, just beyond one pass, and up to the most outputs; the checks and
     bounds of the gradient test above."""
     test_training_gradient_sizes(ctx, 23, 17, block, degree)
+
+
+@pytest.mark.parametrize("block", [5, 65])
+def test_row_component_residual_norm(ctx, block):
+    """The norm that the residual SpMV of blocks above four reduces, as a solver's first residual: rows of 0 to 17
+    entries, a start vector that is not zero.  A sum of squares over n values: a few ulp."""
+    rng = np.random.default_rng(block)
+    n = 137
+    off, col = ragged_pattern(rng, n, 0, rng.integers(0, 18, n))
+    val, diag = rng.uniform(-1, 1, off[-1] * block), rng.uniform(1, 2, n * block)
+    x, b = rng.uniform(-1, 1, n * block), rng.uniform(-1, 1, n * block)
+    ref = np.linalg.norm(b - orc.OMatrix.split(n, 0, block, off, col, diag, val).spmv(x))
+    m = owtk.Matrix.split(ctx, n, 0, block, off, col, diag, val)
+    res = owtk.bicgstab(m, None, ctx.upload(b), ctx.upload(x), owtk.SolverOptions(maximum_iterations=1))
+    assert abs(res["initial_residual_norm"] - ref) <= 1e-14 * ref
+
+
+@pytest.mark.parametrize("n", [8192 * 1024 + 1, 9_000_001, 16384 * 1024 + 77])
+def test_norm_of_more_partials_than_a_pass(ctx, n):
+    """Two values of more than 8,192 blocks: the finisher's second pass, with one block in it, part of one, and at the
+    largest grid.  The exact count: sums of small integers."""
+    a = np.zeros(n)
+    a[::3] = 2.0
+    a[-1] = 5.0
+    d = ctx.upload(a)
+    exact = np.sum(a * a)
+    assert ctx.norm(d) == np.sqrt(exact)
+    assert ctx.dot(d, d) == exact
+    a[-1] = np.inf
+    assert np.isinf(ctx.norm(ctx.upload(a)))
+
+
+def test_solvers_of_more_partials_than_a_pass(ctx):
+    """Reductions of two to six values over 6,157 vector blocks and 8,209 SpMV blocks: the finisher's second and later
+    passes for every width that the solvers use.  The first residual is the right-hand side, the last one is summed
+    again on the host (a few ulp of n values, 1e-13 with room), and the two forms of one recurrence need the same
+    number of iterations to a few."""
+    s = owtk.generate_split(1500, 1401, 3, 4, ordering=owtk.ORDER_HILBERT)
+    n = s.nodes * 3
+    m = owtk.Matrix.split(ctx, s.nodes, 0, 3, s.offsets, s.columns, s.diagonal, s.off_diagonal)
+    pc = owtk.Preconditioner(m, owtk.PC_JACOBI)
+    b, x, r = ctx.upload(s.rhs), ctx.empty(n), ctx.empty(n)
+    norm, counts = np.linalg.norm(s.rhs), []
+    for solve in (owtk.bicgstab, owtk.pipelined_bicgstab, owtk.communication_hiding_bicgstab):
+        x.zero()
+        res = solve(m, pc, b, x, owtk.SolverOptions(relative_tolerance=1e-6, maximum_iterations=200))
+        assert res["status_name"] == "converged"
+        m.residual(b, x, r)
+        assert abs(res["initial_residual_norm"] - norm) <= 1e-13 * norm
+        true = np.linalg.norm(r.download())
+        assert true <= 1e-6 * norm and abs(res["true_residual_norm"] - true) <= 1e-13 * true
+        counts.append(res["iterations"])
+    assert max(counts) - min(counts) <= 3
