@@ -125,8 +125,8 @@ def random_dominant(rng, n, block, low, high):
 @pytest.mark.parametrize("case", ["1-node", "grid-1", "grid-2", "grid-3", "grid-4-rcm", "sparse", "wide", "wider", "dense"])
 def test_red_black_coarse_sweeps(ctx, case):
     """Red-black multigrid against the oracle after two V cycles: one-chunk and partial chunks, 1 to 4 components,
-    coarse rows of 4 to 16 entries (each slot count of the one-wave sweep), longer ones and unsymmetric patterns
-    (several red levels, the workgroup sweep).  The sweeps keep the oracle's operations and their order; the fine
+    black coarse rows of up to 3, 6 and 9 entries (the one-wave sweep with 4, 6 and 10 slots), of 18 to 28 and
+    unsymmetric patterns (the workgroup sweep, several red levels).  The sweeps keep the oracle's operations and their order; the fine
     SpMV and the residual sums bound the difference: 1e-13, as for the other multigrid solves."""
     rng = np.random.default_rng(len(case))
     if case == "1-node":
@@ -459,3 +459,26 @@ def test_solvers_of_more_partials_than_a_pass(ctx):
         assert true <= 1e-6 * norm and abs(res["true_residual_norm"] - true) <= 1e-13 * true
         counts.append(res["iterations"])
     assert max(counts) - min(counts) <= 3
+
+
+@pytest.mark.parametrize("seed,low,high,widest", [(1, 1, 3, 7), (2, 1, 3, 8), (2, 3, 4, 11), (1, 3, 4, 12), (1, 4, 4, 13),
+                                                  (1, 3, 5, 16), (2, 5, 5, 17)])
+def test_red_black_coarse_sweep_widths(ctx, seed, low, high, widest):
+    """The one-wave sweep with 8, 12 and 16 slots at their fewest and most entries per black row, and one entry more
+    (the workgroup sweep); the solve and bound of the test above."""
+    n, block = 500, 2
+    off, col, val = random_dominant(np.random.default_rng(seed), n, block, low, high)
+    m = owtk.Matrix.csr(ctx, n, 0, block, off, col, val)
+    om = orc.OMultigrid(orc.OMatrix.csr(n, 0, block, off, col, val), smoother=1)
+    _, coff, ccol, _, _ = om.coarse()
+    red, rows = set(), [set(ccol[coff[i]:coff[i + 1]]) - {i} for i in range(len(coff) - 1)]
+    for i, row in enumerate(rows):
+        if not row & red:
+            red.add(i)
+    assert max(len(row) for i, row in enumerate(rows) if i not in red) == widest
+    b = np.random.default_rng(seed).uniform(-1, 1, n * block)
+    kw = dict(relative_tolerance=1e-300, maximum_iterations=2)
+    xo, _ = om.solve(b, cycle=0, **kw)
+    x = ctx.empty(n * block)
+    owtk.Multigrid(m, smoother=owtk.MG_RED_BLACK).solve(ctx.upload(b), x, owtk.SolverOptions(**kw))
+    assert np.max(np.abs(x.download() - xo)) <= 1e-13 * np.max(np.abs(xo))
