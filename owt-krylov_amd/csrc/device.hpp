@@ -164,9 +164,9 @@ struct ReduceScratch {
 // Largest grid whose last block finishes a reduction itself.  A finisher
 // launch costs about 4 us; a block's fence and its atomic on the one counter
 // cost less until the blocks queue up.  BiCGSTAB + Jacobi (four reductions an
-// iteration), block 3, us per iteration fused / with finishers: 39 / 50 at
-// 2,048 vertices (8 blocks), 42 / 56 at 8,192 (32), 48 / 54 at 32,768 (128),
-// 63 / 55 at 64,800 (254).
+// iteration), block 3, us per iteration fused / with finishers: 38 / 42 at
+// 2,048 vertices (8 blocks), 39 / 46 at 8,192 (32), 45 / 47 at 32,768 (128),
+// 59 / 51 at 64,800 (254).
 constexpr unsigned int kFuseBlocks = 128;
 
 // Cross-block reductions of more than kFuseBlocks blocks run in two launches
@@ -276,17 +276,20 @@ __device__ inline void stores_in_l2()
 // what the block had stored there by then: the partials, which thread 0 stored
 // itself, and where a vector of this kernel is read next (by block_norm's
 // second pass, or by the host's other streams once it has the result) also the
-// vector, because every wave then waits for its own stores before the block's
-// barriers, which wait for LDS only.  (A release
-// fence in every wave would write the L2 back four times a block: 47 -> 56 us
-// an iteration of BiCGSTAB + Jacobi at 32,768 vertices.)
+// vector, because every wave then waits for its own stores before a barrier of
+// the block (a barrier alone waits for LDS only).  The wait comes after the
+// block's sums, which hide most of it.  (A release fence in every wave would
+// write the L2 back four times a block: 47 -> 56 us an iteration of BiCGSTAB +
+// Jacobi at 32,768 vertices.)
 template<int K, class Fin>
 __device__ inline void reduce_end(double (&v)[K], std::uint64_t max_mask, ReduceScratch scratch, const Fin& fin)
 {
-    if constexpr (reads_stores<Fin>())
-        if (scratch.ticket != nullptr) stores_in_l2();
     store_partials<K>(v, max_mask, scratch);
     if (scratch.ticket == nullptr) return;
+    if constexpr (reads_stores<Fin>()) {
+        stores_in_l2();
+        __syncthreads();
+    }
     __shared__ double totals[K];
     __shared__ unsigned int arrived;
     if (threadIdx.x == 0) {
