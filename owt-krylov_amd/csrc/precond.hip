@@ -1449,13 +1449,15 @@ void build_schedule(owtk_precond pc, const TriHost& t)
     upload(tri.blev, tri.h_blev);
     upload(tri.flev_pos, tri.h_flev_pos);
     upload(tri.blev_pos, tri.h_blev_pos);
-    upload(tri.frow, frow);
-    upload(tri.brow, brow);
     upload(tri.frow_lvl, frow_lvl);
-    upload(tri.fptr, fptr);
-    upload(tri.bptr, bptr);
-    upload(tri.fcol, fcol);
-    upload(tri.bcol, bcol);
+    if (!tri.chain) {  // the chains read codes instead
+        upload(tri.frow, frow);
+        upload(tri.brow, brow);
+        upload(tri.fptr, fptr);
+        upload(tri.bptr, bptr);
+        upload(tri.fcol, fcol);
+        upload(tri.bcol, bcol);
+    }
     upload(tri.fsrc, fsrc);
     upload(tri.bsrc, bsrc);
 }
@@ -1884,8 +1886,12 @@ void build_ilu_chunks(owtk_precond pc, const std::vector<std::int64_t>& upd_ptr,
     std::vector<std::uint32_t> op_a, op_b;
     std::vector<std::uint16_t> upd_a, upd_b;
     int max_src = 0, max_a = 0, max_nua = 0, max_b = 0, max_nub = 0;
-    struct OpA { int es, pt; std::vector<std::pair<int, int>> upd; };
-    struct OpB { int step, es, ps; std::vector<std::pair<int, int>> upd; };
+    // a chunk's operations by lane, their updates (target, source) in one pool;
+    // kept over the chunks, whose allocations would take half the set-up
+    struct Op { int step, es, ps, upd0, count; };
+    std::vector<std::vector<std::int32_t>> srcs(64);
+    std::vector<std::vector<Op>> as(64), bs_(64);
+    std::vector<std::pair<int, int>> upd;
     std::int64_t chunks = 0;
     for (std::int64_t b = 0; b < tri.blocks; ++b) {
         chunk_first[b] = static_cast<std::int32_t>(chunks);
@@ -1893,28 +1899,31 @@ void build_ilu_chunks(owtk_precond pc, const std::vector<std::int64_t>& upd_ptr,
         for (std::int64_t c0 = 0; c0 < nb; c0 += 64, ++chunks) {
             const int cnt = static_cast<int>(std::min<std::int64_t>(64, nb - c0));
             const std::int64_t first = r0 + c0;
-            std::vector<std::vector<std::int32_t>> srcs(64);
-            std::vector<std::vector<OpA>> as(64);
-            std::vector<std::vector<OpB>> bs_(64);
+            upd.clear();
+            for (int lane = 0; lane < 64; ++lane) {
+                srcs[lane].clear();
+                as[lane].clear();
+                bs_[lane].clear();
+            }
             for (int lane = 0; lane < cnt; ++lane) {
                 const std::int64_t row = first + lane;
                 const std::int64_t rb = f.h_offsets[row];
                 for (std::int64_t e = rb; e < f.h_diag[row]; ++e) {
                     const std::int64_t k = f.h_columns[e];
+                    const int upd0 = static_cast<int>(upd.size()), count = static_cast<int>(upd_ptr[e + 1] - upd_ptr[e]);
                     if (k < first) {
-                        OpA op{static_cast<int>(e - rb), static_cast<int>(srcs[lane].size()), {}};
+                        as[lane].push_back({0, static_cast<int>(e - rb), static_cast<int>(srcs[lane].size()), upd0, count});
                         srcs[lane].push_back(static_cast<std::int32_t>(f.h_diag[k]));
                         for (std::int64_t u = upd_ptr[e]; u < upd_ptr[e + 1]; ++u) {
-                            op.upd.push_back({static_cast<int>(upd_target[u] - rb), static_cast<int>(srcs[lane].size())});
+                            upd.push_back({static_cast<int>(upd_target[u] - rb), static_cast<int>(srcs[lane].size())});
                             srcs[lane].push_back(static_cast<std::int32_t>(upd_upper[u]));
                         }
-                        as[lane].push_back(std::move(op));
                     } else {
                         const std::int64_t kb = f.h_offsets[k];
-                        OpB op{static_cast<int>(k - first), static_cast<int>(e - rb), static_cast<int>(f.h_diag[k] - kb), {}};
+                        bs_[lane].push_back({static_cast<int>(k - first), static_cast<int>(e - rb),
+                                             static_cast<int>(f.h_diag[k] - kb), upd0, count});
                         for (std::int64_t u = upd_ptr[e]; u < upd_ptr[e + 1]; ++u)
-                            op.upd.push_back({static_cast<int>(upd_target[u] - rb), static_cast<int>(upd_upper[u] - kb)});
-                        bs_[lane].push_back(std::move(op));
+                            upd.push_back({static_cast<int>(upd_target[u] - rb), static_cast<int>(upd_upper[u] - kb)});
                     }
                 }
             }
@@ -1923,8 +1932,8 @@ void build_ilu_chunks(owtk_precond pc, const std::vector<std::int64_t>& upd_ptr,
                 nsrc = std::max<int>(nsrc, static_cast<int>(srcs[lane].size()));
                 na = std::max<int>(na, static_cast<int>(as[lane].size()));
                 nbo = std::max<int>(nbo, static_cast<int>(bs_[lane].size()));
-                for (const auto& o : as[lane]) nua = std::max<int>(nua, static_cast<int>(o.upd.size()));
-                for (const auto& o : bs_[lane]) nub = std::max<int>(nub, static_cast<int>(o.upd.size()));
+                for (const auto& o : as[lane]) nua = std::max(nua, o.count);
+                for (const auto& o : bs_[lane]) nub = std::max(nub, o.count);
             }
             if (nsrc > 255 || nua > 255 || nub > 255) return;
             hdr.insert(hdr.end(), {first, cnt, static_cast<std::int64_t>(src_a.size()), nsrc,
@@ -1942,19 +1951,19 @@ void build_ilu_chunks(owtk_precond pc, const std::vector<std::int64_t>& upd_ptr,
                 for (std::size_t t2 = 0; t2 < srcs[lane].size(); ++t2) src_a[s0 + t2 * 64 + lane] = srcs[lane][t2];
                 for (std::size_t j = 0; j < as[lane].size(); ++j) {
                     const auto& o = as[lane][j];
-                    op_a[a0 + j * 64 + lane] = static_cast<std::uint32_t>(o.es) | (static_cast<std::uint32_t>(o.pt) << 8)
-                        | (static_cast<std::uint32_t>(o.upd.size()) << 16);
-                    for (std::size_t u = 0; u < o.upd.size(); ++u)
+                    op_a[a0 + j * 64 + lane] = static_cast<std::uint32_t>(o.es) | (static_cast<std::uint32_t>(o.ps) << 8)
+                        | (static_cast<std::uint32_t>(o.count) << 16);
+                    for (int u = 0; u < o.count; ++u)
                         upd_a[ua0 + (j * nua + u) * 64 + lane] =
-                            static_cast<std::uint16_t>(o.upd[u].first | (o.upd[u].second << 8));
+                            static_cast<std::uint16_t>(upd[o.upd0 + u].first | (upd[o.upd0 + u].second << 8));
                 }
                 for (std::size_t j = 0; j < bs_[lane].size(); ++j) {
                     const auto& o = bs_[lane][j];
                     op_b[b0 + j * 64 + lane] = static_cast<std::uint32_t>(o.step) | (static_cast<std::uint32_t>(o.es) << 8)
-                        | (static_cast<std::uint32_t>(o.ps) << 16) | (static_cast<std::uint32_t>(o.upd.size()) << 24);
-                    for (std::size_t u = 0; u < o.upd.size(); ++u)
+                        | (static_cast<std::uint32_t>(o.ps) << 16) | (static_cast<std::uint32_t>(o.count) << 24);
+                    for (int u = 0; u < o.count; ++u)
                         upd_b[ub0 + (j * nub + u) * 64 + lane] =
-                            static_cast<std::uint16_t>(o.upd[u].first | (o.upd[u].second << 8));
+                            static_cast<std::uint16_t>(upd[o.upd0 + u].first | (upd[o.upd0 + u].second << 8));
                 }
             }
             max_src = std::max(max_src, nsrc);
