@@ -41,10 +41,9 @@ struct owtk_multigrid_s {
     owtk::DeviceArray<double> fine_inv, coarse_inv, agg_size;
     owtk::DeviceArray<std::int32_t> f2c, agg_ptr, agg_members, fine_red, fine_black;
     std::int64_t n_red = 0, n_black = 0;
-    // coarse Gauss-Seidel: CSR on the device and the level schedule of each colour
-    owtk::DeviceArray<std::int32_t> coff, ccol, gs_rows;
+    // coarse Gauss-Seidel: the level schedule of each colour
+    owtk::DeviceArray<std::int32_t> gs_rows;
     owtk::DeviceArray<std::int64_t> gs_levels;  // device copy of gs_level_ptr
-    owtk::DeviceArray<double> cval;
     std::vector<std::int64_t> gs_level_ptr;  // red levels, then black levels
     std::int64_t red_levels = 0;
     // the same rows in sweep (level) order as ELL: position p's k-th
@@ -608,7 +607,7 @@ void mg_setup(owtk_multigrid_s* mg)
     mg->n_black = static_cast<std::int64_t>(black.size());
     upload(mg->fine_red, red);
     upload(mg->fine_black, black);
-    // coarse Gauss-Seidel: device CSR and level schedules
+    // coarse Gauss-Seidel: level schedules
     std::vector<std::int32_t> cred, cblack;
     colouring(nc, mg->h_coff, mg->h_ccol, cred, cblack);
     std::vector<std::int32_t> tptr(nc + 1, 0), tcol(mg->h_ccol.size());
@@ -627,10 +626,10 @@ void mg_setup(owtk_multigrid_s* mg)
     gs_levels(nc, mg->h_coff, mg->h_ccol, tptr, tcol, cblack, gs_rows, mg->gs_level_ptr);
     upload(mg->gs_rows, gs_rows);
     upload(mg->gs_levels, mg->gs_level_ptr);
-    upload(mg->coff, mg->h_coff);
-    upload(mg->ccol, mg->h_ccol);
-    upload(mg->cval, mg->h_cval);
-    // level-ordered ELL copy of the coarse rows for the sweep kernel
+    if (mg->opt.smoother == OWTK_MG_RED_BLACK) build_wave(mg, tptr, tcol, cblack);
+    // level-ordered ELL copy of the coarse rows for the sweep kernel (the red
+    // rows alone where the one-wave sweep takes the black ones)
+    if (mg->wave_k) gs_rows.resize(static_cast<std::size_t>(mg->gs_level_ptr[mg->red_levels]));
     const std::int64_t P = static_cast<std::int64_t>(gs_rows.size());
     int K = 0;
     for (const std::int32_t r : gs_rows) {
@@ -665,7 +664,6 @@ void mg_setup(owtk_multigrid_s* mg)
     upload(mg->gs_col, gcol);
     upload(mg->gs_val, gval);
     upload(mg->gs_diag, gdiag);
-    if (mg->opt.smoother == OWTK_MG_RED_BLACK) build_wave(mg, tptr, tcol, cblack);
 }
 
 double smoother_weight(const owtk_multigrid_options& o, std::uint64_t step)
