@@ -751,13 +751,15 @@ __global__ __launch_bounds__(256) void k_tri_apply(TriArgs a, const V* __restric
 // is the reference's order in the forward sweep; backward sweeps take their
 // entries in the order the rows finish.
 //
-// Measured (FP64, the earlier 64-row sweep in brackets): ILU(0) apply at 2M
-// vertices, block 3, 4,096-row blocks 225 (284) us; 2,048 vertices,
-// 512-row blocks 16.5 (24.4) us; SSOR of 1,296 components on a
-// 32 x 32 grid 46.6 (73) us.  A lone chunk takes about 0.25 us, 243 clocks of
-// it the steps; with 384 workgroups running, the padded values and codes (about
-// 1 GB an apply) add memory time.  One wave doing all of this took 266 us, and
-// a third wave touching the coming chunks' lines 282 us.
+// Measured (FP64, the earlier 64-row sweep in brackets; launches that a stopped
+// solver skips left out): ILU(0) apply at 2M vertices, block 3, 4,096-row
+// blocks 237 (307) us; 2,048 vertices, 512-row blocks 18.1 (27.4) us; SSOR of
+// 1,296 components on a 32 x 32 grid 62.0 (94.5) us.  A lone chunk takes about
+// 0.25 us, 243 clocks of it the steps, which bounds the small ones.  At 2M
+// vertices the two sweeps' 512 chunks would take 128 us; there the padded
+// values and codes bound it, about 1 GB an apply at 4.2 TB/s.  One wave doing
+// all of this took 266 us where this form had 225 (a mean with skipped
+// launches), and a third wave touching the coming chunks' lines 282 us.
 template<class X>
 __device__ inline X chain_finish(X acc, X, X, std::integral_constant<int, 0>)  // ILU forward: unit diagonal
 {
